@@ -1,8 +1,9 @@
 // Batched dense kernels over per-fiber blocks of uneven order (n <= 256):
-//   * LU factorisation with partial pivoting (LAPACK dgetrf semantics):
-//     FP64 register/LDS-resident, one persistent 1024-thread workgroup per
-//     block; equilibrated FP32 blocked on MFMA (lu_factor_f32_mfma_kernel
-//     below), two 256-thread workgroups per CU;
+//   * LU factorisation with partial pivoting (LAPACK dgetrf semantics): the
+//     entry point, which runs lu_block.hip, and two alternatives it takes on
+//     request: FP64 register/LDS-resident, one persistent 1024-thread
+//     workgroup per block; equilibrated FP32 blocked on MFMA
+//     (lu_factor_f32_mfma_kernel below), two 256-thread workgroups per CU;
 //   * forward/backward substitution with optional FP64 iterative refinement,
 //     one wavefront per block;
 //   * column-major block GEMV, one wavefront per block.
@@ -774,11 +775,9 @@ lu_solve_kernel(const int* __restrict__ n_arr, const long* __restrict__ a_off,
 // lu_solve_kernel with refine = 0 (FP64 substitutions in the same order).
 constexpr int kLdsSolveBytes = 64 * 1024;
 
-// Launch choices set by the autotuner through f3d_lu_set_launch, per
-// precision (0 = FP64, 1 = FP32): waves per CU of the one-wave blocked
-// factorisation, and whether solves without refinement stage the factor in
-// LDS when it fits.
-static int g_lu_per_cu[2] = {4, 8};
+// Launch choice set by the autotuner through f3d_lu_set_launch, per
+// precision (0 = FP64, 1 = FP32): whether solves without refinement stage the
+// factor in LDS when it fits.
 static int g_lu_solve_staged[2] = {1, 1};
 
 // Substitutions out of LDS.  The loops run over the 64-row slot ms of the
@@ -1099,10 +1098,10 @@ static int num_cus() {
   return cached;
 }
 
-int launch_lu_wave(int precision, int64_t nb, const int32_t* n, const int64_t* a_off,
-                   const int64_t* x_off, const int32_t* order, const double* A, double* lu64,
-                   float* lu32, double* rs, double* cs, int32_t* piv, int32_t* perm,
-                   int32_t* info, int num_cu, int per_cu, hipStream_t st);
+int launch_lu_block(int precision, int64_t nb, const int32_t* n, const int64_t* a_off,
+                    const int64_t* x_off, const int32_t* order, const double* A, double* lu64,
+                    float* lu32, double* rs, double* cs, int32_t* piv, int32_t* perm,
+                    int32_t* info, hipStream_t st);
 
 }  // namespace f3d
 
@@ -1122,9 +1121,9 @@ extern "C" int f3d_lu_factor_batched(int precision, int64_t nb, int32_t nmax, co
   F3D_REQUIRE(n && a_off && x_off && A && piv && perm && info, F3D_EINVAL,
               "lu_factor: NULL argument");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  // default: one wavefront per block, blocked, MFMA trailing update
-  // (lu_wave.hip); F3D_LU_KERNEL=workgroup selects the one-workgroup-per-block
-  // kernels below (FP32: F3D_LU32_KERNEL=vector for the unblocked one)
+  // default: one workgroup per block, left-looking strips in LDS, MFMA updates
+  // (lu_block.hip); F3D_LU_KERNEL=workgroup selects the one-workgroup-per-block
+  // kernels above (FP32: F3D_LU32_KERNEL=vector for the unblocked one)
   const char* sel_k = getenv("F3D_LU_KERNEL");
   if (!(sel_k && strcmp(sel_k, "workgroup") == 0)) {
     if (precision == F3D_F64) {
@@ -1132,8 +1131,8 @@ extern "C" int f3d_lu_factor_batched(int precision, int64_t nb, int32_t nmax, co
     } else {
       F3D_REQUIRE(lu32 && rs && cs, F3D_EINVAL, "lu_factor: lu32/rs/cs is NULL");
     }
-    return launch_lu_wave(precision, nb, n, a_off, x_off, order, A, lu64, lu32, rs, cs, piv,
-                          perm, info, num_cus(), g_lu_per_cu[precision == F3D_F64 ? 0 : 1], st);
+    return launch_lu_block(precision, nb, n, a_off, x_off, order, A, lu64, lu32, rs, cs, piv,
+                           perm, info, st);
   }
   const unsigned grid = (unsigned)(nb < num_cus() ? nb : num_cus());
   if (precision == F3D_F64) {
@@ -1220,7 +1219,6 @@ extern "C" int f3d_lu_set_launch(int precision, int32_t factor_waves_per_cu,
               "lu_set_launch: waves per CU %d outside [0, %d]", factor_waves_per_cu, cap);
   F3D_REQUIRE(solve_staged == 0 || solve_staged == 1, F3D_EINVAL,
               "lu_set_launch: solve_staged must be 0 or 1");
-  g_lu_per_cu[pp] = factor_waves_per_cu ? factor_waves_per_cu : cap;
   g_lu_solve_staged[pp] = solve_staged;
   return F3D_OK;
 }

@@ -35,6 +35,55 @@ def test_lu_factor_f64_matches_lapack():
         assert rel2(LU[b], lu_ref) < 1e-12
 
 
+@pytest.mark.parametrize("n", [15, 16, 31, 32, 33, 48, 63, 65, 129, 161, 224, 241])
+@pytest.mark.parametrize("precision", ["f64", "f32c"])
+def test_lu_factor_strip_edges(precision, n):
+    """Orders at the edges of the factorisation's panels, strips and waves:
+    LAPACK's pivots and factors in FP64, P (Dr A Dc) = L U in FP32.  Beside
+    each, a block of the same order whose columns are full of equal maxima (the
+    first row must win), one with a zero column and one with a column of
+    NaN."""
+    print(f"case lu strip edges {precision} n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    M = rng.normal(size=(n, n))
+    # exact in either precision: entries of L and U in {-1, 0, 1}
+    T = (np.tril(rng.integers(-1, 2, size=(n, n)), -1) + np.eye(n)) @ (
+        np.triu(rng.integers(-1, 2, size=(n, n)), 1) + np.eye(n))
+    Z = M.copy()
+    Z[:, n // 2] = 0.0
+    N = M.copy()
+    N[:, n - 1] = np.nan
+    bs = BlockSet([n] * 4)
+    lu = BatchedLU(bs, bs.pack([M, T, Z, N]), precision=precision)
+    torch.cuda.synchronize()
+    LU = bs.unpack((lu.lu64 if precision == "f64" else lu.lu32).double())
+    piv = lu.piv.cpu().numpy().reshape(4, n)
+    assert lu.info.cpu().numpy().tolist()[:3] == [0, 0, n // 2 + 1]
+    ref, piv_ref = sla.lu_factor(M)
+    if precision == "f64":
+        np.testing.assert_array_equal(piv[0], piv_ref)
+        assert rel2(LU[0], ref) < 1e-12 * n
+    for k in range(4):
+        # the interchanges and the permutation agree, and rows stay in range
+        p = np.arange(n)
+        for j, q in enumerate(piv[k]):
+            assert j <= q < n
+            p[[j, q]] = p[[q, j]]
+        np.testing.assert_array_equal(lu.perm.cpu().numpy()[k * n:(k + 1) * n], p)
+    if precision == "f64":
+        np.testing.assert_array_equal(piv[1], np.arange(n))
+        np.testing.assert_array_equal(LU[1], sla.lu_factor(T)[0])
+    As = M
+    if precision == "f32c":
+        As = lu.rs.cpu().numpy()[:n, None] * M * lu.cs.cpu().numpy()[None, :n]
+    P = lu.perm.cpu().numpy()[:n]
+    back = (np.tril(LU[0], -1) + np.eye(n)) @ np.triu(LU[0])
+    # |L U - P A| <= 2 n eps |L| |U| element by element
+    bound = (np.abs(np.tril(LU[0], -1)) + np.eye(n)) @ np.abs(np.triu(LU[0]))
+    eps = 2.0 ** -53 if precision == "f64" else 2.0 ** -24
+    assert (np.abs(back - As[P]) <= 2 * n * eps * bound + 1e-300).all()
+
+
 @pytest.mark.parametrize("precision", ["f64", "f32c"])
 def test_lu_solve_batched(precision):
     print(f"case lu solve {precision}", flush=True)
