@@ -11,9 +11,9 @@ the 65536 x 65536 shape as the (kernel, precision) default.  The large
 fiber -> fiber Oseen sum (262144 nodes, exclusion ranges) is tuned on its
 own layout, bucket 18/18.
 
-Batched LU (f3d_lu_set_launch): LDS-staged versus streaming solves, timed on
+Batched LU (f3d_lu_set_launch): waves per CU and solve staging, timed on
 fiber blocks of the shapes the stepper factors (the waves-per-CU entry is
-checked and stored, but the factorisation's launch no longer depends on it).  BF16 GEMM (f3d_gemm_set_stream): resident-weight,
+checked and stored, but no launch depends on either any more).  BF16 GEMM (f3d_gemm_set_stream): resident-weight,
 streaming or tiled kernel for the per-node layers (N = 128, 256).
 
 The table lives in fiber3d_amd/tuning.json; the kernels module calls apply()

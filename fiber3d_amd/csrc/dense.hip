@@ -534,149 +534,214 @@ lu_factor_f32_mfma_kernel(int nb, const int* __restrict__ n_arr, const long* __r
 }
 
 // ---------------------------------------------------------------------------
-// One wavefront per block: lane owns rows lane + 64 m, m < 4.
+// Triangular solves, one wavefront per block, row 64 s + lane in slot s.  The
+// rows go 64 at a time: while the columns of segment s are consumed, slot s
+// ("cur") holds the unknowns, and the slots it still changes (NB of them)
+// follow in order, so the pivot entry is always cur's (two readlanes into
+// scalar registers), the slots are static registers, and the slots a
+// triangle excludes are neither loaded nor multiplied.  Within the diagonal
+// slot, lanes outside the triangle read the chunk's first (last) row, a line
+// that is needed anyway.  A sweep therefore reads n^2 / 2 entries plus the
+// chunks' steps at the diagonal, where the former version read all n^2 and
+// searched the pivot among four slots for each column (24 VALU + 21 SALU
+// instructions per column against 6 + NB).  Columns come in chunks in
+// two register sets that trade roles: one loads while the other is used.
+// Measured: 2048 fiber blocks of order 64-256 in FP64 215 -> 123 us (452 MB of
+// factor: 3.7 TB/s of the copy's 5.1); 1000 blocks of order 128 in FP32 without
+// refinement 56 us (factor staged in LDS) and 80 (streamed) -> 22; 32 blocks
+// of order 128 in FP64, where the chain alone counts, 53 -> 17.
 constexpr int kSlots = 4;
+// Columns of a chunk of NS slots: 16 loads of 64 rows in flight per wave.
+__host__ __device__ constexpr int chunk_cols(int NS) { return NS == 1 ? 16 : (NS == 2 ? 8 : 4); }
 
-// In-wave row permutation: w_new[row i] = w_old[row perm[i]], with row r held
-// by lane r % 64 in slot r / 64.
-__device__ __forceinline__ void permute_rows(double (&w)[kSlots], const int (&src_lane)[kSlots],
-                                             const int (&src_slot)[kSlots], int n, int lane) {
-  double out[kSlots];
+// Columns k0, k0 + step, ... (a chunk, clamped into the block) of a
+// column-major block, at the byte offsets of NS rows.
+template <typename T, int NS>
+__device__ __forceinline__ void load_cols(const T* __restrict__ M, int n, int k0, int step,
+                                          const unsigned (&off)[NS], T (&r)[chunk_cols(NS)][NS]) {
 #pragma unroll
-  for (int m = 0; m < kSlots; ++m) {
-    double acc = 0.0;
+  for (int u = 0; u < chunk_cols(NS); ++u) {
+    int k = k0 + u * step;
+    k = k < 0 ? 0 : (k > n - 1 ? n - 1 : k);
+    const char* __restrict__ col = reinterpret_cast<const char*>(M + k * n);
 #pragma unroll
-    for (int ms = 0; ms < kSlots; ++ms) {
-      const double t = __shfl(w[ms], src_lane[m], 64);
-      if (ms == src_slot[m]) acc = t;
-    }
-    out[m] = (64 * m + lane < n) ? acc : 0.0;
+    for (int m = 0; m < NS; ++m) r[u][m] = *reinterpret_cast<const T*>(col + off[m]);
   }
-#pragma unroll
-  for (int m = 0; m < kSlots; ++m) w[m] = out[m];
 }
 
-// Column streaming for the one-wave solves: column k of a column-major n x n
-// block is consumed in order k = k_begin, k_begin + step, ... (count columns),
-// each lane holding rows lane + 64 m.  Columns come in rounds of kPf, in two
-// register sets that trade roles: the next round loads into one set while
-// the other's columns are used, so a wave waits for HBM once per round and
-// never for the loads it has just issued.  (A single ring reloaded in place
-// let the compiler hoist each reload above the mask that reads the old
-// value, copy the loaded value back at the end of the round, and wait there
-// for the round's own loads.)  want(i, k) masks the rows a column
-// contributes (the triangle).
-constexpr int kPf = 4;  // 6 or 8 take more than 256 VGPRs: one wave per SIMD instead of two
-
-// The loads are unconditional (row and column indices clamped into the
-// block; rows past n and columns past the stream are loaded and discarded)
-// and the triangle mask is applied when a column is used: a load under a
-// lane mask would end in a branch whose join waits for every load in flight.
-template <typename T, typename Want, typename Use>
-__device__ __forceinline__ void stream_cols(const T* __restrict__ M, int n, int k_begin, int step,
-                                            int count, int lane, Want&& want, Use&& use) {
-  T ra[kPf][kSlots], rb[kPf][kSlots];
-  auto load = [&](int idx0, T (&r)[kPf][kSlots]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < kPf; ++u) {
-      int k = k_begin + (idx0 + u) * step;
-      k = k < 0 ? 0 : (k > n - 1 ? n - 1 : k);
-      const T* __restrict__ col = M + (long)k * n;
-#pragma unroll
-      for (int m = 0; m < kSlots; ++m) {
-        const int i = 64 * m + lane;
-        r[u][m] = col[i < n ? i : n - 1];
-      }
-    }
-  };
-  // tail: stop at column index count (the whole rounds have no branch, so
-  // their loads stay where they are issued)
-  auto take = [&](auto tail, int idx0, const T (&r)[kPf][kSlots]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < kPf; ++u) {
-      if constexpr (decltype(tail)::value) {
-        if (idx0 + u >= count) break;
-      }
-      const int k = k_begin + (idx0 + u) * step;
-      T v[kSlots];
-#pragma unroll
-      for (int m = 0; m < kSlots; ++m) {
-        const int i = 64 * m + lane;
-        v[m] = (i < n && want(i, k)) ? r[u][m] : (T)0;
-      }
-      use(k, v);
-    }
-  };
+// use(tail, j0, set) for the chunks of cnt columns, load(j0, set) one chunk
+// ahead.  The chunk index passes through an empty asm placed after the loads:
+// the chunk's work depends on it, so the compiler can neither sink the loads
+// to their uses nor hoist the uses to the loads; and the next loads come after
+// an asm that takes the work's result (state), so they reuse the set's
+// registers instead of a third set.
+template <typename T, int NS, typename Load, typename Use>
+__device__ __forceinline__ void stream_chunks(int cnt, double& state, Load&& load, Use&& use) {
+  constexpr int kCh = chunk_cols(NS);
+  T ra[kCh][NS], rb[kCh][NS];
   load(0, ra);
-  // whole pairs of rounds without a branch between the loads and their uses
-  int i0 = 0;
-  for (; i0 + 2 * kPf <= count; i0 += 2 * kPf) {
-    load(i0 + kPf, rb);
-    // The column index of each round passes through an empty asm placed
-    // after the loads: the round's work depends on it, so the compiler can
-    // neither sink the loads to their uses nor hoist the uses to the loads.
-    int ja = i0;
+  int j0 = 0;
+  for (; j0 + 2 * kCh <= cnt; j0 += 2 * kCh) {
+    load(j0 + kCh, rb);
+    int ja = j0;
     asm volatile("" : "+s"(ja) : : "memory");
-    take(std::false_type{}, ja, ra);
-    load(i0 + 2 * kPf, ra);
-    int jb = i0 + kPf;
+    use(std::false_type{}, ja, ra);
+    asm volatile("" : "+v"(state) : : "memory");
+    if (j0 + 2 * kCh < cnt) load(j0 + 2 * kCh, ra);
+    int jb = j0 + kCh;
     asm volatile("" : "+s"(jb) : : "memory");
-    take(std::false_type{}, jb, rb);
+    use(std::false_type{}, jb, rb);
+    asm volatile("" : "+v"(state) : : "memory");
   }
-  if (i0 < count) {
-    load(i0 + kPf, rb);
-    take(std::true_type{}, i0, ra);
-    take(std::true_type{}, i0 + kPf, rb);
+  if (j0 < cnt) {
+    if (j0 + kCh < cnt) load(j0 + kCh, rb);
+    use(std::true_type{}, j0, ra);
+    if (j0 + kCh < cnt) use(std::true_type{}, j0 + kCh, rb);
   }
 }
 
-// v[slot] of lane (k % 64), slot k / 64 (k wave-uniform): one readlane per
-// slot and scalar selects.  (A select chain over the slots folds into a
-// dynamic index of v, which the compiler places in LDS: a write, a read and a
-// wait in the substitution's dependent chain.)
-template <typename T>
-__device__ __forceinline__ double pick_row(const T (&v)[kSlots], int k) {
-  const int ms = k >> 6, l = k & 63;
-  double r = readlane_f64((double)v[0], l);
+// w_i -= L(i, k) w_k, i > k, for the columns k = k0 .. of cur's segment.
+template <typename T, int NB>
+__device__ __forceinline__ void forward_segment(const T* __restrict__ L, int n, int k0, int lane,
+                                                double& cur, double (&next)[kSlots - 1]) {
+  const int cnt = min(64, n - k0);
+  unsigned off[NB + 1];
 #pragma unroll
-  for (int m = 1; m < kSlots; ++m) {
-    const double t = readlane_f64((double)v[m], l);
-    r = ms == m ? t : r;
+  for (int m = 1; m <= NB; ++m) off[m] = (unsigned)min(k0 + 64 * m + lane, n - 1) * (unsigned)sizeof(T);
+  stream_chunks<T, NB + 1>(
+      cnt, cur,
+      [&](int j0, T (&r)[chunk_cols(NB + 1)][NB + 1]) __attribute__((always_inline)) {
+        off[0] = (unsigned)min(k0 + max(lane, j0), n - 1) * (unsigned)sizeof(T);
+        load_cols<T, NB + 1>(L, n, k0 + j0, 1, off, r);
+      },
+      [&](auto tail, int j0, const T (&r)[chunk_cols(NB + 1)][NB + 1]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < chunk_cols(NB + 1); ++u) {
+          const int j = j0 + u;
+          if (decltype(tail)::value && j >= cnt) break;
+          const double wk = readlane_f64(cur, j);
+          cur = lane > j ? fma(-(double)r[u][0], wk, cur) : cur;
+#pragma unroll
+          for (int m = 1; m <= NB; ++m) next[m - 1] = fma(-(double)r[u][m], wk, next[m - 1]);
+        }
+      });
+}
+
+// w_k /= U(k, k); w_i -= U(i, k) w_k, i < k, for the columns of cur's segment
+// from the last to k0; next[m - 1]: slot m above.  Every row's quotient comes
+// from its reciprocal r = 1 / U(i, i), three operations on the chain where a
+// division takes about twelve: q = w r, then q + r (w - q U), the correctly
+// rounded quotient while nothing over- or underflows (Markstein).  A q that is
+// not finite stays as it is, and so does every q of a pivot outside
+// 2^-400 .. 2^400 (zero, infinite and NaN pivots among them).
+template <typename T, int NB>
+__device__ __forceinline__ void backward_segment(const T* __restrict__ U, int n, int k0, int lane,
+                                                 double& cur, double (&next)[kSlots - 1]) {
+  const int cnt = min(64, n - k0);
+  unsigned off[NB + 1];
+#pragma unroll
+  for (int m = 1; m <= NB; ++m) off[m] = (unsigned)(k0 - 64 * m + lane) * (unsigned)sizeof(T);
+  const double dg = (double)U[(long)min(k0 + lane, n - 1) * (n + 1)];
+  const double rc = 1.0 / dg;
+  const bool safe = fabs(dg) > 0x1p-400 && fabs(dg) < 0x1p400;
+  const double ds = safe ? dg : 0.0, rr = safe ? rc : 0.0;
+  stream_chunks<T, NB + 1>(
+      cnt, cur,
+      [&](int j0, T (&r)[chunk_cols(NB + 1)][NB + 1]) __attribute__((always_inline)) {
+        off[0] = (unsigned)(k0 + min(lane, cnt - 1 - j0)) * (unsigned)sizeof(T);
+        load_cols<T, NB + 1>(U, n, k0 + cnt - 1 - j0, -1, off, r);
+      },
+      [&](auto tail, int j0, const T (&r)[chunk_cols(NB + 1)][NB + 1]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < chunk_cols(NB + 1); ++u) {
+          if (decltype(tail)::value && j0 + u >= cnt) break;
+          const int j = cnt - 1 - (j0 + u);
+          const double q = cur * rc;
+          const double t = fma(fma(-q, ds, cur), rr, q);
+          const double wk = readlane_f64(isfinite(q) ? t : q, j);
+          cur = lane == j ? wk : (lane < j ? fma(-(double)r[u][0], wk, cur) : cur);
+#pragma unroll
+          for (int m = 1; m <= NB; ++m) next[m - 1] = fma(-(double)r[u][m], wk, next[m - 1]);
+        }
+      });
+}
+
+// w <- U^-1 L^-1 w (the factor's L unit lower, U upper, column-major), FP64
+// arithmetic; sw: 256 doubles of LDS, each lane its own.
+template <typename T>
+__device__ __forceinline__ void trsv_lu(const T* __restrict__ L, int n, int lane,
+                                        double (&w)[kSlots], double* __restrict__ sw) {
+  const int ns = (n + 63) >> 6;
+  double cur = w[0], next[kSlots - 1] = {w[1], w[2], w[3]};
+  for (int s = 0; s < ns; ++s) {
+    const int nb = ns - 1 - s;
+    if (nb == 3) forward_segment<T, 3>(L, n, 64 * s, lane, cur, next);
+    else if (nb == 2) forward_segment<T, 2>(L, n, 64 * s, lane, cur, next);
+    else if (nb == 1) forward_segment<T, 1>(L, n, 64 * s, lane, cur, next);
+    else forward_segment<T, 0>(L, n, 64 * s, lane, cur, next);
+    sw[64 * s + lane] = cur;
+    cur = next[0];
+    next[0] = next[1];
+    next[1] = next[2];
   }
-  return r;
+  cur = sw[64 * (ns - 1) + lane];
+#pragma unroll
+  for (int m = 0; m < kSlots - 1; ++m) next[m] = sw[64 * max(ns - 2 - m, 0) + lane];
+  for (int s = ns - 1; s >= 0; --s) {
+    if (s == 3) backward_segment<T, 3>(L, n, 64 * s, lane, cur, next);
+    else if (s == 2) backward_segment<T, 2>(L, n, 64 * s, lane, cur, next);
+    else if (s == 1) backward_segment<T, 1>(L, n, 64 * s, lane, cur, next);
+    else backward_segment<T, 0>(L, n, 64 * s, lane, cur, next);
+    sw[64 * s + lane] = cur;
+    cur = next[0];
+    next[0] = next[1];
+    next[1] = next[2];
+  }
+#pragma unroll
+  for (int m = 0; m < kSlots; ++m) w[m] = sw[64 * m + lane];
 }
 
-// In-register LU solve of one block held by one wave: w <- U^-1 L^-1 w (the
-// factor's L unit lower, U upper, column-major), FP64 arithmetic.
-template <typename T>
-__device__ __forceinline__ void trsv_lu(const T* __restrict__ L, int n, int lane, double (&w)[kSlots]) {
-  // forward: w_i -= L(i, k) w_k for i > k
-  stream_cols(L, n, 0, 1, n - 1, lane, [](int i, int k) { return i > k; },
-              [&](int k, const T (&c)[kSlots]) {
-                const double wk = pick_row(w, k);
+// r -= A y over NS slots, and the rows' sums of |A|; y in LDS.
+template <int NS>
+__device__ __forceinline__ void residual(const double* __restrict__ A, int n, int lane,
+                                         const double* __restrict__ sy, double (&r)[kSlots],
+                                         double (&rowabs)[kSlots]) {
+  unsigned off[NS];
 #pragma unroll
-                for (int m = 0; m < kSlots; ++m) w[m] = fma(-(double)c[m], wk, w[m]);
-              });
-  // backward: w_k /= U(k, k); w_i -= U(i, k) w_k for i < k
-  stream_cols(L, n, n - 1, -1, n, lane, [](int i, int k) { return i <= k; },
-              [&](int k, const T (&c)[kSlots]) {
-                const double ukk = pick_row(c, k);
-                const double wk = pick_row(w, k) / ukk;
+  for (int m = 0; m < NS; ++m) off[m] = (unsigned)min(64 * m + lane, n - 1) * 8u;
+  for (int k0 = 0; k0 < n; k0 += 64) {
+    const int cnt = min(64, n - k0);
+    const double y = sy[k0 + lane];
+    stream_chunks<double, NS>(
+        cnt, r[0],
+        [&](int j0, double (&c)[chunk_cols(NS)][NS]) __attribute__((always_inline)) {
+          load_cols<double, NS>(A, n, k0 + j0, 1, off, c);
+        },
+        [&](auto tail, int j0, const double (&c)[chunk_cols(NS)][NS]) __attribute__((always_inline)) {
 #pragma unroll
-                for (int m = 0; m < kSlots; ++m) {
-                  const int i = 64 * m + lane;
-                  w[m] = (i == k) ? wk : ((i < k) ? fma(-(double)c[m], wk, w[m]) : w[m]);
-                }
-              });
+          for (int u = 0; u < chunk_cols(NS); ++u) {
+            if (decltype(tail)::value && j0 + u >= cnt) break;
+            const double yj = readlane_f64(y, j0 + u);
+#pragma unroll
+            for (int m = 0; m < NS; ++m) {
+              r[m] = fma(-c[u][m], yj, r[m]);
+              rowabs[m] += fabs(c[u][m]);
+            }
+          }
+        });
+  }
 }
 
-template <typename T>
-__global__ void __launch_bounds__(64)
+// REFINE false (no refinement asked for) leaves the residual's registers out:
+// two waves per SIMD instead of one.
+template <typename T, bool REFINE>
+__global__ void __launch_bounds__(64, REFINE ? 1 : 2)
 lu_solve_kernel(const int* __restrict__ n_arr, const long* __restrict__ a_off,
                 const long* __restrict__ x_off, const double* __restrict__ A,
                 const T* __restrict__ LU, const double* __restrict__ rs,
                 const double* __restrict__ cs, const int* __restrict__ perm,
                 const double* x, double* y, int refine, double tol, int* __restrict__ iters) {
+  __shared__ double sw[64 * kSlots];
   const int b = blockIdx.x;
   const int lane = threadIdx.x;
   const int n = n_arr[b];
@@ -686,59 +751,49 @@ lu_solve_kernel(const int* __restrict__ n_arr, const long* __restrict__ a_off,
   }
   const long xo = x_off[b];
   const T* __restrict__ L = LU + a_off[b];
-  const double* __restrict__ Ab = A ? A + a_off[b] : nullptr;
   const int* __restrict__ pm = perm + xo;
 
-  double xv[kSlots], yv[kSlots], w[kSlots], csv[kSlots];
+  // w = P (rs .* x): row i of the factor is row perm[i] of A.
+  int src[kSlots];
+  double w[kSlots], yv[kSlots], xv[kSlots], csv[kSlots];
 #pragma unroll
   for (int m = 0; m < kSlots; ++m) {
     const int i = 64 * m + lane;
-    xv[m] = i < n ? x[xo + i] : 0.0;
+    src[m] = i < n ? min(max(pm[i], 0), n - 1) : 0;
+    w[m] = i < n ? x[xo + src[m]] * (rs ? rs[xo + src[m]] : 1.0) : 0.0;
+    xv[m] = REFINE && i < n ? x[xo + i] : 0.0;
     csv[m] = (cs && i < n) ? cs[xo + i] : 1.0;
   }
-  // w = P (rs .* x): row i of the factor is row perm[i] of A.
-  int src_lane[kSlots], src_slot[kSlots];
-#pragma unroll
-  for (int m = 0; m < kSlots; ++m) {
-    const int i = 64 * m + lane;
-    const int src = i < n ? pm[i] : 0;
-    src_lane[m] = src & 63;
-    src_slot[m] = src >> 6;
-    const double rsv = (rs && i < n) ? rs[xo + i] : 1.0;
-    w[m] = xv[m] * rsv;  // still in A's row order
-  }
-  permute_rows(w, src_lane, src_slot, n, lane);
-  trsv_lu<T>(L, n, lane, w);
-#pragma unroll
-  for (int m = 0; m < kSlots; ++m) yv[m] = w[m] * csv[m];
-
   int it = 0;
   double anorm = -1.0;
   double rprev = 0.0;
-  for (; it < refine; ++it) {
-    // r = x - A y in FP64 (first sweep also measures ||A||_inf)
+  for (bool first = true;; first = false) {
+    trsv_lu<T>(L, n, lane, w, sw);
+#pragma unroll
+    for (int m = 0; m < kSlots; ++m) yv[m] = first ? w[m] * csv[m] : yv[m] + w[m] * csv[m];
+    if (!first) ++it;
+    if (!REFINE || it >= refine) break;
+    // r = x - A y in FP64, and ||A||_inf
+    const double* __restrict__ Ab = A + a_off[b];
     double r[kSlots], rowabs[kSlots];
 #pragma unroll
     for (int m = 0; m < kSlots; ++m) {
       r[m] = xv[m];
       rowabs[m] = 0.0;
+      sw[64 * m + lane] = yv[m];
     }
-    const bool first = anorm < 0.0;
-    stream_cols(Ab, n, 0, 1, n, lane, [](int, int) { return true; },
-                [&](int j, const double (&c)[kSlots]) {
-                  const double yj = pick_row(yv, j);
-#pragma unroll
-                  for (int mm = 0; mm < kSlots; ++mm) {
-                    r[mm] = fma(-c[mm], yj, r[mm]);
-                    if (first) rowabs[mm] += fabs(c[mm]);
-                  }
-                });
+    if (n > 192) residual<4>(Ab, n, lane, sw, r, rowabs);
+    else if (n > 128) residual<3>(Ab, n, lane, sw, r, rowabs);
+    else if (n > 64) residual<2>(Ab, n, lane, sw, r, rowabs);
+    else residual<1>(Ab, n, lane, sw, r, rowabs);
     double rn = 0.0, yn = 0.0, an = 0.0;
 #pragma unroll
     for (int m = 0; m < kSlots; ++m) {
-      rn = fmax(rn, fabs(r[m]));
-      yn = fmax(yn, fabs(yv[m]));
-      an = fmax(an, rowabs[m]);
+      if (64 * m + lane < n) {
+        rn = fmax(rn, fabs(r[m]));
+        yn = fmax(yn, fabs(yv[m]));
+        an = fmax(an, rowabs[m]);
+      }
     }
     rn = wave_max_f64(rn);
     yn = wave_max_f64(yn);
@@ -751,187 +806,19 @@ lu_solve_kernel(const int* __restrict__ n_arr, const long* __restrict__ a_off,
 #pragma unroll
     for (int m = 0; m < kSlots; ++m) {
       const int i = 64 * m + lane;
-      w[m] = r[m] * ((rs && i < n) ? rs[xo + i] : 1.0);
+      sw[i] = r[m] * ((rs && i < n) ? rs[xo + i] : 1.0);
     }
-    permute_rows(w, src_lane, src_slot, n, lane);
-    trsv_lu<T>(L, n, lane, w);
+    __syncthreads();  // one wave: the rows are read across lanes
 #pragma unroll
-    for (int m = 0; m < kSlots; ++m) yv[m] += w[m] * csv[m];
+    for (int m = 0; m < kSlots; ++m) w[m] = 64 * m + lane < n ? sw[src[m]] : 0.0;
+    __syncthreads();
   }
-  if (iters) iters[b] = it;
+  if (iters && lane == 0) iters[b] = it;
 #pragma unroll
   for (int m = 0; m < kSlots; ++m) {
     const int i = 64 * m + lane;
     if (i < n) y[xo + i] = yv[m];
   }
-}
-
-// ---------------------------------------------------------------------------
-// Solve without refinement with the factor staged in LDS: the workgroup's
-// four waves copy the block's packed factor (n^2 entries, at most
-// kLdsSolveBytes) into LDS in 16-byte pieces, all of it in flight at once,
-// and one wave then runs both substitutions out of LDS, where a column costs
-// an LDS read instead of an HBM round trip.  Same arithmetic as
-// lu_solve_kernel with refine = 0 (FP64 substitutions in the same order).
-constexpr int kLdsSolveBytes = 64 * 1024;
-
-// Launch choice set by the autotuner through f3d_lu_set_launch, per
-// precision (0 = FP64, 1 = FP32): whether solves without refinement stage the
-// factor in LDS when it fits.
-static int g_lu_solve_staged[2] = {1, 1};
-
-// Substitutions out of LDS.  The loops run over the 64-row slot ms of the
-// pivot row k as an unrolled constant, so every register of w is addressed
-// statically, and the columns of the next kLdsGroup pivots are read while the
-// current group is applied (LDS latency off the dependent chain).
-constexpr int kLdsGroup = 8;
-
-template <typename T>
-__device__ __forceinline__ void trsv_lu_lds(const T* __restrict__ sL, int n, int lane,
-                                            double (&w)[kSlots]) {
-  constexpr int G = kLdsGroup;
-  // forward: w_i -= L(i, k) w_k for i > k (rows i > k sit in slots >= ms)
-#pragma unroll
-  for (int ms = 0; ms < kSlots; ++ms) {
-    const int k0 = 64 * ms, kend = min(64 * ms + 64, n - 1);
-    if (k0 >= kend) continue;
-    T cur[G][kSlots], nxt[G][kSlots];
-    auto load = [&](int kg, T (&buf)[G][kSlots]) __attribute__((always_inline)) {
-#pragma unroll
-      for (int u = 0; u < G; ++u)
-#pragma unroll
-        for (int m = ms; m < kSlots; ++m) {
-          const int k = kg + u, i = 64 * m + lane;
-          buf[u][m] = (k < kend && i > k && i < n) ? sL[(long)k * n + i] : (T)0;
-        }
-    };
-    load(k0, cur);
-    for (int kg = k0; kg < kend; kg += G) {
-      if (kg + G < kend) load(kg + G, nxt);
-#pragma unroll
-      for (int u = 0; u < G; ++u) {
-        if (kg + u < kend) {
-          const double wk = readlane_f64(w[ms], (kg + u) & 63);
-#pragma unroll
-          for (int m = ms; m < kSlots; ++m) w[m] = fma(-(double)cur[u][m], wk, w[m]);
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < G; ++u)
-#pragma unroll
-        for (int m = ms; m < kSlots; ++m) cur[u][m] = nxt[u][m];
-    }
-  }
-  // backward: w_k /= U(k, k); w_i -= U(i, k) w_k for i < k (slots <= ms)
-#pragma unroll
-  for (int ms = kSlots - 1; ms >= 0; --ms) {
-    const int khi = min(64 * ms + 63, n - 1), klo = 64 * ms;
-    if (khi < klo) continue;
-    T cur[G][kSlots], nxt[G][kSlots];
-    double dg[G], dn[G];
-    auto load = [&](int kg, T (&buf)[G][kSlots], double (&d)[G]) __attribute__((always_inline)) {
-#pragma unroll
-      for (int u = 0; u < G; ++u) {
-        const int k = kg - u;
-#pragma unroll
-        for (int m = 0; m <= ms; ++m) {
-          const int i = 64 * m + lane;
-          buf[u][m] = (k >= klo && i < k) ? sL[(long)k * n + i] : (T)0;
-        }
-        d[u] = k >= klo ? (double)sL[(long)k * n + k] : 1.0;
-      }
-    };
-    load(khi, cur, dg);
-    for (int kg = khi; kg >= klo; kg -= G) {
-      if (kg - G >= klo) load(kg - G, nxt, dn);
-#pragma unroll
-      for (int u = 0; u < G; ++u) {
-        const int k = kg - u;
-        if (k >= klo) {
-          const double wk = readlane_f64(w[ms], k & 63) / dg[u];
-#pragma unroll
-          for (int m = 0; m <= ms; ++m) {
-            const int i = 64 * m + lane;
-            w[m] = (i == k) ? wk : ((i < k) ? fma(-(double)cur[u][m], wk, w[m]) : w[m]);
-          }
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < G; ++u) {
-        dg[u] = dn[u];
-#pragma unroll
-        for (int m = 0; m <= ms; ++m) cur[u][m] = nxt[u][m];
-      }
-    }
-  }
-}
-
-template <typename T>
-__global__ void __launch_bounds__(256)
-lu_solve_lds_kernel(int nmax, const int* __restrict__ n_arr, const long* __restrict__ a_off,
-                    const long* __restrict__ x_off, const T* __restrict__ LU,
-                    const double* __restrict__ rs, const double* __restrict__ cs,
-                    const int* __restrict__ perm, const double* __restrict__ x,
-                    double* __restrict__ y, int* __restrict__ iters) {
-  extern __shared__ __align__(16) unsigned char lds_solve[];
-  T* __restrict__ sL = reinterpret_cast<T*>(lds_solve);
-  const int b = blockIdx.x, t = threadIdx.x, lane = t & 63;
-  const int n = n_arr[b];
-  // the whole workgroup leaves together (n is uniform), before any barrier;
-  // the launch sized the LDS for nmax
-  if (n < 1 || n > nmax) {
-    if (iters && t == 0) iters[b] = -1;
-    return;
-  }
-  const T* __restrict__ L = LU + a_off[b];
-  const long nn = (long)n * n;
-  if ((reinterpret_cast<uintptr_t>(L) & 15) == 0) {
-    constexpr int per = 16 / (int)sizeof(T);
-    const long nv = nn / per;
-    const uint4* __restrict__ src = reinterpret_cast<const uint4*>(L);
-    uint4* __restrict__ dst = reinterpret_cast<uint4*>(sL);
-    long e0 = t;
-    for (; e0 + 256 * 7 < nv; e0 += 256 * 8) {
-      uint4 v0 = src[e0], v1 = src[e0 + 256], v2 = src[e0 + 512], v3 = src[e0 + 768];
-      uint4 v4 = src[e0 + 1024], v5 = src[e0 + 1280], v6 = src[e0 + 1536], v7 = src[e0 + 1792];
-      dst[e0] = v0;
-      dst[e0 + 256] = v1;
-      dst[e0 + 512] = v2;
-      dst[e0 + 768] = v3;
-      dst[e0 + 1024] = v4;
-      dst[e0 + 1280] = v5;
-      dst[e0 + 1536] = v6;
-      dst[e0 + 1792] = v7;
-    }
-    for (; e0 < nv; e0 += 256) dst[e0] = src[e0];
-    for (long e = nv * per + t; e < nn; e += 256) sL[e] = L[e];
-  } else {
-    for (long e = t; e < nn; e += 256) sL[e] = L[e];
-  }
-  __syncthreads();
-  if (t >= 64) return;
-
-  const long xo = x_off[b];
-  const int* __restrict__ pm = perm + xo;
-  double w[kSlots];
-  int src_lane[kSlots], src_slot[kSlots];
-#pragma unroll
-  for (int m = 0; m < kSlots; ++m) {
-    const int i = 64 * m + lane;
-    const int sidx = i < n ? pm[i] : 0;
-    src_lane[m] = sidx & 63;
-    src_slot[m] = sidx >> 6;
-    const double rsv = (rs && i < n) ? rs[xo + i] : 1.0;
-    w[m] = (i < n ? x[xo + i] : 0.0) * rsv;  // still in A's row order
-  }
-  permute_rows(w, src_lane, src_slot, n, lane);
-  trsv_lu_lds<T>(sL, n, lane, w);
-#pragma unroll
-  for (int m = 0; m < kSlots; ++m) {
-    const int i = 64 * m + lane;
-    if (i < n) y[xo + i] = w[m] * ((cs && i < n) ? cs[xo + i] : 1.0);
-  }
-  if (iters && lane == 0) iters[b] = 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1175,36 +1062,26 @@ extern "C" int f3d_lu_solve_batched(int precision, int64_t nb, int32_t nmax, con
   F3D_REQUIRE(n && a_off && x_off && perm && x && y, F3D_EINVAL, "lu_solve: NULL argument");
   F3D_REQUIRE(refine == 0 || A != nullptr, F3D_EINVAL, "lu_solve: refinement needs A");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  // without refinement, factors that fit the LDS budget are staged there
-  const size_t elem = precision == F3D_F64 ? sizeof(double) : sizeof(float);
-  const size_t lds = align_up((size_t)nmax * nmax * elem, 16);
-  // F3D_LU_SOLVE_STREAM=1 keeps the streaming kernel (for comparison)
-  const char* force_stream = getenv("F3D_LU_SOLVE_STREAM");
-  const bool staged = refine == 0 && lds <= (size_t)kLdsSolveBytes &&
-                      g_lu_solve_staged[precision == F3D_F64 ? 0 : 1] &&
-                      !(force_stream && *force_stream && *force_stream != '0');
-  if (staged && precision == F3D_F64) {
-    F3D_REQUIRE(lu64 != nullptr, F3D_EINVAL, "lu_solve: lu64 is NULL");
-    F3D_LAUNCH((lu_solve_lds_kernel<double>), dim3((unsigned)nb), dim3(256), lds, st, nmax,
-               n, (const long*)a_off, (const long*)x_off, lu64, rs, cs, perm, x, y, iters);
-    return F3D_OK;
-  }
-  if (staged) {
-    F3D_REQUIRE(lu32 && rs && cs, F3D_EINVAL, "lu_solve: lu32/rs/cs is NULL");
-    F3D_LAUNCH((lu_solve_lds_kernel<float>), dim3((unsigned)nb), dim3(256), lds, st, nmax,
-               n, (const long*)a_off, (const long*)x_off, lu32, rs, cs, perm, x, y, iters);
-    return F3D_OK;
-  }
   if (precision == F3D_F64) {
     F3D_REQUIRE(lu64 != nullptr, F3D_EINVAL, "lu_solve: lu64 is NULL");
-    F3D_LAUNCH((lu_solve_kernel<double>), dim3((unsigned)nb), dim3(64), 0, st, n,
-               (const long*)a_off, (const long*)x_off, A, lu64, rs, cs, perm, x, y, refine, tol,
-               iters);
+    if (refine > 0)
+      F3D_LAUNCH((lu_solve_kernel<double, true>), dim3((unsigned)nb), dim3(64), 0, st, n,
+                 (const long*)a_off, (const long*)x_off, A, lu64, rs, cs, perm, x, y, refine, tol,
+                 iters);
+    else
+      F3D_LAUNCH((lu_solve_kernel<double, false>), dim3((unsigned)nb), dim3(64), 0, st, n,
+                 (const long*)a_off, (const long*)x_off, A, lu64, rs, cs, perm, x, y, refine, tol,
+                 iters);
   } else {
     F3D_REQUIRE(lu32 && rs && cs, F3D_EINVAL, "lu_solve: lu32/rs/cs is NULL");
-    F3D_LAUNCH((lu_solve_kernel<float>), dim3((unsigned)nb), dim3(64), 0, st, n,
-               (const long*)a_off, (const long*)x_off, A, lu32, rs, cs, perm, x, y, refine, tol,
-               iters);
+    if (refine > 0)
+      F3D_LAUNCH((lu_solve_kernel<float, true>), dim3((unsigned)nb), dim3(64), 0, st, n,
+                 (const long*)a_off, (const long*)x_off, A, lu32, rs, cs, perm, x, y, refine, tol,
+                 iters);
+    else
+      F3D_LAUNCH((lu_solve_kernel<float, false>), dim3((unsigned)nb), dim3(64), 0, st, n,
+                 (const long*)a_off, (const long*)x_off, A, lu32, rs, cs, perm, x, y, refine, tol,
+                 iters);
   }
   return F3D_OK;
 }
@@ -1213,13 +1090,11 @@ extern "C" int f3d_lu_set_launch(int precision, int32_t factor_waves_per_cu,
                                  int32_t solve_staged) {
   F3D_REQUIRE(precision == F3D_F64 || precision == F3D_F32C, F3D_EINVAL,
               "lu_set_launch: unknown precision %d", precision);
-  const int pp = precision == F3D_F64 ? 0 : 1;
-  const int cap = pp == 0 ? 4 : 8;
+  const int cap = precision == F3D_F64 ? 4 : 8;
   F3D_REQUIRE(factor_waves_per_cu >= 0 && factor_waves_per_cu <= cap, F3D_EINVAL,
               "lu_set_launch: waves per CU %d outside [0, %d]", factor_waves_per_cu, cap);
   F3D_REQUIRE(solve_staged == 0 || solve_staged == 1, F3D_EINVAL,
               "lu_set_launch: solve_staged must be 0 or 1");
-  g_lu_solve_staged[pp] = solve_staged;
   return F3D_OK;
 }
 

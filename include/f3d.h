@@ -87,11 +87,11 @@ int f3d_pairsum_plan(int kernel, int precision, int64_t ns, int64_t nt, int32_t*
 
 /*
  * Launch choices of the batched LU for one precision (F3D_F64 or F3D_F32C):
- * waves per CU of the factorisation (1..4 for FP64, 1..8 for FP32, 0;
- * checked, but without effect: one workgroup per block, scheduled by the
- * hardware), and whether solves without refinement
- * stage the factor in LDS when it fits in 64 KB (1, the default) or stream
- * it from HBM (0).  Set by the autotuner; no reference counterpart.
+ * waves per CU of the factorisation (1..4 for FP64, 1..8 for FP32, or 0) and
+ * whether solves without refinement stage the factor in LDS (0 or 1).  Both
+ * are checked and have no effect: the factorisation runs one workgroup per
+ * block, scheduled by the hardware, and the streaming solve is the faster one
+ * at every size.  No reference counterpart.
  */
 int f3d_lu_set_launch(int precision, int32_t factor_waves_per_cu, int32_t solve_staged);
 

@@ -111,6 +111,49 @@ def test_lu_solve_batched(precision):
     assert rel2(bb.cpu().numpy(), np.concatenate(xs)) < tol
 
 
+@pytest.mark.parametrize("precision", ["f64", "f32c"])
+def test_lu_solve_segment_edges(precision):
+    """One unrefined solve at the edges of the substitutions' 64-row segments
+    and column chunks: the backward error of L U z = P (rs x), y = cs z with
+    the kernel's own factors, element by element (3 n eps |L| |U| |z|)."""
+    print(f"case lu solve segment edges {precision}", flush=True)
+    sizes = [1, 2, 3, 5, 8, 63, 64, 65, 72, 80, 127, 128, 129, 135, 191, 192, 193, 200, 255, 256]
+    mats = _mats(sizes, 11)
+    bs = BlockSet(sizes)
+    lu = BatchedLU(bs, bs.pack(mats), precision=precision, refine=0)
+    x = np.random.default_rng(12).normal(size=bs.nrows)
+    y = lu.solve(torch.from_numpy(x).cuda()).cpu().numpy()
+    LU = bs.unpack((lu.lu64 if precision == "f64" else lu.lu32).double())
+    perm = lu.perm.cpu().numpy()
+    for k, n in enumerate(sizes):
+        rows = slice(bs.x_off_h[k], bs.x_off_h[k] + n)
+        rs, cs = (np.ones(n), np.ones(n)) if precision == "f64" else (
+            lu.rs.cpu().numpy()[rows], lu.cs.cpu().numpy()[rows])
+        Lo, U = np.tril(LU[k], -1) + np.eye(n), np.triu(LU[k])
+        z = y[rows] / cs
+        r = Lo @ (U @ z) - (rs * x[rows])[perm[rows]]
+        bound = 3 * n * 2.0 ** -53 * (np.abs(Lo) @ (np.abs(U) @ np.abs(z)))
+        assert (np.abs(r) <= bound).all(), n
+
+
+def test_lu_solve_quotients_outside_the_safe_range():
+    """Diagonal blocks whose pivots or right-hand sides lie where the
+    reciprocal form of the quotient is not exact: the same numbers as a
+    division, infinities and NaN included (the extreme pivots to 2 ulp)."""
+    print("case lu solve quotients", flush=True)
+    d = np.array([3.0, 7e200, 5e-201, 0.0, np.inf, 1.1e150, 3e-130, np.nan])
+    x = np.array([1.0, 2.0, 3.0, 1.0, 2.0, 1e300, np.inf, 1.0])
+    sizes = [1] * len(d)
+    bs = BlockSet(sizes)
+    lu = BatchedLU(bs, bs.pack([np.array([[v]]) for v in d]), precision="f64", refine=0)
+    y = lu.solve(torch.from_numpy(x).cuda()).cpu().numpy()
+    with np.errstate(divide="ignore", invalid="ignore"):
+        ref = x / d
+    fin = np.isfinite(ref)
+    np.testing.assert_allclose(y[fin], ref[fin], rtol=2.0 ** -51, atol=0)
+    np.testing.assert_array_equal(y[~fin], ref[~fin])
+
+
 def test_lu_zero_pivot_info():
     M = np.eye(8)
     M[3, 3] = 0.0
