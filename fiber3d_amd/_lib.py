@@ -75,6 +75,17 @@ SIGNATURES = {
     "f3d_gemm_bf16": (ctypes.c_int, [
         ctypes.c_int, _i64, _i64, _i64, _i32, _c_p, _i64, _i64, _c_p, _i64, _i64,
         _c_p, _i64, _i64, _c_p, _c_p, _c_p, ctypes.c_float, _c_p]),
+    "f3d_mse_workspace_size": (_sz, []),
+    "f3d_mse": (ctypes.c_int, [_i64, _c_p, _c_p, _c_p, _c_p, _c_p, _sz, _c_p]),
+    "f3d_adam": (ctypes.c_int, [_i32, _c_p, _c_p, _c_p, _c_p, _c_p, _f64, _f64, _f64, _f64, _i64,
+                                _c_p]),
+    "f3d_mlp_workspace_size": (_sz, [_i64, _i32, _i32, _i32]),
+    "f3d_mlp_forward": (ctypes.c_int, [
+        _i64, _i32, _i32, _i32, _c_p, _i64, _i64, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p,
+        _c_p, _c_p, _c_p, _c_p]),
+    "f3d_mlp_backward": (ctypes.c_int, [
+        _i64, _i32, _i32, _i32, _c_p, _i64, _i64, _c_p, _c_p, _c_p, _i64, _i64, _c_p, _c_p,
+        _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _sz, _c_p]),
     "f3d_fiber_assemble": (ctypes.c_int, [
         _i64, _i32, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p,
         _f64, _f64, _f64, _f64, _f64, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p]),

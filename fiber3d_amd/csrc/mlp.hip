@@ -7,83 +7,205 @@
 //   rounded to BF16 -- round to nearest even -- when staged into LDS);
 //   C(m, n) = C[m*scm + n*scn] (FP32).
 //
-// General tiling for CDNA4 (any shape, K splits): a 256-thread workgroup owns
-// a 64 x 64 tile of C; each wave owns a 32 x 32 quarter and issues
-// v_mfma_f32_32x32x16_bf16 on 16-deep
-// K slices staged through LDS (A row-major, B transposed so both fragments
-// are 16-byte contiguous LDS reads).  grid.z splits K for the weight-gradient
-// products (K = number of nodes), whose tiles are then added atomically.
-// The per-node layers (N = 128 or 256, K <= 256) take the streaming kernel
-// below.
+// General tiling for CDNA4 (any shape and strides, K splits): a 256-thread
+// workgroup owns a 64 x 64 tile of C; each wave owns a 32 x 32 quarter and
+// issues v_mfma_f32_32x32x16_bf16 on 64-deep K chunks, double buffered in LDS
+// (both operands with K contiguous, so a fragment is one 16-byte read).  An
+// operand is loaded along its unit-stride direction, 256 bytes of a row at a
+// time, with float4 where it is aligned: along K, or along its rows with
+// pairs of K packed on the way into LDS.
+// (Loading both operands element by element with K fastest, whatever their
+// strides, was bound by uncoalesced reads of the transposed ones: 103-130 us
+// for a gradient product of 8192 samples at 256 x 256.)
+// The weight gradients A^T B (K = number of samples) split K over grid.y into
+// partial sums that a second kernel adds in a fixed order, with the column sums
+// of B (the bias gradients) from the same pass over B; all layers are one
+// launch: 22 + 4 us for 23 -> 256 -> 256 -> 4 at 8192 samples (three products
+// with atomic sums and three column sums took 360).
+// The per-node layers (N = 128 or 256, K <= 256) of many rows take the
+// streaming or resident kernels below.
 #include "common.h"
+
+#include <math.h>
 
 namespace f3d {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
-constexpr int kMT = 64, kNT = 64, kKT = 16;
+constexpr int kMT = 64, kNT = 64, kKT = 64;
+constexpr int kTP = kKT + 8;  // LDS row pitch (bf16): 144 B, 16-byte aligned
 
-__device__ __forceinline__ unsigned short f2bf(float f) {
-  unsigned u = __float_as_uint(f);
-  if ((u & 0x7f800000u) == 0x7f800000u) return (unsigned short)(u >> 16);  // inf / nan
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (unsigned short)(u >> 16);
+// two values, round to nearest even (one v_cvt_pk_bf16_f32)
+__device__ __forceinline__ unsigned pack_bf16(float lo, float hi) {
+  const f32x2_t v = {lo, hi};
+  return __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2_t));
 }
 
 // epilogue modes
 enum { EPI_STORE = 0, EPI_BIAS_RELU = 1, EPI_RELU_GRAD = 2, EPI_ATOMIC = 3, EPI_BIAS = 4 };
 
-template <int EPI>
-__global__ void __launch_bounds__(256)
-gemm_bf16_kernel(int M, int N, int K, int kchunk, const float* __restrict__ A, long sam,
-                 long sak, const float* __restrict__ B, long sbk, long sbn,
-                 float* __restrict__ C, long scm, long scn, const float* __restrict__ bias,
-                 float* __restrict__ Z, const float* __restrict__ Zin, float alpha) {
-  __shared__ __attribute__((aligned(16))) unsigned short As[kMT][kKT + 8];
-  __shared__ __attribute__((aligned(16))) unsigned short Bt[kNT][kKT + 8];
+// One operand of a tile: entry (r, k) at p[r * sr + k * sk], r < R.
+struct TileOperand {
+  const float* p;
+  long sr, sk;
+  int R;
+};
+
+// Registers of one chunk (64 rows x 64 k): 16 values per thread.
+// KC (K contiguous): row tid / 4, 16 consecutive k.  Otherwise (rows
+// contiguous): two items of two k and four rows each.
+template <bool KC>
+__device__ __forceinline__ void tile_load(const TileOperand& o, bool vec, int r0, int k0, int kend,
+                                          float (&v)[16]) {
   const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
+  if constexpr (KC) {
+    const int r = r0 + (tid >> 2), k = k0 + 16 * (tid & 3);
+    const float* __restrict__ p = o.p + (long)min(r, o.R - 1) * o.sr + (long)k * o.sk;
+    const bool in = r < o.R;
+    if (vec && in && k + 16 <= kend) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float4 f = reinterpret_cast<const float4*>(p)[q];
+        v[4 * q] = f.x; v[4 * q + 1] = f.y; v[4 * q + 2] = f.z; v[4 * q + 3] = f.w;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) v[i] = in && k + i < kend ? p[(long)i * o.sk] : 0.0f;
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int item = tid + 256 * e;
+      const int r = r0 + 4 * (item & 15), k = k0 + 2 * (item >> 4);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int w = 8 * e + 4 * h;
+        const float* __restrict__ p = o.p + (long)min(k + h, kend - 1) * o.sk + (long)r * o.sr;
+        const bool in = k + h < kend;
+        float4 f;
+        if (vec && in && r + 4 <= o.R) {
+          f = *reinterpret_cast<const float4*>(p);
+        } else {
+          f.x = in && r < o.R ? p[0] : 0.0f;
+          f.y = in && r + 1 < o.R ? p[o.sr] : 0.0f;
+          f.z = in && r + 2 < o.R ? p[2 * o.sr] : 0.0f;
+          f.w = in && r + 3 < o.R ? p[3 * o.sr] : 0.0f;
+        }
+        v[w] = f.x;
+        v[w + 1] = f.y;
+        v[w + 2] = f.z;
+        v[w + 3] = f.w;
+      }
+    }
+  }
+}
+
+template <bool KC>
+__device__ __forceinline__ void tile_store(unsigned short (&s)[kMT][kTP], const float (&v)[16]) {
+  const int tid = threadIdx.x;
+  if constexpr (KC) {
+    uint4* d = reinterpret_cast<uint4*>(&s[tid >> 2][16 * (tid & 3)]);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const float* w = v + 8 * q;
+      d[q] = make_uint4(pack_bf16(w[0], w[1]), pack_bf16(w[2], w[3]), pack_bf16(w[4], w[5]),
+                        pack_bf16(w[6], w[7]));
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int item = tid + 256 * e;
+      const int r = 4 * (item & 15), k = 2 * (item >> 4);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        *reinterpret_cast<unsigned*>(&s[r + i][k]) = pack_bf16(v[8 * e + i], v[8 * e + 4 + i]);
+    }
+  }
+}
+
+// Whether float4 loads along the unit-stride direction are aligned.
+__device__ __forceinline__ bool tile_vec(const TileOperand& o, bool kc) {
+  const long unit = kc ? o.sk : o.sr, other = kc ? o.sr : o.sk;
+  return unit == 1 && ((reinterpret_cast<uintptr_t>(o.p) | (uintptr_t)(other * 4)) & 15) == 0;
+}
+
+struct TileShared {
+  __attribute__((aligned(16))) unsigned short a[2][kMT][kTP];
+  __attribute__((aligned(16))) unsigned short b[2][kNT][kTP];
+};
+
+// acc (this wave's 32 x 32 quarter) = sum over k in [kbeg, kend) of
+// A(m0 + .., k) B(k, n0 + ..); colsum: this thread's column sums of B (rows-
+// contiguous B: columns 4 (tid % 16) .. + 3) when wanted.
+template <bool AKC, bool BKC, bool SUM>
+__device__ __forceinline__ f32x16_t tile_product(TileShared& sh, const TileOperand& A,
+                                                 const TileOperand& B, int m0, int n0, int kbeg,
+                                                 int kend, float (&colsum)[4]) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave >> 1, wn = wave & 1;
-  const int m0 = blockIdx.y * kMT, n0 = blockIdx.x * kNT;
-  const int kbeg = blockIdx.z * kchunk;
-  const int kend = min(K, kbeg + kchunk);
+  const bool va = tile_vec(A, AKC), vb = tile_vec(B, BKC);
   f32x16_t acc;
 #pragma unroll
   for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
-
-  for (int k0 = kbeg; k0 < kend; k0 += kKT) {
-    // stage A (64 x 16) and B^T (64 x 16): 4 elements per thread each
+  float ra[16], rb[16];
+  auto load = [&](int k0) __attribute__((always_inline)) {
+    tile_load<AKC>(A, va, m0, k0, kend, ra);
+    tile_load<BKC>(B, vb, n0, k0, kend, rb);
+  };
+  auto store = [&](int buf) __attribute__((always_inline)) {
+    tile_store<AKC>(sh.a[buf], ra);
+    tile_store<BKC>(sh.b[buf], rb);
+    if constexpr (SUM) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int idx = tid + 256 * e;   // 0..1023
-      const int r = idx >> 4, kk = idx & 15;
-      const int m = m0 + r, k = k0 + kk;
-      float va = (m < M && k < kend) ? A[(long)m * sam + (long)k * sak] : 0.0f;
-      As[r][kk] = f2bf(va);
-      const int n = n0 + r;
-      float vb = (n < N && k < kend) ? B[(long)k * sbk + (long)n * sbn] : 0.0f;
-      Bt[r][kk] = f2bf(vb);
+      for (int i = 0; i < 4; ++i) colsum[i] += (rb[i] + rb[4 + i]) + (rb[8 + i] + rb[12 + i]);
     }
-    __syncthreads();
-    const int row = 32 * wm + (lane & 31);
-    const int col = 32 * wn + (lane & 31);
-    const int kofs = 8 * (lane >> 5);
-    // 16-byte LDS reads (row pitch 48 B, offsets 0 / 16 B: aligned)
-    const bf16x8_t a = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(&As[row][kofs]));
-    const bf16x8_t b = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(&Bt[col][kofs]));
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+  };
+  if (kbeg >= kend) return acc;
+  load(kbeg);
+  store(0);
+  __syncthreads();
+  int buf = 0;
+  for (int k0 = kbeg; k0 < kend; k0 += kKT, buf ^= 1) {
+    const bool more = k0 + kKT < kend;
+    if (more) load(k0 + kKT);  // in flight during the MFMAs
+    const int row = 32 * wm + (lane & 31), col = 32 * wn + (lane & 31);
+#pragma unroll
+    for (int ks = 0; ks < kKT; ks += 16) {
+      const int kofs = ks + 8 * (lane >> 5);
+      const bf16x8_t a =
+          __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(&sh.a[buf][row][kofs]));
+      const bf16x8_t b =
+          __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(&sh.b[buf][col][kofs]));
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+    }
+    if (more) store(buf ^ 1);
     __syncthreads();
   }
+  return acc;
+}
 
+template <int EPI, bool AKC, bool BKC>
+__global__ void __launch_bounds__(256)
+gemm_bf16_kernel(TileOperand A, TileOperand B, int K, int kchunk, float* __restrict__ C, long scm,
+                 long scn, const float* __restrict__ bias, float* __restrict__ Z,
+                 const float* __restrict__ Zin, float alpha) {
+  __shared__ TileShared sh;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int m0 = blockIdx.y * kMT, n0 = blockIdx.x * kNT;
+  const int kbeg = blockIdx.z * kchunk;
+  float unused[4];
+  const f32x16_t acc =
+      tile_product<AKC, BKC, false>(sh, A, B, m0, n0, kbeg, min(K, kbeg + kchunk), unused);
   // C layout of the 32 x 32 MFMA: register i of lane l holds
   // row 8*(i/4) + 4*(l/32) + i%4, column l%32.
-  const int n = n0 + 32 * wn + (lane & 31);
+  const int n = n0 + 32 * (wave & 1) + (lane & 31);
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
-    const int m = m0 + 32 * wm + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-    if (m >= M || n >= N) continue;
+    const int m = m0 + 32 * (wave >> 1) + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+    if (m >= A.R || n >= B.R) continue;
     float v = alpha * acc[i];
     const long ci = (long)m * scm + (long)n * scn;
     if (EPI == EPI_ATOMIC) {
@@ -104,6 +226,80 @@ gemm_bf16_kernel(int M, int N, int K, int kchunk, const float* __restrict__ A, l
 }
 
 // ---------------------------------------------------------------------------
+// Weight and bias gradients of several layers in one launch: layer l's
+// W = A^T B (A: K x M, B: K x N) and b = column sums of B, K = samples, over
+// one K slice per grid.y; partial sums at ws[slice * total + off + m * N + n]
+// (weights) and ... + off + M * N + n (biases).
+constexpr int kGradLayers = 3;
+struct GradLayer {
+  TileOperand a, b;  // rows: m (a), n (b)
+  int tile0, tiles_n;
+  long off;
+  float* w;   // the layer's gradients, dense
+  float* bs;
+};
+struct GradPlan {
+  GradLayer l[kGradLayers];
+  int K, kchunk, slices;
+  long total;
+};
+
+__global__ void __launch_bounds__(256)
+grad_partial_kernel(GradPlan p, float* __restrict__ ws) {
+  __shared__ TileShared sh;
+  int li = 0;
+#pragma unroll
+  for (int i = 1; i < kGradLayers; ++i)
+    if ((int)blockIdx.x >= p.l[i].tile0) li = i;
+  const GradLayer& L = p.l[li];
+  const int t = (int)blockIdx.x - L.tile0;
+  const int m0 = (t / L.tiles_n) * kMT, n0 = (t % L.tiles_n) * kNT;
+  const int kbeg = blockIdx.y * p.kchunk, kend = min(p.K, kbeg + p.kchunk);
+  float cs[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  const f32x16_t acc = tile_product<false, false, true>(sh, L.a, L.b, m0, n0, kbeg, kend, cs);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int M = L.a.R, N = L.b.R;
+  float* __restrict__ out = ws + blockIdx.y * p.total + L.off;
+  const int n = n0 + 32 * (wave & 1) + (lane & 31);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int m = m0 + 32 * (wave >> 1) + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
+    if (m < M && n < N) out[(long)m * N + n] = acc[i];
+  }
+  if (m0 == 0) {
+    // the 16 threads of a column quad, in a fixed order
+    float* __restrict__ red = reinterpret_cast<float*>(&sh);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) red[(threadIdx.x >> 4) * 64 + 4 * (threadIdx.x & 15) + i] = cs[i];
+    __syncthreads();
+    if (threadIdx.x < 64 && n0 + (int)threadIdx.x < N) {
+      float s = 0.0f;
+#pragma unroll
+      for (int q = 0; q < 16; ++q) s += red[q * 64 + threadIdx.x];
+      out[(long)M * N + n0 + threadIdx.x] = s;
+    }
+  }
+}
+
+__global__ void __launch_bounds__(256)
+grad_reduce_kernel(GradPlan p, const float* __restrict__ ws) {
+  const long i = (long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= p.total) return;
+  float s = 0.0f;
+#pragma unroll 8
+  for (int q = 0; q < p.slices; ++q) s += ws[q * p.total + i];
+  int li = 0;
+#pragma unroll
+  for (int l = 1; l < kGradLayers; ++l)
+    if (i >= p.l[l].off) li = l;
+  const GradLayer& L = p.l[li];
+  const long e = i - L.off, mn = (long)L.a.R * L.b.R;
+  if (e < mn) L.w[e] = s;
+  else L.bs[e - mn] = s;
+}
+
+// ---------------------------------------------------------------------------
 // Streaming path for the per-node layers (M = nodes, large; N = 64 NT up to
 // 256; K <= 256): a workgroup owns 128 rows and ALL N columns, so every
 // activation row is read from HBM once and written once.  2 x NT waves, each
@@ -115,6 +311,7 @@ gemm_bf16_kernel(int M, int N, int K, int kchunk, const float* __restrict__ A, l
 // every A fragment across the wave's two column tiles and every B fragment
 // across its two row tiles.
 constexpr int kSM = 128;  // rows per workgroup
+constexpr int kStreamRows = 49152;  // fewer rows take the tiled kernel
 constexpr int kSK = 32;   // K chunk
 constexpr int kSP = kSK + 8;  // LDS row pitch (bf16 elements): 80 B, 16-byte aligned
 
@@ -188,9 +385,7 @@ gemm_bf16_stream_kernel(int M, int N, int K, const float* __restrict__ A, long s
       }
     }
   };
-  auto pack2 = [](float lo, float hi) __attribute__((always_inline)) {
-    return (unsigned)f2bf(lo) | ((unsigned)f2bf(hi) << 16);
-  };
+  auto pack2 = [](float lo, float hi) __attribute__((always_inline)) { return pack_bf16(lo, hi); };
   auto store = [&](int buf) __attribute__((always_inline)) {
     const int r = tid / NT, kh = (tid % NT) * AK;
 #pragma unroll
@@ -307,9 +502,7 @@ gemm_bf16_resident_kernel(int M, int N, int K, const float* __restrict__ A, long
   const int pieces = RM * K4;                 // per block (<= 512 PP)
   const int nblocks = (M + RM - 1) / RM;
 
-  auto pack2 = [](float lo, float hi) __attribute__((always_inline)) {
-    return (unsigned)f2bf(lo) | ((unsigned)f2bf(hi) << 16);
-  };
+  auto pack2 = [](float lo, float hi) __attribute__((always_inline)) { return pack_bf16(lo, hi); };
   // A pieces of block bl into registers: piece q = tid + 512 j is row q / K4,
   // columns 4 (q % K4) ..; rows past M and pieces past the block read row 0
   // (in bounds) and are zeroed when staged.
@@ -478,11 +671,15 @@ extern "C" int f3d_gemm_bf16(int epi, int64_t M, int64_t N, int64_t K, int32_t k
   if (M == 0 || N == 0) return F3D_OK;
   F3D_REQUIRE(A && B && C, F3D_EINVAL, "gemm_bf16: NULL operand");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  // the streaming path: row-major A (unit K stride) and C (unit N stride),
-  // N in {128, 256}, K <= 256, no K split
+  // the streaming paths: row-major A (unit K stride) and C (unit N stride),
+  // N in {128, 256}, 16 < K <= 256, no K split, from kStreamRows rows on.
+  // Fewer rows leave CUs idle or pay B's set-up for a block or two: at 256 x
+  // 256, 8192 rows take 15 us tiled, 26 streaming, 39 resident; 32768 rows 39,
+  // 33, 47; 65536 rows 73, 61, 55; 262144 rows 288, 253, 130.  (At K = 4 the
+  // tiled kernel is the fastest at every size: 174 against 220 us at 262144.)
   const int mode = (N == 128 || N == 256) ? g_gemm_stream[N == 256 ? 1 : 0] : 0;
   const bool stream_ok = epi != EPI_ATOMIC && ksplit == 1 && sak == 1 && scn == 1 && mode > 0 &&
-                         K <= 256 && M >= kSM;
+                         K > 16 && K <= 256 && M >= kStreamRows;
   // the resident-weight path also needs K a multiple of 16 and 16-byte rows of A
   const bool resident_ok = stream_ok && mode == 2 && K > 0 && K % 16 == 0 && sam % 4 == 0 &&
                            (reinterpret_cast<uintptr_t>(A) & 15) == 0;
@@ -522,10 +719,20 @@ extern "C" int f3d_gemm_bf16(int epi, int64_t M, int64_t N, int64_t K, int32_t k
   kchunk = (int64_t)align_up((size_t)kchunk, kKT);
   const unsigned gz = (unsigned)ceil_div(K > 0 ? K : 1, kchunk);
   const dim3 grid((unsigned)ceil_div(N, kNT), (unsigned)ceil_div(M, kMT), gz);
-#define F3D_G(E)                                                                            \
-  F3D_LAUNCH((gemm_bf16_kernel<E>), grid, dim3(256), 0, st, (int)M, (int)N, (int)K,         \
-             (int)kchunk, A, (long)sam, (long)sak, B, (long)sbk, (long)sbn, C, (long)scm,   \
-             (long)scn, bias, Z, Zin, alpha)
+  // each operand along its unit-stride direction (along K where both are or
+  // neither is)
+  const TileOperand oa{A, (long)sam, (long)sak, (int)M}, ob{B, (long)sbn, (long)sbk, (int)N};
+  const bool akc = sak == 1 || sam != 1, bkc = sbk == 1 || sbn != 1;
+#define F3D_GK(E, X, Y)                                                                     \
+  F3D_LAUNCH((gemm_bf16_kernel<E, X, Y>), grid, dim3(256), 0, st, oa, ob, (int)K, (int)kchunk, \
+             C, (long)scm, (long)scn, bias, Z, Zin, alpha)
+#define F3D_G(E)                                   \
+  do {                                             \
+    if (akc && bkc) F3D_GK(E, true, true);         \
+    else if (akc) F3D_GK(E, true, false);          \
+    else if (bkc) F3D_GK(E, false, true);          \
+    else F3D_GK(E, false, false);                  \
+  } while (0)
   switch (epi) {
     case EPI_STORE: F3D_G(EPI_STORE); break;
     case EPI_BIAS_RELU: F3D_G(EPI_BIAS_RELU); break;
@@ -534,5 +741,205 @@ extern "C" int f3d_gemm_bf16(int epi, int64_t M, int64_t N, int64_t K, int32_t k
     default: F3D_G(EPI_BIAS); break;
   }
 #undef F3D_G
+#undef F3D_GK
+  return F3D_OK;
+}
+
+// ---------------------------------------------------------------------------
+namespace f3d {
+// Mean squared error over n outputs and its gradient 2 (y - t) / n; the sum in
+// FP64, per block and then over the blocks in a fixed order.
+constexpr int kMseBlocks = 64;
+__global__ void __launch_bounds__(256)
+mse_kernel(int64_t n, const float* __restrict__ y, const float* __restrict__ t,
+           float* __restrict__ dy, double* __restrict__ part) {
+  __shared__ double red[4];
+  const float c = 2.0f / (float)n;
+  double s = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+    const float d = y[i] - t[i];
+    dy[i] = c * d;
+    s = fma((double)d, (double)d, s);
+  }
+  s = wave_sum_f64(s);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+  __syncthreads();
+  if (threadIdx.x == 0) part[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+}
+__global__ void __launch_bounds__(kMseBlocks)
+mse_final_kernel(int64_t n, const double* __restrict__ part, float* __restrict__ loss) {
+  const double s = wave_sum_f64(part[threadIdx.x]);
+  if (threadIdx.x == 0) loss[0] = (float)(s / (double)n);
+}
+
+// One Adam step over several tensors in one launch (a step of the net is 6
+// tensors; one launch per tensor and operation took 66, and the host longer
+// than all of the step's products).
+constexpr int kAdamTensors = 8;
+struct AdamArgs {
+  float* p[kAdamTensors];
+  const float* g[kAdamTensors];
+  float* m[kAdamTensors];
+  float* v[kAdamTensors];
+  int64_t begin[kAdamTensors];  // of the tensor's elements in the launch
+  int64_t total;
+  int count;
+};
+__global__ void __launch_bounds__(256)
+adam_kernel(AdamArgs a, float lr, float b1, float c1, float b2, float c2, float eps, float inv1,
+            float inv2) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= a.total) return;
+  int k = 0;
+#pragma unroll
+  for (int q = 1; q < kAdamTensors; ++q)
+    if (q < a.count && i >= a.begin[q]) k = q;
+  const int64_t e = i - a.begin[k];
+  const float g = a.g[k][e];
+  const float m = a.m[k][e] * b1 + c1 * g;
+  const float v = a.v[k][e] * b2 + c2 * g * g;
+  a.m[k][e] = m;
+  a.v[k][e] = v;
+  a.p[k][e] -= lr * (m * inv1) / (sqrtf(v * inv2) + eps);
+}
+}  // namespace f3d
+
+extern "C" size_t f3d_mse_workspace_size(void) { return kMseBlocks * sizeof(double); }
+
+extern "C" int f3d_mse(int64_t n, const float* y, const float* t, float* dy, float* loss, void* ws,
+                       size_t ws_bytes, void* stream) {
+  F3D_REQUIRE(n >= 1, F3D_EINVAL, "mse: n=%lld", (long long)n);
+  F3D_REQUIRE(y && t && dy && loss, F3D_EINVAL, "mse: NULL argument");
+  F3D_REQUIRE(ws != nullptr && ws_bytes >= f3d_mse_workspace_size(), F3D_EWORKSPACE,
+              "mse: workspace %zu bytes < required %zu", ws_bytes, f3d_mse_workspace_size());
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  double* part = reinterpret_cast<double*>(ws);
+  F3D_LAUNCH(mse_kernel, dim3(kMseBlocks), dim3(256), 0, st, n, y, t, dy, part);
+  F3D_LAUNCH(mse_final_kernel, dim3(1), dim3(kMseBlocks), 0, st, n, (const double*)part, loss);
+  return F3D_OK;
+}
+
+extern "C" int f3d_adam(int32_t count, const int64_t* sizes, float* const* p,
+                        const float* const* g, float* const* m, float* const* v, double lr,
+                        double b1, double b2, double eps, int64_t t, void* stream) {
+  F3D_REQUIRE(count >= 0 && t >= 1, F3D_EINVAL, "adam: count=%d t=%lld", count, (long long)t);
+  F3D_REQUIRE(count == 0 || (sizes && p && g && m && v), F3D_EINVAL, "adam: NULL argument");
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  const float inv1 = (float)(1.0 / (1.0 - pow(b1, (double)t)));
+  const float inv2 = (float)(1.0 / (1.0 - pow(b2, (double)t)));
+  for (int32_t k0 = 0; k0 < count; k0 += kAdamTensors) {
+    AdamArgs a{};
+    for (int32_t k = k0; k < count && k < k0 + kAdamTensors; ++k) {
+      F3D_REQUIRE(sizes[k] >= 0 && (sizes[k] == 0 || (p[k] && g[k] && m[k] && v[k])), F3D_EINVAL,
+                  "adam: tensor %d", k);
+      a.p[k - k0] = p[k];
+      a.g[k - k0] = g[k];
+      a.m[k - k0] = m[k];
+      a.v[k - k0] = v[k];
+      a.begin[k - k0] = a.total;
+      a.total += sizes[k];
+      ++a.count;
+    }
+    if (a.total == 0) continue;
+    F3D_REQUIRE(a.total < (1ll << 38), F3D_EINVAL, "adam: too many elements");
+    F3D_LAUNCH(adam_kernel, dim3((unsigned)ceil_div(a.total, 256)), dim3(256), 0, st, a, (float)lr,
+               (float)b1, (float)(1.0 - b1), (float)b2, (float)(1.0 - b2), (float)eps, inv1, inv2);
+  }
+  return F3D_OK;
+}
+
+// ---------------------------------------------------------------------------
+// The MLP in -> width -> width -> out as whole passes (three and four
+// launches): the products through f3d_gemm_bf16 and the kernels above.
+extern "C" int f3d_mlp_forward(int64_t M, int32_t n_in, int32_t width, int32_t n_out,
+                               const float* X, int64_t sxm, int64_t sxk, const float* W1,
+                               const float* b1, const float* W2, const float* b2, const float* W3,
+                               const float* b3, float* H1, float* H2, float* Y, void* stream) {
+  F3D_REQUIRE(M >= 0 && n_in >= 1 && width >= 1 && n_out >= 1, F3D_EINVAL, "mlp_forward: bad sizes");
+  if (M == 0) return F3D_OK;
+  F3D_REQUIRE(X && W1 && b1 && W2 && b2 && W3 && b3 && H1 && H2 && Y, F3D_EINVAL,
+              "mlp_forward: NULL argument");
+  int rc = f3d_gemm_bf16(EPI_BIAS_RELU, M, width, n_in, 1, X, sxm, sxk, W1, width, 1, H1, width, 1,
+                         b1, nullptr, nullptr, 1.0f, stream);
+  if (rc != F3D_OK) return rc;
+  rc = f3d_gemm_bf16(EPI_BIAS_RELU, M, width, width, 1, H1, width, 1, W2, width, 1, H2, width, 1,
+                     b2, nullptr, nullptr, 1.0f, stream);
+  if (rc != F3D_OK) return rc;
+  return f3d_gemm_bf16(EPI_BIAS, M, n_out, width, 1, H2, width, 1, W3, n_out, 1, Y, n_out, 1, b3,
+                       nullptr, nullptr, 1.0f, stream);
+}
+
+// Samples per K slice of the gradient products: slices of at least 256 samples,
+// at most 64 of them (24 tiles at 23 -> 256 -> 256 -> 4, so 768 workgroups at a
+// batch of 8192).
+static void grad_slices(int64_t M, int* kchunk, int* slices) {
+  int64_t c = ceil_div(M > 0 ? M : 1, (int64_t)64);
+  c = (int64_t)align_up((size_t)(c < 256 ? 256 : c), kKT);
+  *kchunk = (int)c;
+  *slices = (int)ceil_div(M > 0 ? M : 1, c);
+}
+
+static int64_t mlp_params(int64_t n_in, int64_t width, int64_t n_out) {
+  return n_in * width + width + width * width + width + width * n_out + n_out;
+}
+
+extern "C" size_t f3d_mlp_workspace_size(int64_t M, int32_t n_in, int32_t width, int32_t n_out) {
+  if (M < 0 || M >= (1ll << 31) || n_in < 1 || width < 1 || n_out < 1) return 0;
+  int kchunk, slices;
+  grad_slices(M, &kchunk, &slices);
+  return sizeof(float) * ((size_t)slices * (size_t)mlp_params(n_in, width, n_out) +
+                          2 * (size_t)M * (size_t)width);
+}
+
+extern "C" int f3d_mlp_backward(int64_t M, int32_t n_in, int32_t width, int32_t n_out,
+                                const float* X, int64_t sxm, int64_t sxk, const float* H1,
+                                const float* H2, const float* dY, int64_t sym, int64_t syk,
+                                const float* W2, const float* W3, float* gW1, float* gW2,
+                                float* gW3, float* gb1, float* gb2, float* gb3, void* ws,
+                                size_t ws_bytes, void* stream) {
+  F3D_REQUIRE(M >= 0 && M < (1ll << 31) && n_in >= 1 && width >= 1 && n_out >= 1, F3D_EINVAL,
+              "mlp_backward: bad sizes");
+  F3D_REQUIRE(X && H1 && H2 && dY && W2 && W3 && gW1 && gW2 && gW3 && gb1 && gb2 && gb3, F3D_EINVAL,
+              "mlp_backward: NULL argument");
+  const size_t need = f3d_mlp_workspace_size(M, n_in, width, n_out);
+  F3D_REQUIRE(ws != nullptr && ws_bytes >= need, F3D_EWORKSPACE,
+              "mlp_backward: workspace %zu bytes < required %zu", ws_bytes, need);
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  float* dZ2 = reinterpret_cast<float*>(ws);
+  float* dZ1 = dZ2 + (size_t)M * width;
+  float* part = dZ1 + (size_t)M * width;
+  // dZ = (dOut W^T) where the layer's ReLU was open
+  int rc = f3d_gemm_bf16(EPI_RELU_GRAD, M, width, n_out, 1, dY, sym, syk, W3, 1, n_out, dZ2, width,
+                         1, nullptr, nullptr, H2, 1.0f, stream);
+  if (rc != F3D_OK) return rc;
+  rc = f3d_gemm_bf16(EPI_RELU_GRAD, M, width, width, 1, dZ2, width, 1, W2, 1, width, dZ1, width, 1,
+                     nullptr, nullptr, H1, 1.0f, stream);
+  if (rc != F3D_OK) return rc;
+  GradPlan p;
+  grad_slices(M, &p.kchunk, &p.slices);
+  p.K = (int)M;
+  int tiles = 0;
+  long off = 0;
+  auto layer = [&](int i, const float* a, int64_t am, int64_t ak, int m, const float* b, int64_t bn,
+                   int64_t bk, int n, float* w, float* bs) {
+    GradLayer& L = p.l[i];
+    L.a = TileOperand{a, (long)am, (long)ak, m};
+    L.b = TileOperand{b, (long)bn, (long)bk, n};
+    L.tile0 = tiles;
+    L.tiles_n = (int)ceil_div(n, kNT);
+    L.off = off;
+    L.w = w;
+    L.bs = bs;
+    tiles += (int)ceil_div(m, kMT) * L.tiles_n;
+    off += (long)m * n + n;
+  };
+  layer(0, X, sxk, sxm, n_in, dZ1, 1, width, width, gW1, gb1);
+  layer(1, H1, 1, width, width, dZ2, 1, width, width, gW2, gb2);
+  layer(2, H2, 1, width, width, dY, syk, sym, n_out, gW3, gb3);
+  p.total = off;
+  F3D_LAUNCH(grad_partial_kernel, dim3((unsigned)tiles, (unsigned)p.slices), dim3(256), 0, st, p,
+             part);
+  F3D_LAUNCH(grad_reduce_kernel, dim3((unsigned)ceil_div(p.total, (int64_t)256)), dim3(256), 0, st,
+             p, (const float*)part);
   return F3D_OK;
 }

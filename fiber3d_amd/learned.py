@@ -16,6 +16,8 @@ Guess assembly per step: the previous solutions extrapolated (positions by a
 least-squares quadratic in time, the rest linearly), corrected by the net
 (see LearnedGuess).
 """
+import ctypes
+
 import numpy as np
 import torch
 
@@ -63,54 +65,62 @@ class MLP:
         self.n_in, self.n_out, self.width = n_in, n_out, width
 
     def forward(self, X, keep=False):
-        M = X.shape[0]
-        dev = X.device
-        Z1 = torch.empty((M, self.width), device=dev)
-        H1 = torch.empty_like(Z1)
-        gemm(X, self.W[0], H1, EPI_BIAS_RELU, bias=self.b[0], Z=Z1)
-        Z2 = torch.empty_like(Z1)
-        H2 = torch.empty_like(Z1)
-        gemm(H1, self.W[1], H2, EPI_BIAS_RELU, bias=self.b[1], Z=Z2)
+        M, dev = X.shape[0], X.device
+        assert X.dtype == torch.float32 and X.shape[1] == self.n_in
+        H1 = torch.empty((M, self.width), device=dev)
+        H2 = torch.empty_like(H1)
         Y = torch.empty((M, self.n_out), device=dev)
-        gemm(H2, self.W[2], Y, EPI_BIAS, bias=self.b[2])
+        p = L.ptr
+        rc = L.load().f3d_mlp_forward(
+            M, self.n_in, self.width, self.n_out, p(X), X.stride(0), X.stride(1), p(self.W[0]),
+            p(self.b[0]), p(self.W[1]), p(self.b[1]), p(self.W[2]), p(self.b[2]), p(H1), p(H2),
+            p(Y), _stream())
+        L.check(rc, "f3d_mlp_forward")
         if keep:
-            self._cache = (X, Z1, H1, Z2, H2)
+            self._cache = (X, H1, H2)
         return Y
 
     def backward(self, dY):
         """Gradients of the loss wrt all parameters, given dL/dY."""
-        X, Z1, H1, Z2, H2 = self._cache
+        X, H1, H2 = self._cache
         M = X.shape[0]
-        ks = max(1, min(64, M // 1024))
-        grads = [torch.zeros_like(p) for p in self.params]
-        gemm(H2, dY, grads[2], EPI_ATOMIC, transA=True, ksplit=ks)
-        grads[5] = dY.sum(0)
-        dZ2 = torch.empty_like(Z2)
-        gemm(dY, self.W[2], dZ2, EPI_RELU_GRAD, Zin=Z2, transB=True)
-        gemm(H1, dZ2, grads[1], EPI_ATOMIC, transA=True, ksplit=ks)
-        grads[4] = dZ2.sum(0)
-        dZ1 = torch.empty_like(Z1)
-        gemm(dZ2, self.W[1], dZ1, EPI_RELU_GRAD, Zin=Z1, transB=True)
-        gemm(X, dZ1, grads[0], EPI_ATOMIC, transA=True, ksplit=ks)
-        grads[3] = dZ1.sum(0)
+        assert dY.dtype == torch.float32 and dY.shape == (M, self.n_out)
+        lib = L.load()
+        grads = [torch.empty_like(q) for q in self.params]
+        need = lib.f3d_mlp_workspace_size(M, self.n_in, self.width, self.n_out)
+        ws = torch.empty(need, dtype=torch.uint8, device=X.device)
+        p = L.ptr
+        rc = lib.f3d_mlp_backward(
+            M, self.n_in, self.width, self.n_out, p(X), X.stride(0), X.stride(1), p(H1), p(H2),
+            p(dY), dY.stride(0), dY.stride(1), p(self.W[1]), p(self.W[2]),
+            *(p(g) for g in grads), p(ws), need, _stream())
+        L.check(rc, "f3d_mlp_backward")
         return grads
 
     def adam(self, grads, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8):
         self.t += 1
-        for p, g, m, v in zip(self.params, grads, self.m, self.v):
-            m.mul_(b1).add_(g, alpha=1 - b1)
-            v.mul_(b2).addcmul_(g, g, value=1 - b2)
-            mh = m / (1 - b1**self.t)
-            vh = v / (1 - b2**self.t)
-            p.sub_(lr * mh / (vh.sqrt() + eps))
+        k = len(self.params)
+        grads = [g.contiguous() for g in grads]
+        ptrs = lambda ts: (ctypes.c_void_p * k)(*(t.data_ptr() for t in ts))
+        sizes = (ctypes.c_int64 * k)(*(q.numel() for q in self.params))
+        rc = L.load().f3d_adam(k, sizes, ptrs(self.params), ptrs(grads), ptrs(self.m),
+                               ptrs(self.v), lr, b1, b2, eps, self.t, _stream())
+        L.check(rc, "f3d_adam")
 
     def train_step(self, X, target, lr=1e-3):
         Y = self.forward(X, keep=True)
-        diff = Y - target
-        loss = float((diff * diff).mean())
-        dY = (2.0 / diff.numel()) * diff
-        self.adam(self.backward(dY.contiguous()), lr=lr)
-        return loss
+        assert torch.result_type(Y, target) == torch.float32
+        target = target.to(Y.dtype).expand_as(Y).contiguous()
+        lib = L.load()
+        dY = torch.empty_like(Y)
+        loss = torch.empty((), device=Y.device)
+        need = lib.f3d_mse_workspace_size()
+        ws = torch.empty(need, dtype=torch.uint8, device=Y.device)
+        rc = lib.f3d_mse(Y.numel(), L.ptr(Y), L.ptr(target), L.ptr(dY), L.ptr(loss), L.ptr(ws),
+                         need, _stream())
+        L.check(rc, "f3d_mse")
+        self.adam(self.backward(dY), lr=lr)
+        return float(loss)  # waits for the device once the whole step is queued
 
 
 class Normalizer:

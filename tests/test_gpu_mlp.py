@@ -113,3 +113,92 @@ def test_per_node_layer_kernels_agree(N, M, K, epi):
     finally:
         from fiber3d_amd import autotune
         autotune.apply()
+
+
+@pytest.mark.parametrize("M,n_in,n_out,width", [(1, 1, 1, 256), (63, 5, 2, 64), (64, 23, 4, 256),
+                                               (257, 23, 4, 256), (1000, 7, 65, 130),
+                                               (20000, 23, 4, 256)])
+def test_mlp_passes_against_fp64(M, n_in, n_out, width):
+    """The net's forward and backward passes at the edges of the products'
+    tiles and sample slices, for a strided input and output gradient, against
+    FP64 products of the same BF16-rounded operands: FP32 accumulation over K
+    terms (2 K eps of the absolute products, element by element)."""
+    print(f"case mlp passes M={M} {n_in}-{width}-{n_out}", flush=True)
+    rng = np.random.default_rng(M + width)
+    net = LG.MLP(n_in, n_out, width=width, seed=1)
+    X = torch.from_numpy(rng.normal(size=(n_in + 1, M)).astype(np.float32)).cuda().t()[:, :n_in]
+    dY = torch.from_numpy(rng.normal(size=(n_out, M)).astype(np.float32)).cuda().t()
+    Y = net.forward(X, keep=True)
+    _, H1, H2 = net._cache
+    g = [t.cpu().double().numpy() for t in net.backward(dY)]
+    h = lambda t: t.detach().cpu().double().numpy()
+    W, b = [h(t) for t in net.W], [h(t) for t in net.b]
+
+    def check(got, A, B, add=0.0, mask=None):
+        A, B = _bf16(A), _bf16(B)
+        ref, mag = A @ B + add, np.abs(A) @ np.abs(B) + np.abs(add)
+        if mask is not None:
+            ref, mag = ref * mask, mag * mask
+        assert (np.abs(got - ref) <= 2 * (A.shape[1] + 2) * 2.0 ** -24 * mag).all()
+        return ref
+    pre = check(h(H1), h(X), W[0], b[0], mask=h(H1) > 0)
+    assert (pre[h(H1) > 0] > -1e-3).all()
+    check(h(H2), h(H1), W[1], b[1], mask=h(H2) > 0)
+    check(h(Y), h(H2), W[2], b[2])
+    # the gradients' inner factors are not returned: FP64 from the same masks
+    # and BF16 operands, to the rounding of one BF16 operand of each product
+    d2 = (_bf16(h(dY)) @ _bf16(W[2]).T) * (h(H2) > 0)
+    d1 = (_bf16(d2) @ _bf16(W[1]).T) * (h(H1) > 0)
+    for got, A, B in ((g[2], h(H2).T, h(dY)), (g[1], h(H1).T, d2), (g[0], h(X).T, d1)):
+        mag = np.abs(_bf16(A)) @ np.abs(_bf16(B))
+        assert (np.abs(got - _bf16(A) @ _bf16(B)) <= 2.0 ** -7 * mag + 1e-30).all()
+    for got, B in ((g[5], h(dY)), (g[4], d2), (g[3], d1)):
+        assert (np.abs(got - B.sum(0)) <= 2.0 ** -7 * np.abs(B).sum(0) + 1e-30).all()
+
+
+@pytest.mark.parametrize("N", [128, 256])
+@pytest.mark.parametrize("M,K", [(49152, 32), (49153, 48), (65599, 256)])
+def test_per_node_layer_kernels_of_many_rows(N, M, K):
+    """The streaming and resident kernels from the row count at which they
+    take over, whole and partial last blocks."""
+    from fiber3d_amd import _lib as L
+    print(f"case layer kernels of many rows {M}x{N}x{K}", flush=True)
+    rng = np.random.default_rng(M + N + K)
+    A = rng.normal(size=(M, K)).astype(np.float32)
+    B = rng.normal(size=(K, N)).astype(np.float32)
+    bias = rng.normal(size=N).astype(np.float32)
+    ref = np.maximum(_bf16(A) @ _bf16(B) + bias, 0.0)
+    try:
+        for mode in (2, 1):
+            L.check(L.load().f3d_gemm_set_stream(N, mode), "f3d_gemm_set_stream")
+            C = torch.full((M, N), 7.0, device="cuda")
+            LG.gemm(torch.from_numpy(A).cuda(), torch.from_numpy(B).cuda(), C, LG.EPI_BIAS_RELU,
+                    bias=torch.from_numpy(bias).cuda())
+            assert rel2(C.cpu().numpy(), ref) < 1e-6, mode
+    finally:
+        from fiber3d_amd import autotune
+        autotune.apply()
+
+
+def test_adam_and_mse_against_fp64():
+    """Three fused optimiser steps and the loss's gradient against FP64."""
+    print("case adam mse", flush=True)
+    rng = np.random.default_rng(4)
+    net = LG.MLP(3, 2, seed=2)
+    P = [p.cpu().double().numpy() for p in net.params]
+    m, v = [np.zeros_like(p) for p in P], [np.zeros_like(p) for p in P]
+    for t in range(1, 4):
+        G = [rng.normal(size=p.shape).astype(np.float32) for p in P]
+        net.adam([torch.from_numpy(q).cuda() for q in G], lr=1e-2)
+        for k, q in enumerate(G):
+            q = q.astype(np.float64)
+            m[k] = 0.9 * m[k] + 0.1 * q
+            v[k] = 0.999 * v[k] + 0.001 * q * q
+            P[k] -= 1e-2 * (m[k] / (1 - 0.9 ** t)) / (np.sqrt(v[k] / (1 - 0.999 ** t)) + 1e-8)
+    for p, r in zip(net.params, P):
+        np.testing.assert_allclose(p.cpu().double().numpy(), r, rtol=0, atol=3e-6)
+    X = torch.from_numpy(rng.normal(size=(777, 3)).astype(np.float32)).cuda()
+    T = torch.from_numpy(rng.normal(size=(777, 2)).astype(np.float32)).cuda()
+    Y = net.forward(X)
+    loss = net.train_step(X, T, lr=0.0)
+    assert abs(loss - float(((Y.double() - T.double()) ** 2).mean())) <= 1e-6 * loss
