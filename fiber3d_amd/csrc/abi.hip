@@ -3,6 +3,8 @@
 
 #include "common.h"
 
+#include <atomic>
+
 namespace f3d {
 
 static thread_local char g_last_error[512] = "";
@@ -14,6 +16,18 @@ void set_error(const char* fmt, ...) {
   va_end(ap);
 }
 
+int num_cus() {
+  static std::atomic<int> cached{0};
+  int n = cached.load(std::memory_order_relaxed);
+  if (n > 0) return n;
+  int dev = 0;
+  hipDeviceProp_t prop;
+  if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess)
+    return 256;
+  n = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
+  cached.store(n, std::memory_order_relaxed);
+  return n;
+}
 }  // namespace f3d
 
 extern "C" const char* f3d_last_error(void) { return f3d::g_last_error; }

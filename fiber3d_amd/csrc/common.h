@@ -42,10 +42,21 @@ void set_error(const char* fmt, ...);
     }                                                                         \
   } while (0)
 
+// Compute units of the current device (256 where it cannot be asked).
+int num_cus();
+
 inline size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 constexpr double kPi = 3.14159265358979323846;
+
+// Workgroup barrier that orders LDS only: global loads and stores stay in
+// flight (a __syncthreads waits for them).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
 
 // ---- wave64 reductions (device) -----------------------------------------
 __device__ __forceinline__ int wave_min_i32(int v) {

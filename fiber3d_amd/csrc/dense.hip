@@ -973,18 +973,6 @@ dense_gemv_kernel(int64_t waves_total, int32_t m, int32_t groups, int vec,
   }
 }
 
-static int num_cus() {
-  static int cached = 0;
-  if (cached == 0) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 256;
-    hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, dev) != hipSuccess) return 256;
-    cached = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
-  }
-  return cached;
-}
-
 int launch_lu_block(int precision, int64_t nb, const int32_t* n, const int64_t* a_off,
                     const int64_t* x_off, const int32_t* order, const double* A, double* lu64,
                     float* lu32, double* rs, double* cs, int32_t* piv, int32_t* perm,

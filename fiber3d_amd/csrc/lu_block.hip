@@ -131,20 +131,6 @@ __device__ __forceinline__ void sfor(F&& f) {
   }
 }
 
-// Workgroup barrier that orders LDS only: global loads stay in flight (a
-// __syncthreads waits for them).
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-// The same between the lanes of one wave.
-__device__ __forceinline__ void lds_wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-}
-
 // |v| as an integer that orders like |v|, plus one; 0 for NaN.  FP64: the
 // high word here, the low word breaks its ties.
 __device__ __forceinline__ unsigned abs_key(double v) {

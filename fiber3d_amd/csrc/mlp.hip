@@ -642,18 +642,6 @@ extern "C" int f3d_gemm_set_stream(int32_t n, int32_t enable) {
   return F3D_OK;
 }
 
-static int gemm_num_cus() {
-  static int cached = 0;
-  if (cached == 0) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 256;
-    hipDeviceProp_t prop;
-    if (hipGetDeviceProperties(&prop, dev) != hipSuccess) return 256;
-    cached = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
-  }
-  return cached;
-}
-
 extern "C" int f3d_gemm_bf16(int epi, int64_t M, int64_t N, int64_t K, int32_t ksplit,
                              const float* A, int64_t sam, int64_t sak, const float* B,
                              int64_t sbk, int64_t sbn, float* C, int64_t scm, int64_t scn,
@@ -686,7 +674,7 @@ extern "C" int f3d_gemm_bf16(int epi, int64_t M, int64_t N, int64_t K, int32_t k
   if (resident_ok) {
     const int RM = N == 256 ? 32 : 64;
     const int64_t nblocks = ceil_div(M, (int64_t)RM);
-    const dim3 g((unsigned)std::min<int64_t>(nblocks, gemm_num_cus()));
+    const dim3 g((unsigned)std::min<int64_t>(nblocks, num_cus()));
 #define F3D_R(E, T)                                                                          \
   F3D_LAUNCH((gemm_bf16_resident_kernel<E, T>), g, dim3(512), 0, st, (int)M, (int)N, (int)K, A, \
              (long)sam, B, (long)sbk, (long)sbn, C, (long)scm, bias, Z, Zin, alpha)

@@ -196,6 +196,44 @@ def test_hip_assembly_matches_torch_assembly(N):
     assert rel2(y.cpu().numpy(), yo) < 1e-9
 
 
+@pytest.mark.parametrize("N,nfib,dense", [(12, 7, False), (16, 3, False), (17, 5, True),
+                                          (31, 5, False), (32, 9, True), (33, 3, False),
+                                          (47, 3, True), (48, 2, False), (49, 3, True),
+                                          (63, 2, False), (64, 3, True), (20, 1101, False)])
+def test_hip_assembly_at_tile_edges(N, nfib, dense):
+    """Assembly and right-hand side at the edges of the 16-column tiles and of
+    the two kernel sizes, with more fibers than workgroups, and with derivative
+    matrices that are dense (no band to skip), against the torch assembly.
+
+    All entries are sums of at most 64 products of O(1) factors (dense), or the
+    two assemblies of the same banded D in different orders: 64 eps of the
+    largest terms, whose cancellation the existing test bounds by 1e-9 at
+    N = 64 for A_sq; the dense factors do not cancel (1e-12)."""
+    print(f"case assembly edges N={N} nfib={nfib} dense={dense}", flush=True)
+    rng = np.random.default_rng(N)
+    fibers = configs.make_fibers(configs.FiberSpec(nfib, N, 1.0, 8.0), seed=5)
+    lengths = rng.uniform(0.8, 1.6, nfib)
+    ref = FiberSystem(fibers, None, lengths=lengths, assembly="torch")
+    hip = FiberSystem(fibers, None, lengths=lengths, assembly="hip")
+    if dense:
+        D = torch.from_numpy(rng.normal(size=(4, N, N)) / np.sqrt(N)).cuda()
+        for s in (ref, hip):
+            bk = s.buckets[N]
+            bk["D0"] = list(D)
+            if "asm" in bk:
+                bk["asm"]["D0"] = D
+            s.prepare(refactor=False)
+    torch.cuda.synchronize()
+    t = lambda v: v.cpu().numpy()
+    assert rel2(t(hip.A_buf), t(ref.A_buf)) < (1e-12 if dense else 1e-9)
+    assert rel2(t(hip.F_buf), t(ref.F_buf)) < 1e-12
+    for c in range(3):
+        assert rel2(t(hip.Q_buf[c]), t(ref.Q_buf[c])) < 1e-12
+    assert rel2(t(hip.xs), t(ref.xs)) < 1e-12
+    assert rel2(t(hip.weights), t(ref.weights)) < 1e-15
+    assert rel2(t(hip.rhs), t(ref.rhs)) < 1e-12
+
+
 def test_ellipsoidal_periphery_matches_oracle():
     """An ellipsoidal shell (semi-axes 3, 2.5, 2; 900 nodes) around 12
     fibers: right-hand side, operator in FP64 and FP32-compensated,
