@@ -35,6 +35,7 @@
 //   * Spatial order: Oseen and rotlet calls of at least 65536 sources
 //     and targets, without exclusion ranges, visit both in Morton order
 //     (sorted on the device each call), so that tiles and waves are compact.
+//   * Small FP64 calls take one launch instead: pairsum_direct_kernel.
 //   * Far tiles: a tile whose centre is more than twice its radius (and more
 //     than its radius + 2 eps) from the box of the wave's targets has no near
 //     pair, so it runs without the vote; FP32C evaluates it on FP32
@@ -45,6 +46,7 @@
 #include <stdarg.h>
 #include <stdlib.h>
 
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -955,6 +957,31 @@ struct ShellEpi {
   const double* sigma_part;  // kPackBlocks partial sums of n.q
 };
 
+// Target i's sum u, with the epilogue's terms, to the caller's layout.
+__device__ __forceinline__ void store_target(int i, double (&u)[3], double sigma,
+                                             double* __restrict__ out, long o_sp, long o_sc,
+                                             int accumulate, const ShellEpi& epi) {
+  const long b = (long)i * o_sp;
+  if (epi.q) {
+    const double wi = epi.w[i];
+    const double q0 = epi.q[b], q1 = epi.q[b + o_sc], q2 = epi.q[b + 2 * o_sc];
+    const double a0 = q0 / wi, a1 = q1 / wi, a2 = q2 / wi;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const long bc = b + c * o_sc;
+      u[c] -= a0 * epi.ex[bc] + a1 * epi.ey[bc] + a2 * epi.ez[bc];
+      u[c] -= epi.q[bc] / wi;
+      u[c] += epi.nrm[bc] * sigma;
+      if (epi.add) u[c] += epi.add[bc];
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    const long bc = b + c * o_sc;
+    out[bc] = accumulate ? out[bc] + u[c] : u[c];
+  }
+}
+
 // Targets per block of reduce_kernel: its four waves split the source
 // chunks p = w, w + 4, ... of the same 64 targets (4x the waves of one
 // target per lane, so enough loads are in flight to cover HBM latency at
@@ -1003,26 +1030,172 @@ reduce_kernel(const T* __restrict__ part_hi, const T* __restrict__ part_lo, int 
 #pragma unroll
   for (int c = 0; c < 3; ++c)
     u[c] = factor * (((a[c] + sums[0][c][lane]) + sums[1][c][lane]) + sums[2][c][lane]);
-  const long b = (long)i * o_sp;
-  if (epi.q) {
-    const double wi = epi.w[i];
-    const double q0 = epi.q[b], q1 = epi.q[b + o_sc], q2 = epi.q[b + 2 * o_sc];
-    const double a0 = q0 / wi, a1 = q1 / wi, a2 = q2 / wi;
+  store_target(i, u, sigma, out, o_sp, o_sc, accumulate, epi);
+}
+
+// ---------------------------------------------------------------------------
+// FP64 sums of small calls in one launch: no records, boxes or partial sums.
+// A workgroup has K 2^lg targets; its 256 threads are 2^lg target lanes times
+// 256 / 2^lg slices of the sources.  The sources (weights applied) are staged
+// through LDS, kDirectStage at a time, the next stage's loads in flight during
+// this one; the slices' sums meet in registers, then in LDS, in a fixed order.
+// Every pair takes the regularised form (MODE_EXACT), so that no tile is
+// voted on or repeated.
+//
+// What bounds a small call is the chain of dependent launches and, inside
+// one, of sources: 64 per wave in pairsum_kernel, ns 2^lg / 256 here.  1024 x
+// 1024 Oseen: 19.6 us in four launches, 5.9 us here; 32 x 1024: 19.6 and 3.1.
+constexpr int kDirectStage = 512;
+
+template <int KIND, int K, bool MASK>
+__global__ void __launch_bounds__(256)
+pairsum_direct_kernel(int ns, const double* __restrict__ pos, const double* __restrict__ nrm,
+                      const double* __restrict__ den, const double* __restrict__ w, long s_sp,
+                      long s_sc, int nt, const double* __restrict__ tpos, long t_sp, long t_sc,
+                      const int* __restrict__ excl_lo, const int* __restrict__ excl_hi,
+                      double reg2, double eps2, double factor, int lg, double* __restrict__ out,
+                      long o_sp, long o_sc, int accumulate, ShellEpi epi) {
+  // words per source: x, f (6) or x, n, q (9, padded to whole 16 bytes)
+  constexpr int R = KIND == F3D_STRESSLET ? 10 : 6;
+  constexpr int PER = kDirectStage / 256;
+  typedef double v2d __attribute__((ext_vector_type(2)));
+  __shared__ __align__(16) double rec[kDirectStage * R];
+  __shared__ double red[4][3][K * 64];
+  __shared__ double red_sig[4];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const int TG = 1 << lg, tau = t & (TG - 1), slice = t >> lg, S = 256 >> lg;
+  const int i0 = blockIdx.x * (K * TG);
+  double tx[K], ty[K], tz[K], ax[K], ay[K], az[K];
+  int lo[K], hi[K];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      const long bc = b + c * o_sc;
-      u[c] -= a0 * epi.ex[bc] + a1 * epi.ey[bc] + a2 * epi.ez[bc];
-      u[c] -= epi.q[bc] / wi;
-      u[c] += epi.nrm[bc] * sigma;
-      if (epi.add) u[c] += epi.add[bc];
+  for (int q = 0; q < K; ++q) {
+    const int i = min(i0 + q * TG + tau, nt - 1);
+    tx[q] = tpos[i * t_sp];
+    ty[q] = tpos[i * t_sp + t_sc];
+    tz[q] = tpos[i * t_sp + 2 * t_sc];
+    lo[q] = hi[q] = 0;
+    if (MASK) {
+      lo[q] = excl_lo ? excl_lo[i] : i;
+      hi[q] = excl_lo ? excl_hi[i] : i + 1;
+    }
+    ax[q] = ay[q] = az[q] = 0.0;
+  }
+  const bool want_sigma = KIND == F3D_STRESSLET && epi.q != nullptr;
+  double sig = 0.0;
+  double nx[PER][R];
+  auto fetch = [&](int j0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      const int j = j0 + t + 256 * u;
+      if (j < ns) {
+        const long b = (long)j * s_sp;
+        const double wj = w ? w[j] : 1.0;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          nx[u][c] = pos[b + c * s_sc];
+          if constexpr (KIND == F3D_STRESSLET) {
+            nx[u][3 + c] = nrm[b + c * s_sc];
+            nx[u][6 + c] = den[b + c * s_sc] * wj;
+          } else {
+            nx[u][3 + c] = den[b + c * s_sc] * wj;
+          }
+        }
+      }
+    }
+  };
+  fetch(0);
+  for (int j0 = 0; j0 < ns; j0 += kDirectStage) {
+    if (j0 > 0) lds_barrier();
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+      if (j0 + t + 256 * u < ns) {
+        v2d* d = reinterpret_cast<v2d*>(rec + (t + 256 * u) * R);
+        if constexpr (KIND == F3D_STRESSLET) {
+          nx[u][9] = 0.0;
+          sig += nx[u][3] * nx[u][6] + nx[u][4] * nx[u][7] + nx[u][5] * nx[u][8];
+        }
+#pragma unroll
+        for (int c = 0; c < R / 2; ++c) d[c] = v2d{nx[u][2 * c], nx[u][2 * c + 1]};
+      }
+    }
+    lds_barrier();
+    fetch(j0 + kDirectStage);
+    const int cnt = min(kDirectStage, ns - j0);
+    auto one = [&](int k) __attribute__((always_inline)) {
+      const v2d* r = reinterpret_cast<const v2d*>(rec + k * R);
+      double s[R];
+#pragma unroll
+      for (int c = 0; c < R / 2; ++c) {
+        const v2d v = r[c];
+        s[2 * c] = v[0];
+        s[2 * c + 1] = v[1];
+      }
+#pragma unroll
+      for (int q = 0; q < K; ++q) {
+        const double dx = tx[q] - s[0], dy = ty[q] - s[1], dz = tz[q] - s[2];
+        double r2 = dx * dx + dy * dy + dz * dz;
+        r2 = (r2 < eps2) ? r2 + reg2 : r2;
+        double ri = rsqrt2_t(r2);  // 2 / r
+        if (MASK) ri = (unsigned)(j0 + k - lo[q]) < (unsigned)(hi[q] - lo[q]) ? 0.0 : ri;
+        if constexpr (KIND == F3D_OSEEN) {
+          const double fd = dx * s[3] + dy * s[4] + dz * s[5];
+          const double h = (0.25 * fd) * (ri * ri);
+          ax[q] += ri * fma(h, dx, s[3]);
+          ay[q] += ri * fma(h, dy, s[4]);
+          az[q] += ri * fma(h, dz, s[5]);
+        } else {
+          accum<double, KIND>(s + 3, dx, dy, dz, ri, ax[q], ay[q], az[q]);
+        }
+      }
+    };
+    int k = slice;
+    for (; k + 3 * S < cnt; k += 4 * S) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) one(k + u * S);
+    }
+    for (; k < cnt; k += S) one(k);
+  }
+  // the slices of a wave, then the four waves
+#pragma unroll
+  for (int q = 0; q < K; ++q) {
+    for (int o = 32; o >= TG; o >>= 1) {
+      ax[q] += __shfl_xor(ax[q], o, 64);
+      ay[q] += __shfl_xor(ay[q], o, 64);
+      az[q] += __shfl_xor(az[q], o, 64);
+    }
+    if (lane < TG) {
+      red[wv][0][q * TG + lane] = ax[q];
+      red[wv][1][q * TG + lane] = ay[q];
+      red[wv][2][q * TG + lane] = az[q];
     }
   }
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    const long bc = b + c * o_sc;
-    out[bc] = accumulate ? out[bc] + u[c] : u[c];
+  if (want_sigma) {
+    sig = wave_sum_f64(sig);
+    if (lane == 0) red_sig[wv] = sig;
   }
+  lds_barrier();
+  if (t >= K * TG || i0 + t >= nt) return;
+  double u[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+    u[c] = factor * (((red[0][c][t] + red[1][c][t]) + red[2][c][t]) + red[3][c][t]);
+  store_target(i0 + t, u, want_sigma ? red_sig[0] + red_sig[1] + red_sig[2] + red_sig[3] : 0.0,
+               out, o_sp, o_sc, accumulate, epi);
 }
+
+// Byte range of n points of three components at strides (sp, sc).
+struct Span {
+  const char *b, *e;
+};
+static Span span_of(const void* p, int64_t n, int64_t sp, int64_t sc, size_t size) {
+  if (p == nullptr || n <= 0) return {nullptr, nullptr};
+  const int64_t last = (n - 1) * sp, comp = 2 * sc;
+  const int64_t lo = std::min<int64_t>(0, last) + std::min<int64_t>(0, comp);
+  const int64_t hi = std::max<int64_t>(0, last) + std::max<int64_t>(0, comp);
+  const char* c = reinterpret_cast<const char*>(p);
+  return {c + lo * (int64_t)size, c + (hi + 1) * (int64_t)size};
+}
+static bool overlap(Span a, Span b) { return a.b && b.b && a.b < b.e && b.b < a.e; }
 
 // ---------------------------------------------------------------------------
 // Host-side plan: split count and chunk length.
@@ -1034,6 +1207,7 @@ struct Plan {
   int G;      // chunks per block (waves of a block, combined in LDS)
   int Pg;     // partial sums per target: ceil(P / G)
   int sort;   // sources and targets in spatial order
+  int forced; // shape set by the environment: no direct kernel
 };
 
 static void set_groups(Plan& pl) {
@@ -1084,6 +1258,8 @@ static Plan make_plan(int kernel, int precision, int64_t ns, int64_t nt) {
   const int w0 = tuned ? g_bucket_waves[kk][pp][bt][bs] : g_launch_waves[kk][pp];
   pl.K = env_int(precision == F3D_F64 ? "F3D_PAIRSUM_K64" : "F3D_PAIRSUM_K32", k0);
   if (pl.K != 1 && pl.K != 2 && pl.K != 4) pl.K = 2;
+  pl.forced = env_int(precision == F3D_F64 ? "F3D_PAIRSUM_K64" : "F3D_PAIRSUM_K32", 0) != 0 ||
+              env_int("F3D_PAIRSUM_WAVES", 0) != 0;
   pl.ns_pad = (int)align_up((size_t)(ns > 0 ? ns : 1), kTile);
   const int64_t waves_per_split = ceil_div(nt > 0 ? nt : 1, 64 * pl.K);
   int target_waves = env_int("F3D_PAIRSUM_WAVES", w0);
@@ -1166,6 +1342,50 @@ static Plan make_plan_within(int kernel, int precision, int64_t ns, int64_t nt, 
   return pl;
 }
 
+// Shape of pairsum_direct_kernel for a call (targets per lane, log2 of the
+// target lanes), or k = 0: the call takes the general path.
+//
+// The line: a workgroup reads all sources, so its share of them (ns / slices)
+// and the call's reads of LDS grow with ns, while the general path's scalar
+// records cost the same for every target.  Measured, general against direct,
+// us (FP64 Oseen; stresslet): 1024 x 1024 19.6 / 5.9 (19.4 / 6.5), 4096 sources
+// x 256 20.2 / 10.8 (20.1 / 13.9), 4096 x 4096 30.4 / 26.3 (32.0 / 30.7), 2048
+// x 16384 45.2 / 36.4 (46.6 / 42.6), 512 x 65536 39.1 / 32.8 (41.7 / 39.0);
+// past the line 8192 x 4096 46.3 / 47.3 (49.2 / 56.4), 1024 x 262144 222 / 227
+// (253 / 253), 8192 x 256 21.4 / 18.9 (21.2 / 25.0).
+//
+// Within it: 256 to 512 workgroups (two per CU), with at least four target
+// lanes once every CU has a workgroup (fewer distinct LDS reads per wave); two
+// targets per lane from 4096 on, which halves the LDS reads per pair (10.5 /
+// 9.4 us at 1024 x 4096, but 5.9 / 6.9 at 1024 x 1024).
+constexpr int64_t kDirectSources = 4096;
+constexpr int64_t kDirectPairs = 1ll << 25;
+struct DirectShape {
+  int k, lg;
+};
+static DirectShape direct_shape(const Plan& pl, int64_t ns, int64_t nt) {
+  if (pl.forced || pl.sort || ns > kDirectSources || ns * nt > kDirectPairs) return {0, 0};
+  DirectShape d{nt > 2048 ? 2 : 1, 0};
+  while (d.lg < 6 && (nt > ((int64_t)512 * d.k << d.lg) || (d.lg < 2 && nt > (int64_t)256 << d.lg)))
+    ++d.lg;
+  return d;
+}
+
+// Whether the output overlaps an input: the direct kernel's workgroups read
+// inputs after others have written.  (The epilogue's arrays are read at the
+// written index by the thread that writes it; its q is den.)
+static bool direct_aliases(int64_t ns, const double* pos, const double* nrm, const double* den,
+                           const double* w, int64_t s_sp, int64_t s_sc, int64_t nt,
+                           const double* tpos, int64_t t_sp, int64_t t_sc, const int32_t* lo,
+                           const int32_t* hi, const double* out, int64_t o_sp, int64_t o_sc) {
+  const Span o = span_of(out, nt, o_sp, o_sc, 8);
+  return overlap(o, span_of(pos, ns, s_sp, s_sc, 8)) ||
+         overlap(o, span_of(nrm, ns, s_sp, s_sc, 8)) ||
+         overlap(o, span_of(den, ns, s_sp, s_sc, 8)) || overlap(o, span_of(w, ns, 1, 0, 8)) ||
+         overlap(o, span_of(tpos, nt, t_sp, t_sc, 8)) || overlap(o, span_of(lo, nt, 1, 0, 4)) ||
+         overlap(o, span_of(hi, nt, 1, 0, 4));
+}
+
 template <typename T, int KIND>
 static int launch_pairsum(const Plan& pl, uint32_t flags, int64_t ns, const double* pos,
                           const double* nrm, const double* den, const double* w, int64_t s_sp,
@@ -1174,6 +1394,37 @@ static int launch_pairsum(const Plan& pl, uint32_t flags, int64_t ns, const doub
                           double reg, double eps, double* out, int64_t o_sp, int64_t o_sc,
                           char* ws, const ShellEpi* epi_in, hipStream_t st) {
   constexpr bool kQuant = std::is_same<T, float>::value;
+  double factor = KIND == F3D_STRESSLET ? -3.0 / (4.0 * kPi * eta) : 1.0 / (8.0 * kPi * eta);
+  factor *= TwoOverR<T, KIND>::scale;
+  const bool timed = g_timer.on && g_timer.n < kTimerSlots;
+  if constexpr (!kQuant) {
+    const DirectShape d = direct_shape(pl, ns, nt);
+    if (d.k > 0 && !direct_aliases(ns, pos, nrm, den, w, s_sp, s_sc, nt, tpos, t_sp, t_sc, lo, hi,
+                                   out, o_sp, o_sc)) {
+      if (timed) F3D_HIP_CHECK(hipEventRecord(g_timer.ev[2 * g_timer.n], st));
+      const dim3 grid((unsigned)ceil_div(nt, (int64_t)d.k << d.lg));
+      const ShellEpi epi = epi_in ? *epi_in : ShellEpi{};
+#define F3D_PD(K, MASK)                                                                         \
+  F3D_LAUNCH((pairsum_direct_kernel<KIND, K, MASK>), grid, dim3(256), 0, st, (int)ns, pos, nrm, \
+             den, w, (long)s_sp, (long)s_sc, (int)nt, tpos, (long)t_sp, (long)t_sc, lo, hi,     \
+             reg * reg, eps * eps, factor, d.lg, out, (long)o_sp, (long)o_sc,                   \
+             (flags & F3D_ACCUMULATE) ? 1 : 0, epi)
+      const bool mask = lo != nullptr || (flags & F3D_EXCLUDE_SELF) != 0;
+      if (d.k == 1) {
+        if (mask) F3D_PD(1, true);
+        else F3D_PD(1, false);
+      } else {
+        if (mask) F3D_PD(2, true);
+        else F3D_PD(2, false);
+      }
+#undef F3D_PD
+      if (timed) {
+        F3D_HIP_CHECK(hipEventRecord(g_timer.ev[2 * g_timer.n + 1], st));
+        ++g_timer.n;
+      }
+      return F3D_OK;
+    }
+  }
   const int prec = kQuant ? F3D_F32C : F3D_F64;
   T* rec = reinterpret_cast<T*>(ws);
   T* rec_far = kQuant ? reinterpret_cast<T*>(ws + rec_bytes(KIND, prec, pl.ns_pad) / 2) : nullptr;
@@ -1239,7 +1490,6 @@ static int launch_pairsum(const Plan& pl, uint32_t flags, int64_t ns, const doub
   // turns the near/far split off)
   const char* fr = getenv("F3D_PAIRSUM_FAR_RATIO");
   const double far_ratio = kQuant ? ((fr && *fr) ? atof(fr) : kFarRatio32) : 0.0;
-  const bool timed = g_timer.on && g_timer.n < kTimerSlots;
   if (timed) F3D_HIP_CHECK(hipEventRecord(g_timer.ev[2 * g_timer.n], st));
 #define F3D_PS(KK, CL)                                                                        \
   F3D_LAUNCH((pairsum_kernel<T, KIND, KK, CL>), grid, block, 0, st, rec, (const T*)rec_far,  \
@@ -1262,10 +1512,6 @@ static int launch_pairsum(const Plan& pl, uint32_t flags, int64_t ns, const doub
     ++g_timer.n;
   }
 
-  double factor;
-  if (KIND == F3D_STRESSLET) factor = -3.0 / (4.0 * kPi * eta);
-  else factor = 1.0 / (8.0 * kPi * eta);
-  factor *= TwoOverR<T, KIND>::scale;
   ShellEpi epi{};
   if (epi_in) {
     epi = *epi_in;

@@ -186,3 +186,74 @@ def test_self_sum_drops_the_diagonal_without_regularisation(precision):
     got = FK.pairsum("stresslet", X, _dev(q), X, src_nrm=_dev(n), reg=0.0, eps=0.0,
                      precision=precision, exclude_self=True).cpu().numpy().ravel()
     assert rel2(got, ref) < TOL[precision]
+
+
+@pytest.mark.parametrize("kernel", ["oseen", "rotlet", "stresslet"])
+@pytest.mark.parametrize("ns,nt", [(1, 1), (32, 1024), (511, 255), (512, 257), (513, 513),
+                                   (1025, 2048), (700, 2049), (4096, 260), (3, 70001)])
+def test_one_launch_sums_match_the_general_path(kernel, ns, nt, monkeypatch):
+    """Small FP64 calls run in one launch; an explicit launch shape keeps them
+    on the general path.  Both over every form a call can take: weights,
+    exclusion ranges (empty, partial, whole), the self flag, accumulation, AoS,
+    SoA and reversed strides, near and coincident pairs, output over an input.
+
+    Each pair carries a few 1e-15 in both; sums of up to 4096 random terms
+    cancel by at most their root (64): 64 x 1e-14."""
+    print(f"case one-launch {kernel} ns={ns} nt={nt}", flush=True)
+    tol = 64 * 1e-14
+    s, t, d, n = (_dev(a) for a in _problem(ns + nt, ns, nt))
+    rng = np.random.default_rng(nt)
+    w = _dev(rng.uniform(0.5, 2.0, size=ns))
+    lo = rng.integers(0, ns, size=nt)
+    hi = np.minimum(lo + rng.integers(0, 40, size=nt), ns)
+    hi[0], lo[0] = ns, 0  # a target without sources
+    excl = tuple(torch.from_numpy(a.astype(np.int32)).cuda() for a in (lo, hi))
+    soa = lambda a: a.t().contiguous().t()
+    back = lambda a: torch.flip(a, (0,))
+    base = _dev(rng.normal(size=(nt, 3)))
+    kw = dict(src_nrm=n, eta=0.7)
+
+    def call(form):
+        if form == "plain":
+            return FK.pairsum(kernel, s, d, t, **kw)
+        if form == "weights, ranges, accumulate, SoA":
+            out = soa(base.clone())
+            return FK.pairsum(kernel, soa(s), soa(d), soa(t), src_nrm=soa(n), eta=0.7, src_w=w,
+                              excl=excl, out=out, accumulate=True)
+        if form == "mixed strides":
+            return FK.pairsum(kernel, s, d, soa(t), out=torch.empty_like(back(t)), **kw)
+        if form == "output over the densities":
+            dd = torch.zeros((max(ns, nt), 3), dtype=torch.float64, device="cuda")
+            dd[:ns] = d
+            FK.pairsum(kernel, s, dd[:ns], t, out=dd[:nt], **kw)
+            return dd[:nt].clone()
+        m = min(ns, nt)
+        return FK.pairsum(kernel, s[:m], d[:m], s[:m], src_nrm=n[:m], eta=0.7, reg=0.0, eps=0.0,
+                          exclude_self=True)
+
+    for form in ("plain", "weights, ranges, accumulate, SoA", "mixed strides",
+                 "output over the densities", "self"):
+        got = call(form).cpu().numpy()
+        monkeypatch.setenv("F3D_PAIRSUM_K64", "1")
+        ref = call(form).cpu().numpy()
+        monkeypatch.delenv("F3D_PAIRSUM_K64")
+        if form == "self" and min(ns, nt) == 1:
+            assert not got.any() and not ref.any()
+        else:
+            assert rel2(got, ref) < tol, form
+
+
+@pytest.mark.parametrize("n", [258, 1400])
+def test_one_launch_shell_matches_the_general_path(n, monkeypatch):
+    """The shell operator's epilogue (singularity subtraction, completion sum,
+    added flow) on both paths."""
+    from fiber3d_amd import configs
+    from fiber3d_amd.system import Shell
+    xs, ns_, ws_ = configs.make_periphery(n, 3.0)
+    sh = Shell(xs, ns_, ws_)
+    rng = np.random.default_rng(n)
+    q, add = _dev(rng.normal(size=(len(xs), 3))), _dev(rng.normal(size=(len(xs), 3)))
+    got = sh.apply(q, add=add).cpu().numpy()
+    monkeypatch.setenv("F3D_PAIRSUM_K64", "1")
+    ref = sh.apply(q, add=add).cpu().numpy()
+    assert rel2(got, ref) < 64 * 1e-14
