@@ -183,6 +183,32 @@ def test_block_gemv():
     assert rel2(y.cpu().numpy(), ref) < 1e-13
 
 
+@pytest.mark.parametrize("beta", [0.0, 1.0])
+def test_block_gemv_edges(beta):
+    """Row counts at the edges of the segments and column counts at the edges
+    of the waves' column groups (none, one, a group and one more, all waves).
+    Sums of k <= 260 O(1) products: 260 eps of their absolute sum, here taken
+    against |alpha| |M| |x| + |beta y|."""
+    print(f"case block gemv edges beta={beta}", flush=True)
+    rng = np.random.default_rng(11)
+    ms, ks = zip(*[(m, k) for m in (1, 2, 31, 32, 33, 63, 64, 65, 127, 128, 129, 255, 256)
+                   for k in (0, 1, 4, 7, 8, 9, 15, 16, 17, 31, 33, 64, 65, 127, 128, 129, 260)])
+    mats = [rng.normal(size=(m, k)) for m, k in zip(ms, ks)]
+    x_off = np.concatenate([[0], np.cumsum(ks)[:-1]])
+    y_off = np.concatenate([[0], np.cumsum(ms)[:-1]])
+    g = BlockGemv(ms, ks, x_off, y_off)
+    x, y0 = rng.normal(size=sum(ks)), rng.normal(size=sum(ms))
+    y = torch.from_numpy(y0.copy()).cuda()
+    g(g.pack(mats), torch.from_numpy(x).cuda(), y, alpha=-1.5, beta=beta)
+    got = y.cpu().numpy()
+    for M, xo, yo in zip(mats, x_off, y_off):
+        m, k = M.shape
+        xb, yb = x[xo:xo + k], y0[yo:yo + m]
+        ref = -1.5 * (M @ xb) + beta * yb
+        scale = 1.5 * (np.abs(M) @ np.abs(xb)) + np.abs(beta * yb)
+        assert (np.abs(got[yo:yo + m] - ref) <= 260 * 2.3e-16 * scale + 1e-300).all(), (m, k)
+
+
 def test_batched_lu_on_real_fiber_blocks_config2_shape():
     """Workload 2 shape: fibers with N in {16, 24, 32, 48, 64} (n = 4N up to
     256), A_sq assembled from the fiber discretisation; FP32 LU + FP64
