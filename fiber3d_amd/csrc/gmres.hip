@@ -96,6 +96,27 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
   return s;
 }
 
+// sum over i, i + step, ... < end of a[i] b[i], in that order, the loads of
+// eight terms in flight together
+__device__ __forceinline__ double strided_dot(const double* __restrict__ a,
+                                              const double* __restrict__ b, int64_t i,
+                                              int64_t end, int64_t step) {
+  double s = 0.0;
+  for (; i < end; i += 8 * step) {
+    double u[8], v[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int64_t e = i + q * step < end ? i + q * step : i;
+      u[q] = a[e];
+      v[q] = b[e];
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (i + q * step < end) s = fma(u[q], v[q], s);
+  }
+  return s;
+}
+
 // Is this block the last of `total` to arrive at counter ctr?  (The caller
 // wrote its partial results before; the fence orders them before the count.)
 __device__ __forceinline__ bool last_block(int* ctr, int total) {
@@ -112,24 +133,28 @@ __device__ __forceinline__ bool last_block(int* ctr, int total) {
   return last;
 }
 
+// The blocks' partial sums added by one block, in a fixed order.
+__device__ __forceinline__ double part_sum(const double* part, int nb, double* red) {
+  double s = 0.0;
+  for (int b = threadIdx.x; b < nb; b += kGb) s += part[b];
+  return block_sum(s, red);
+}
+
 // ---- start of a cycle: beta = ||r||, V_0 = r / beta, g = beta e_1 ----------
 __global__ void __launch_bounds__(kGb)
 gm_norm_kernel(int64_t n, int m, const double* __restrict__ r, GmresPtrs p) {
   __shared__ double red[kGb / 64];
   const int nb = gridDim.x;
-  double s = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * kGb + threadIdx.x; i < n; i += (int64_t)nb * kGb)
-    s = fma(r[i], r[i], s);
+  double s = strided_dot(r, r, (int64_t)blockIdx.x * kGb + threadIdx.x, n, (int64_t)nb * kGb);
   s = block_sum(s, red);
   if (threadIdx.x == 0) p.part[blockIdx.x] = s;
-  if (last_block(&p.ctl[CTL_CNT0], nb) && threadIdx.x == 0) {
-    double t = 0.0;
-    for (int b = 0; b < nb; ++b) t += p.part[b];
-    const double beta = sqrt(t);
-    for (int k = 0; k <= m; ++k) p.g[k] = 0.0;
-    p.g[0] = beta;
-    p.ctl[CTL_J] = 0;
-    p.ctl[CTL_BREAK] = 0;
+  if (last_block(&p.ctl[CTL_CNT0], nb)) {
+    const double t = part_sum(p.part, nb, red);
+    for (int k = threadIdx.x; k <= m; k += kGb) p.g[k] = k == 0 ? sqrt(t) : 0.0;
+    if (threadIdx.x == 0) {
+      p.ctl[CTL_J] = 0;
+      p.ctl[CTL_BREAK] = 0;
+    }
   }
 }
 
@@ -158,18 +183,19 @@ gm_dots_kernel(int64_t n, int m, const double* __restrict__ V, const double* __r
                GmresPtrs p, int add, int cnt) {
   __shared__ double red[kGb / 64];
   const int j = p.ctl[CTL_J];
+  // slices past the last vector leave at once and are not counted: an arrival
+  // at the counter costs its fences (21 us for 256 blocks at j = 3, 8 for eight)
+  if ((int)blockIdx.y > j) return;
   const int nc = gridDim.x;
   const int c = blockIdx.x;
   const int64_t i0 = (int64_t)c * kGchunk;
   const int64_t i1 = i0 + kGchunk < n ? i0 + kGchunk : n;
   for (int k = blockIdx.y; k <= j; k += gridDim.y) {
     const double* __restrict__ vk = V + (int64_t)k * n;
-    double s = 0.0;
-    for (int64_t i = i0 + threadIdx.x; i < i1; i += kGb) s = fma(vk[i], w[i], s);
-    s = block_sum(s, red);
+    const double s = block_sum(strided_dot(vk, w, i0 + threadIdx.x, i1, kGb), red);
     if (threadIdx.x == 0) p.part[(int64_t)k * nc + c] = s;
   }
-  if (last_block(&p.ctl[cnt], nc * gridDim.y)) {
+  if (last_block(&p.ctl[cnt], nc * min((int)gridDim.y, j + 1))) {
     for (int k = threadIdx.x; k <= j; k += kGb) {
       double t = 0.0;
       for (int b = 0; b < nc; ++b) t += p.part[(int64_t)k * nc + b];
@@ -202,33 +228,48 @@ gm_update_kernel(int64_t n, int m, const double* __restrict__ V, double* __restr
   if (!norm) return;
   s = block_sum(s, red);
   if (threadIdx.x == 0) p.part[blockIdx.x] = s;
-  if (last_block(&p.ctl[CTL_CNT2], gridDim.x) && threadIdx.x == 0) {
-    double t = 0.0;
-    for (int b = 0; b < (int)gridDim.x; ++b) t += p.part[b];
-    const double hn = sqrt(t);
+  if (last_block(&p.ctl[CTL_CNT2], gridDim.x)) {
+    // the column and the earlier rotations come to LDS at once: the chain of
+    // rotations then waits for no memory (10 us for the kernel at j = 3
+    // before, 8 with them in LDS)
+    __shared__ double hc[161], cs[160], sn[160];
+    const double hn = sqrt(part_sum(p.part, (int)gridDim.x, red));
     const int ld = m + 1;
     double* __restrict__ Hc = p.H + (int64_t)j * ld;
     double* __restrict__ Hrc = p.Hr + (int64_t)j * ld;
-    for (int k = 0; k <= j; ++k) Hc[k] = Hrc[k] = p.h[k];
-    Hc[j + 1] = Hrc[j + 1] = hn;
-    // earlier rotations, then this column's
-    for (int k = 0; k < j; ++k) {
-      const double a = Hc[k], b = Hc[k + 1];
-      Hc[k] = p.cs[k] * a + p.sn[k] * b;
-      Hc[k + 1] = -p.sn[k] * a + p.cs[k] * b;
+    for (int k = threadIdx.x; k <= j; k += kGb) {
+      const double v = p.h[k];
+      hc[k] = v;
+      Hrc[k] = v;
+      if (k < j) {
+        cs[k] = p.cs[k];
+        sn[k] = p.sn[k];
+      }
     }
-    const double a = Hc[j], b = Hc[j + 1];
-    const double den = hypot(a, b);
-    const double c = den > 0.0 ? a / den : 1.0, sn = den > 0.0 ? b / den : 0.0;
-    p.cs[j] = c;
-    p.sn[j] = sn;
-    Hc[j] = den;
-    Hc[j + 1] = 0.0;
-    const double gj = p.g[j];
-    p.g[j + 1] = -sn * gj;
-    p.g[j] = c * gj;
-    p.est[j] = fabs(p.g[j + 1]);
-    if (!(hn > 0.0)) p.ctl[CTL_BREAK] = j + 1;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      // earlier rotations, then this column's
+      double a = hc[0];
+      for (int k = 0; k < j; ++k) {
+        const double b = hc[k + 1];
+        hc[k] = cs[k] * a + sn[k] * b;
+        a = -sn[k] * a + cs[k] * b;
+      }
+      const double den = hypot(a, hn);
+      const double c = den > 0.0 ? a / den : 1.0, s1 = den > 0.0 ? hn / den : 0.0;
+      const double gj = p.g[j];
+      Hrc[j + 1] = hn;
+      p.cs[j] = c;
+      p.sn[j] = s1;
+      hc[j] = den;
+      hc[j + 1] = 0.0;
+      p.g[j + 1] = -s1 * gj;
+      p.g[j] = c * gj;
+      p.est[j] = fabs(s1 * gj);
+      if (!(hn > 0.0)) p.ctl[CTL_BREAK] = j + 1;
+    }
+    __syncthreads();
+    for (int k = threadIdx.x; k <= j + 1; k += kGb) Hc[k] = hc[k];
   }
 }
 

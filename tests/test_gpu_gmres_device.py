@@ -88,3 +88,21 @@ def test_invariant_subspace_converges_in_three_steps():
     torch.cuda.synchronize()
     assert r.info == 0 and r.iterations == 3
     assert rel2((d * r.x).cpu().numpy(), b.cpu().numpy()) < 1e-13
+
+
+@pytest.mark.parametrize("n", [2, 255, 257, 2049, 4096, 4097, 33000, 131077])
+def test_steps_at_chunk_edges(n):
+    """Vectors of one and several chunks of the dot products, with fewer and
+    more basis vectors than slices of the grid: the device steps reach the
+    solution of a diagonal system (condition number 2) like the host's."""
+    print(f"case gmres chunk edges n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    d = torch.from_numpy(rng.uniform(1.0, 2.0, size=n)).cuda()
+    b = torch.from_numpy(rng.normal(size=n)).cuda()
+    mv = lambda v, out=None: torch.mul(d, v, out=out) if out is not None else d * v
+    pc = lambda v, out=None: v.clone() if out is None else out.copy_(v)
+    dev = gmres(mv, b, pc, tol=1e-12, engine="device")
+    host = gmres(mv, b, pc, tol=1e-12, engine="host")
+    assert dev.info == 0 and dev.iterations == host.iterations
+    # a residual of 1e-12 |b| and a smallest eigenvalue of 1: |x - b/d| <= 1e-12 |b|
+    assert rel2(dev.x.cpu().numpy(), (b / d).cpu().numpy()) < 2.1e-12
