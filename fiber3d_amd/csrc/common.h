@@ -59,25 +59,57 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // ---- wave64 reductions (device) -----------------------------------------
-__device__ __forceinline__ int wave_min_i32(int v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v = min(v, __shfl_xor(v, o, 64));
+// Lane l meets lane l ^ O, for O = 32, 16, 8, 4, 2, 1: exchanges of register
+// halves and rows, and row rotations (after the step over 8, lanes 8 apart
+// agree, so that a rotation by 4 reaches lane l ^ 4).  No step goes through
+// LDS, whose shuffles cost a wave's start several microseconds when all eight
+// waves of a SIMD reduce at once; the pairs and their order are those of a
+// butterfly of shuffles, so sums are the same to the bit.
+template <int O>
+__device__ __forceinline__ void wave_meet(int v, int& x, int& y) {
+  typedef unsigned u2 __attribute__((ext_vector_type(2)));
+  if constexpr (O == 32 || O == 16) {
+    const u2 s = O == 32 ? __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false)
+                         : __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+    x = (int)s[0];
+    y = (int)s[1];
+  } else {
+    constexpr int ctrl = O == 8 ? 0x128 : O == 4 ? 0x124 : O == 2 ? 0x4e : 0xb1;
+    x = v;
+    y = __builtin_amdgcn_mov_dpp(v, ctrl, 0xf, 0xf, false);
+  }
+}
+template <int O>
+__device__ __forceinline__ void wave_meet(double v, double& x, double& y) {
+  const unsigned long long u = __double_as_longlong(v);
+  int xl, yl, xh, yh;
+  wave_meet<O>((int)(unsigned)u, xl, yl);
+  wave_meet<O>((int)(u >> 32), xh, yh);
+  x = __longlong_as_double(((unsigned long long)(unsigned)xh << 32) | (unsigned)xl);
+  y = __longlong_as_double(((unsigned long long)(unsigned)yh << 32) | (unsigned)yl);
+}
+template <int O = 32, typename T, typename Op>
+__device__ __forceinline__ T wave_fold(T v, Op op) {
+  T x, y;
+  wave_meet<O>(v, x, y);
+  v = op(x, y);
+  if constexpr (O > 1) v = wave_fold<O / 2>(v, op);
   return v;
+}
+__device__ __forceinline__ int wave_min_i32(int v) {
+  return wave_fold(v, [](int a, int b) { return min(a, b); });
 }
 __device__ __forceinline__ int wave_max_i32(int v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
-  return v;
+  return wave_fold(v, [](int a, int b) { return max(a, b); });
 }
 __device__ __forceinline__ double wave_sum_f64(double v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  return wave_fold(v, [](double a, double b) { return a + b; });
+}
+__device__ __forceinline__ double wave_min_f64(double v) {
+  return wave_fold(v, [](double a, double b) { return fmin(a, b); });
 }
 __device__ __forceinline__ double wave_max_f64(double v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-  return v;
+  return wave_fold(v, [](double a, double b) { return fmax(a, b); });
 }
 
 }  // namespace f3d

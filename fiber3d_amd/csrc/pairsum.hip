@@ -6,18 +6,18 @@
 // distance is regularised, r <- sqrt(r^2 + reg^2), while d is kept.
 //
 // Design (MI355X / CDNA4, wave64):
-//   * pack_kernel converts the caller's sources (any AoS/SoA strides, FP64) into
-//     one contiguous record per source (6 or 9 32/64-bit words: position,
+//   * prepare_kernel converts the caller's sources (any AoS/SoA strides, FP64)
+//     into one contiguous record per source (6 or 9 32/64-bit words: position,
 //     density[, normal]), multiplying an optional per-source weight, and
-//     zero-padding to a multiple of the 64-source tile.  tile_box_kernel
-//     records each tile's centre and radius.
+//     zero-padding to a multiple of the 64-source tile; it records each tile's
+//     centre and radius and each target group's box.
 //   * pairsum_kernel: each lane owns K targets (registers).  The source index
 //     is wave-uniform, so source records are fetched with scalar loads into
 //     SGPRs and every VALU op takes its source operand straight from an SGPR:
 //     no LDS traffic and no VGPRs spent on sources.  Sources are split into
 //     P chunks over grid.y so the launch carries thousands of waves.
 //   * FP32C: positions are quantised once per call to 31-bit integers on the
-//     bounding box of sources and targets (bbox_partial/final), so d = t - s is an
+//     bounding box of sources and targets (bbox_partial_kernel), so d = t - s is an
 //     exact integer difference rounded once to FP32; the pair is then
 //     evaluated in FP32 in units of the quantum h and the sum rescaled by
 //     h^-p (the kernels are homogeneous of degree -1 / -2 in d).  Rounding the
@@ -54,7 +54,7 @@ namespace f3d {
 
 constexpr int kTile = 64;        // sources per compensated tile
 constexpr int kBlock = 256;      // threads per block (4 waves)
-constexpr int kPackBlocks = 256; // grid of the pack kernel (sigma partials)
+constexpr int kPackBlocks = 256; // grid of the prepare kernel (sigma partials)
 constexpr double kQuantLevels = 2147483648.0 - 65536.0;  // 2^31 minus margin
 
 // FP64 pairs use w = 2/r, one Newton step on v_rsq_f64 without its factor
@@ -138,11 +138,8 @@ constexpr int kBoxBlocks = 128;
 __device__ __forceinline__ void block_minmax(double (&lo)[3], double (&hi)[3], double* red) {
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      lo[a] = fmin(lo[a], __shfl_xor(lo[a], o, 64));
-      hi[a] = fmax(hi[a], __shfl_xor(hi[a], o, 64));
-    }
+    lo[a] = wave_min_f64(lo[a]);
+    hi[a] = wave_max_f64(hi[a]);
   }
   const int w = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) {
@@ -190,46 +187,39 @@ bbox_partial_kernel(int ns, const double* __restrict__ pos, long sp, long sc, in
   }
 }
 
-__global__ void __launch_bounds__(kBoxBlocks)
-bbox_final_kernel(const double* __restrict__ part, double min_extent, Geo* __restrict__ geo) {
+// The call's geometry from the partial boxes, formed by every block (of 256
+// threads) that needs it: 6 KB from L2 instead of a launch in between.  Block 0
+// leaves it in geo_out for the later kernels.
+__device__ __forceinline__ Geo block_geo(const double* __restrict__ part, double min_extent,
+                                         Geo* __restrict__ geo_out) {
+  __shared__ double red[(256 / 64) * 6];
+  __shared__ Geo g;
+  const int e = (int)threadIdx.x % kBoxBlocks;
   double lo[3], hi[3];
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
-    lo[a] = part[threadIdx.x * 6 + a];
-    hi[a] = part[threadIdx.x * 6 + 3 + a];
+    lo[a] = part[e * 6 + a];
+    hi[a] = part[e * 6 + 3 + a];
   }
-  __shared__ double red[(kBoxBlocks / 64) * 6];
   block_minmax(lo, hi, red);
   if (threadIdx.x == 0) {
     double ext = 0.0;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      geo->origin[a] = lo[a];
+      g.origin[a] = lo[a];
       ext = fmax(ext, hi[a] - lo[a]);
     }
     ext = fmax(ext, min_extent);
-    geo->h = ext / kQuantLevels;
-    geo->inv_h = kQuantLevels / ext;
+    g.h = ext / kQuantLevels;
+    g.inv_h = kQuantLevels / ext;
+    if (blockIdx.x == 0) *geo_out = g;
   }
+  __syncthreads();
+  return g;
 }
 
 __device__ __forceinline__ int quantise(double x, double origin, double inv_h) {
   return (int)rint((x - origin) * inv_h);
-}
-
-// ---------------------------------------------------------------------------
-// Tile boxes: one wave per 64-source tile, the bounding box's centre and the
-// largest distance of a real source from it.
-__device__ __forceinline__ double readfirst_f64(double v) {
-  const unsigned long long u = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readfirstlane((int)(u & 0xffffffffu));
-  const int hi = __builtin_amdgcn_readfirstlane((int)(u >> 32));
-  return __longlong_as_double(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
-}
-__device__ __forceinline__ double wave_min_f64(double v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v = fmin(v, __shfl_xor(v, o, 64));
-  return v;
 }
 
 // ---------------------------------------------------------------------------
@@ -258,12 +248,14 @@ __device__ __forceinline__ unsigned spread3(unsigned v) {
 
 __global__ void __launch_bounds__(256)
 morton_kernel(int n, const double* __restrict__ pos, long sp, long sc,
-              const Geo* __restrict__ geo, unsigned* __restrict__ key, int* __restrict__ val) {
+              const double* __restrict__ box_part, double min_extent, Geo* __restrict__ geo_out,
+              unsigned* __restrict__ key, int* __restrict__ val) {
+  const Geo geo = block_geo(box_part, min_extent, geo_out);
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     unsigned c = 0;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
-      const int q = quantise(pos[(long)i * sp + a * sc], geo->origin[a], geo->inv_h);
+      const int q = quantise(pos[(long)i * sp + a * sc], geo.origin[a], geo.inv_h);
       c |= spread3((unsigned)q >> (31 - kSortBits)) << a;
     }
     key[i] = c;
@@ -417,12 +409,14 @@ static SortBufs sort_set(char* p, int64_t n) {
 }
 
 // Morton order of n points: *perm = the permutation (sorted place -> index).
-static int spatial_order(int64_t n, const double* pos, int64_t sp, int64_t sc, const Geo* geo,
-                         SortBufs b, int* counts, hipStream_t st, const int** perm) {
+static int spatial_order(int64_t n, const double* pos, int64_t sp, int64_t sc,
+                         const double* box_part, double min_extent, Geo* geo, SortBufs b,
+                         int* counts, hipStream_t st, const int** perm) {
   int chunk;
   const int nb = sort_blocks(n, &chunk);
   F3D_LAUNCH(morton_kernel, dim3((unsigned)std::min<int64_t>(ceil_div(n, (int64_t)256), 1024)),
-             dim3(256), 0, st, (int)n, pos, (long)sp, (long)sc, geo, b.key[0], b.val[0]);
+             dim3(256), 0, st, (int)n, pos, (long)sp, (long)sc, box_part, min_extent, geo, b.key[0],
+             b.val[0]);
   int cur = 0;
   for (int shift = 0; shift < 3 * kSortBits; shift += 8) {
     F3D_LAUNCH(radix_count_kernel, dim3(nb), dim3(kSortBlock), 0, st, (int)n, chunk, shift,
@@ -438,73 +432,59 @@ static int spatial_order(int64_t n, const double* pos, int64_t sp, int64_t sc, c
 }
 
 // ---------------------------------------------------------------------------
-// Tile boxes: one wave per 64-source tile (sources in the order of perm when
-// given), the bounding box's centre and the largest distance of a real
-// source from it.
-__global__ void __launch_bounds__(64)
-tile_box_kernel(int ns, int tiles, const double* __restrict__ pos, long sp, long sc,
-                const Geo* __restrict__ geo, const int* __restrict__ perm,
-                TileBox* __restrict__ box) {
-  const int t = blockIdx.x;
-  if (t >= tiles) return;
-  const int j = t * kTile + (int)threadIdx.x;
-  const bool valid = j < ns;
-  const int o = valid ? (perm ? perm[j] : j) : 0;
-  double x[3], lo[3], hi[3], c[3];
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    x[a] = valid ? pos[(long)o * sp + a * sc] : 0.0;
-    lo[a] = wave_min_f64(valid ? x[a] : 1e300);
-    hi[a] = wave_max_f64(valid ? x[a] : -1e300);
-    c[a] = 0.5 * (lo[a] + hi[a]);
-  }
-  double r2 = 0.0;
-  if (valid) {
-#pragma unroll
-    for (int a = 0; a < 3; ++a) r2 += (x[a] - c[a]) * (x[a] - c[a]);
-  }
-  const double rmax = sqrt(wave_max_f64(r2));
-  const bool any = t * kTile < ns;
-  if (threadIdx.x == 0) {
-    TileBox b;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      b.c[a] = any ? c[a] : 0.0;
-      b.q[a] = (any && geo) ? quantise(c[a], geo->origin[a], geo->inv_h) : 0;
-    }
-    // rounding of the centre and the root: a relative margin
-    b.r = any ? rmax * (1.0 + 1e-12) + 1e-300 : -1.0;
-    b.pad = 0;
-    box[t] = b;
-  }
-}
+// Box of a target group (the 64 K targets of a wave of the pair kernel, in the
+// order of tperm when given) and the union of its exclusion ranges; every wave
+// with these targets (one per source chunk) reads it with scalar loads instead
+// of reducing 64 lanes itself.
+struct TargetBox {
+  double lo[3], hi[3];
+  int wlo, whi;
+  double pad;
+};
+static_assert(sizeof(TargetBox) == 64, "one box per half line");
 
 // ---------------------------------------------------------------------------
-// pack: sources -> records.  Also accumulates sigma = sum_j n_j . q_j per
-// block when sigma_part != nullptr (periphery complementary term).
-// FP32C records hold the quantised position as int32 bits in words 0..2.
+// prepare: everything the pair kernel reads, in one launch of kPackBlocks
+// blocks.  A wave takes whole 64-source tiles (in the order of sperm when
+// given): the tile's box (its centre and the largest distance of a real source
+// from it) and its records; then target groups: their boxes.  Also accumulates
+// sigma = sum_j n_j . q_j per block when sigma_part != nullptr (periphery
+// complementary term).  FP32C records hold the quantised position as int32
+// bits in words 0..2; the geometry of the quantisation is formed by each block.
 template <typename T, int KIND>
 __global__ void __launch_bounds__(256)
-pack_kernel(int ns, int ns_pad, const double* __restrict__ pos, const double* __restrict__ nrm,
-            const double* __restrict__ den, const double* __restrict__ w, long sp, long sc,
-            const Geo* __restrict__ geo, const TileBox* __restrict__ tbox,
-            const int* __restrict__ perm, T* __restrict__ rec, T* __restrict__ rec_far,
-            double* __restrict__ sigma_part) {
+prepare_kernel(int ns, int tiles, const double* __restrict__ pos, const double* __restrict__ nrm,
+               const double* __restrict__ den, const double* __restrict__ w, long sp, long sc,
+               const int* __restrict__ sperm, int nt, int groups, int K,
+               const double* __restrict__ tpos, long t_sp, long t_sc,
+               const int* __restrict__ tperm, const int* __restrict__ excl_lo,
+               const int* __restrict__ excl_hi, int self_excl,
+               const double* __restrict__ box_part, double min_extent, Geo* __restrict__ geo_out,
+               TileBox* __restrict__ tbox, TargetBox* __restrict__ gbox, T* __restrict__ rec,
+               T* __restrict__ rec_far, double* __restrict__ sigma_part) {
   constexpr int R = RecLen<T, KIND>::value;
   constexpr bool kQuant = std::is_same<T, float>::value;
+  Geo geo{};
+  if constexpr (kQuant) geo = block_geo(box_part, min_extent, geo_out);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  const int waves = gridDim.x * 4;
   double sig = 0.0;
-  for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < ns_pad; j += gridDim.x * blockDim.x) {
+  for (int tl = wave; tl < tiles; tl += waves) {
+    const int j = tl * kTile + lane;
+    const bool valid = j < ns;
     T r[R];
 #pragma unroll
     for (int c = 0; c < R; ++c) r[c] = 0;
-    // far record position words (FP32C)
-    T f[3] = {0, 0, 0};
+    double x[3] = {0.0, 0.0, 0.0};
     // Zero-density padding for j >= ns; the pair kernel masks those sources,
     // so a target at the padding position never meets an unregularised r = 0.
-    if (j < ns) {
-      const int o = perm ? perm[j] : j;  // original source index
+    if (valid) {
+      const int o = sperm ? sperm[j] : j;  // original source index
       const double wj = w ? w[o] : 1.0;
       const long b = (long)o * sp;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) x[a] = pos[b + a * sc];
       if constexpr (KIND == F3D_STRESSLET) {
         const double n0 = nrm[b], n1 = nrm[b + sc], n2 = nrm[b + 2 * sc];
         const double q0 = den[b] * wj, q1 = den[b + sc] * wj, q2 = den[b + 2 * sc] * wj;
@@ -521,26 +501,88 @@ pack_kernel(int ns, int ns_pad, const double* __restrict__ pos, const double* __
           r[8] = 0.25 * r[5];
         }
       }
+    }
+    double c[3], r2 = 0.0;
+    int q[3] = {0, 0, 0};
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const double lo = wave_min_f64(valid ? x[a] : 1e300);
+      const double hi = wave_max_f64(valid ? x[a] : -1e300);
+      c[a] = 0.5 * (lo + hi);
+      if constexpr (kQuant) q[a] = quantise(c[a], geo.origin[a], geo.inv_h);
+    }
+    if (valid) {
+#pragma unroll
+      for (int a = 0; a < 3; ++a) r2 += (x[a] - c[a]) * (x[a] - c[a]);
+    }
+    const double rmax = sqrt(wave_max_f64(r2));
+    const bool any = tl * kTile < ns;
+    if (lane == 0) {
+      TileBox b;
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
-        const double x = pos[b + a * sc];
+        b.c[a] = any ? c[a] : 0.0;
+        b.q[a] = any ? q[a] : 0;
+      }
+      // rounding of the centre and the root: a relative margin
+      b.r = any ? rmax * (1.0 + 1e-12) + 1e-300 : -1.0;
+      b.pad = 0;
+      tbox[tl] = b;
+    }
+    T f[3] = {0, 0, 0};  // far record position words (FP32C)
+    if (valid) {
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
         if constexpr (kQuant) {
-          const int q = quantise(x, geo->origin[a], geo->inv_h);
-          r[a] = __int_as_float(q);
-          f[a] = (float)(q - tbox[j / kTile].q[a]);
+          const int qa = quantise(x[a], geo.origin[a], geo.inv_h);
+          r[a] = __int_as_float(qa);
+          f[a] = (float)(qa - q[a]);
         } else {
-          r[a] = x;
+          r[a] = x[a];
         }
       }
     }
     T* out = rec + (size_t)j * R;
 #pragma unroll
-    for (int c = 0; c < R; ++c) out[c] = r[c];
+    for (int e = 0; e < R; ++e) out[e] = r[e];
     if constexpr (kQuant) {
       T* of = rec_far + (size_t)j * R;
 #pragma unroll
-      for (int c = 0; c < R; ++c) of[c] = c < 3 ? f[c] : r[c];
+      for (int e = 0; e < R; ++e) of[e] = e < 3 ? f[e] : r[e];
     }
+  }
+  // (from the last wave on: the first ones have a tile more)
+  for (int g = waves - 1 - wave; g < groups; g += waves) {
+    double lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
+    int wlo = 0x7fffffff, whi = -0x7fffffff;
+    for (int k = 0; k < K; ++k) {
+      const int sl = (g * K + k) * 64 + lane;
+      if (sl >= nt) continue;
+      const int i = tperm ? tperm[sl] : sl;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        const double v = tpos[(long)i * t_sp + a * t_sc];
+        lo[a] = fmin(lo[a], v);
+        hi[a] = fmax(hi[a], v);
+      }
+      if (excl_lo != nullptr || self_excl) {
+        const int l = self_excl ? sl : excl_lo[i], h = self_excl ? sl + 1 : excl_hi[i];
+        if (h > l) {
+          wlo = min(wlo, l);
+          whi = max(whi, h);
+        }
+      }
+    }
+    TargetBox b;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      b.lo[a] = wave_min_f64(lo[a]);
+      b.hi[a] = wave_max_f64(hi[a]);
+    }
+    b.wlo = wave_min_i32(wlo);
+    b.whi = wave_max_i32(whi);
+    b.pad = 0.0;
+    if (lane == 0) gbox[g] = b;
   }
   if (sigma_part) {
     __shared__ double red[4];
@@ -759,8 +801,8 @@ pairsum_kernel(const T* __restrict__ rec, const T* __restrict__ rec_far,
                int ns_pad, const double* __restrict__ tpos, long t_sp, long t_sc, int nt,
                const int* __restrict__ excl_lo, const int* __restrict__ excl_hi, int self_excl,
                double reg, double eps, const Geo* __restrict__ geo,
-               const TileBox* __restrict__ tbox, double far_ratio, T* __restrict__ part_hi,
-               T* __restrict__ part_lo) {
+               const TileBox* __restrict__ tbox, const TargetBox* __restrict__ gbox,
+               double far_ratio, T* __restrict__ part_hi, T* __restrict__ part_lo) {
   constexpr bool kQuant = std::is_same<T, float>::value;
   // regularisation constants in the units of the coordinates used
   const double hs = kQuant ? geo->h : 1.0;
@@ -778,8 +820,11 @@ pairsum_kernel(const T* __restrict__ rec, const T* __restrict__ rec_far,
   const int base = blockIdx.x * (64 * K) + lane;
   TCoord<T> tx[K], ty[K], tz[K];
   int lo[K], hi[K];
-  int wlo = 0x7fffffff, whi = -0x7fffffff;
-  double bl[3] = {1e300, 1e300, 1e300}, bh[3] = {-1e300, -1e300, -1e300};
+  // box of the targets and union of their exclusion ranges (wave-uniform)
+  const TargetBox* __restrict__ gb = gbox + blockIdx.x;
+  const double bl[3] = {gb->lo[0], gb->lo[1], gb->lo[2]};
+  const double bh[3] = {gb->hi[0], gb->hi[1], gb->hi[2]};
+  const int wlo = gb->wlo, whi = gb->whi;
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     // slot base + k 64 (the partial's index) holds target i (in spatial
@@ -790,11 +835,6 @@ pairsum_kernel(const T* __restrict__ rec, const T* __restrict__ rec_far,
     const int i = tperm ? tperm[sc] : sc;
     const long b = (long)i * t_sp;
     const double px = tpos[b], py = tpos[b + t_sc], pz = tpos[b + 2 * t_sc];
-    if (sl < nt) {
-      bl[0] = fmin(bl[0], px); bh[0] = fmax(bh[0], px);
-      bl[1] = fmin(bl[1], py); bh[1] = fmax(bh[1], py);
-      bl[2] = fmin(bl[2], pz); bh[2] = fmax(bh[2], pz);
-    }
     if constexpr (kQuant) {
       tx[k] = quantise(px, geo->origin[0], geo->inv_h);
       ty[k] = quantise(py, geo->origin[1], geo->inv_h);
@@ -809,20 +849,7 @@ pairsum_kernel(const T* __restrict__ rec, const T* __restrict__ rec_far,
     if ((excl_lo != nullptr || self_excl) && sl < nt) {
       lo[k] = self_excl ? sl : excl_lo[i];
       hi[k] = self_excl ? sl + 1 : excl_hi[i];
-      if (hi[k] > lo[k]) {
-        wlo = min(wlo, lo[k]);
-        whi = max(whi, hi[k]);
-      }
     }
-  }
-  // Wave-uniform union of the exclusion ranges (kept in SGPRs).
-  wlo = __builtin_amdgcn_readfirstlane(wave_min_i32(wlo));
-  whi = __builtin_amdgcn_readfirstlane(wave_max_i32(whi));
-  // Wave-uniform box of the wave's targets (FP64).
-#pragma unroll
-  for (int a = 0; a < 3; ++a) {
-    bl[a] = readfirst_f64(wave_min_f64(bl[a]));
-    bh[a] = readfirst_f64(wave_max_f64(bh[a]));
   }
 
   T sx[K], sy[K], sz[K], cx[K], cy[K], cz[K];
@@ -1297,6 +1324,11 @@ static size_t tile_bytes(int ns_pad) {
   return align_up((size_t)(ns_pad / kTile) * sizeof(TileBox), 256);
 }
 
+static int64_t target_groups(int K, int64_t nt) { return ceil_div(nt > 0 ? nt : 1, 64 * K); }
+static size_t group_bytes(int K, int64_t nt) {
+  return align_up((size_t)target_groups(K, nt) * sizeof(TargetBox), 256);
+}
+
 static size_t part_bytes(int precision, int P, int64_t nt) {
   const size_t per = precision == F3D_F64 ? 8 : 8;  // f64, or 2 x f32
   return align_up((size_t)P * 3 * (size_t)(nt > 0 ? nt : 1) * per, 256);
@@ -1308,7 +1340,7 @@ static size_t sort_bytes(const Plan& pl, int64_t nt) {
 
 static size_t plan_ws(int kernel, int precision, const Plan& pl, int64_t nt) {
   return rec_bytes(kernel, precision, pl.ns_pad) + tile_bytes(pl.ns_pad) +
-         part_bytes(precision, pl.Pg, nt) +
+         group_bytes(pl.K, nt) + part_bytes(precision, pl.Pg, nt) +
          align_up(kPackBlocks * sizeof(double), 256) + align_up(sizeof(Geo), 256) +
          align_up(kBoxBlocks * 6 * sizeof(double), 256) + sort_bytes(pl, nt);
 }
@@ -1431,6 +1463,8 @@ static int launch_pairsum(const Plan& pl, uint32_t flags, int64_t ns, const doub
   char* p = ws + rec_bytes(KIND, prec, pl.ns_pad);
   TileBox* tbox = reinterpret_cast<TileBox*>(p);
   p += tile_bytes(pl.ns_pad);
+  TargetBox* gbox = reinterpret_cast<TargetBox*>(p);
+  p += group_bytes(pl.K, nt);
   T* part_hi = reinterpret_cast<T*>(p);
   T* part_lo = part_hi + (size_t)pl.Pg * 3 * nt;
   p += part_bytes(prec, pl.Pg, nt);
@@ -1447,14 +1481,11 @@ static int launch_pairsum(const Plan& pl, uint32_t flags, int64_t ns, const doub
   const bool self_excl_flag = (flags & F3D_EXCLUDE_SELF) != 0;
   const bool sorted = pl.sort && lo == nullptr && (!self_excl_flag || same);
 
-  if (kQuant || sorted) {
-    // the quantum must resolve eps; an extent below 64 (eps + reg) is raised
-    const double min_extent = 64.0 * (eps + reg) + 1e-300;
+  // the quantum must resolve eps; an extent below 64 (eps + reg) is raised
+  const double min_extent = 64.0 * (eps + reg) + 1e-300;
+  if (kQuant || sorted)
     F3D_LAUNCH(bbox_partial_kernel, dim3(kBoxBlocks), dim3(256), 0, st, (int)ns, pos, (long)s_sp,
                (long)s_sc, (int)nt, tpos, (long)t_sp, (long)t_sc, box_part);
-    F3D_LAUNCH(bbox_final_kernel, dim3(1), dim3(kBoxBlocks), 0, st, (const double*)box_part,
-               min_extent, geo_buf);
-  }
   // spatial order of sources and targets (one order when they are the same points)
   const int* sperm = nullptr;
   const int* tperm = nullptr;
@@ -1466,26 +1497,27 @@ static int launch_pairsum(const Plan& pl, uint32_t flags, int64_t ns, const doub
     const SortBufs bt = sort_set(p, nt);
     p += sort_set_bytes(nt);
     int* counts = reinterpret_cast<int*>(p);
-    int rc = spatial_order(ns, pos, s_sp, s_sc, geo_buf, bs, counts, st, &sperm);
+    int rc = spatial_order(ns, pos, s_sp, s_sc, box_part, min_extent, geo_buf, bs, counts, st,
+                           &sperm);
     if (rc != F3D_OK) return rc;
     tperm = sperm;
     if (!same) {
-      rc = spatial_order(nt, tpos, t_sp, t_sc, geo_buf, bt, counts, st, &tperm);
+      rc = spatial_order(nt, tpos, t_sp, t_sc, box_part, min_extent, geo_buf, bt, counts, st,
+                         &tperm);
       if (rc != F3D_OK) return rc;
     }
   }
   const bool want_sigma = epi_in != nullptr;
-  const int tiles = pl.ns_pad / kTile;
-  F3D_LAUNCH(tile_box_kernel, dim3((unsigned)tiles), dim3(64), 0, st, (int)ns, tiles, pos,
-             (long)s_sp, (long)s_sc, (const Geo*)geo, sperm, tbox);
-  F3D_LAUNCH((pack_kernel<T, KIND>), dim3(kPackBlocks), dim3(256), 0, st, (int)ns, pl.ns_pad,
-             pos, nrm, den, w, (long)s_sp, (long)s_sc, (const Geo*)geo,
-             (const TileBox*)tbox, sperm, rec, rec_far, want_sigma ? sigma_part : nullptr);
+  const int self_excl = (flags & F3D_EXCLUDE_SELF) ? 1 : 0;
+  F3D_LAUNCH((prepare_kernel<T, KIND>), dim3(kPackBlocks), dim3(256), 0, st, (int)ns,
+             pl.ns_pad / kTile, pos, nrm, den, w, (long)s_sp, (long)s_sc, sperm, (int)nt,
+             (int)target_groups(pl.K, nt), pl.K, tpos, (long)t_sp, (long)t_sc, tperm, lo, hi,
+             self_excl, (const double*)box_part, min_extent, geo_buf, tbox, gbox, rec, rec_far,
+             want_sigma ? sigma_part : nullptr);
 
   const dim3 grid((unsigned)ceil_div(nt, (int64_t)64 * pl.K), (unsigned)pl.Pg);
   const dim3 block((unsigned)(64 * pl.G));
   const bool clamp = kQuant && (flags & F3D_CLAMP_NEAR);
-  const int self_excl = (flags & F3D_EXCLUDE_SELF) ? 1 : 0;
   // F3D_PAIRSUM_FAR_RATIO overrides the FP32C far ratio (a very large value
   // turns the near/far split off)
   const char* fr = getenv("F3D_PAIRSUM_FAR_RATIO");
@@ -1495,8 +1527,8 @@ static int launch_pairsum(const Plan& pl, uint32_t flags, int64_t ns, const doub
   F3D_LAUNCH((pairsum_kernel<T, KIND, KK, CL>), grid, block, 0, st, rec, (const T*)rec_far,  \
              tperm, pl.chunk, (int)ns, pl.ns_pad, tpos, (long)t_sp, (long)t_sc,               \
              (int)nt, lo, hi,                                                                 \
-             self_excl, reg, eps, (const Geo*)geo, (const TileBox*)tbox, far_ratio, part_hi,  \
-             part_lo)
+             self_excl, reg, eps, (const Geo*)geo, (const TileBox*)tbox,                      \
+             (const TargetBox*)gbox, far_ratio, part_hi, part_lo)
   if (clamp) {
     if (pl.K == 1) F3D_PS(1, true);
     else if (pl.K == 2) F3D_PS(2, true);
@@ -1696,7 +1728,10 @@ extern "C" int f3d_pairsum(int kernel, int precision, uint32_t flags, int64_t ns
 // the records, partial sums and bounding box it reads.
 namespace f3d {
 constexpr size_t kScratchBytes = size_t(F3D_NOALLOC_SCRATCH_BYTES);
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+// room for the target boxes beside it, so that they take none of a call's
+// share: at most kScratchBytes / 24 targets have room for one partial sum
+constexpr size_t kScratchBoxes = (kScratchBytes / 24 / 64 + 1) * sizeof(TargetBox) + 256;
+static __device__ __align__(256) unsigned char scratch[kScratchBytes + kScratchBoxes];
 constexpr int kMaxDevices = 64;
 static void* g_scratch_ptr[kMaxDevices];
 static std::mutex g_scratch_mu;
@@ -1727,9 +1762,11 @@ extern "C" int f3d_pairsum_noalloc(int kernel, int precision, uint32_t flags, in
   void* ws = nullptr;
   const int rc = scratch_for_current_device(&ws);
   if (rc != F3D_OK) return rc;
+  const size_t boxes = group_bytes(make_plan(kernel, precision, ns, nt).K, nt);
+  const size_t cap = kScratchBytes + std::min(boxes, kScratchBoxes);
   return pairsum_impl(kernel, precision, flags, ns, src_pos, src_nrm, src_den, src_w, s_sp, s_sc,
                       nt, trg_pos, t_sp, t_sc, excl_lo, excl_hi, eta, reg, eps, out, o_sp, o_sc,
-                      ws, kScratchBytes, nullptr, stream, true);
+                      ws, cap, nullptr, stream, true);
 }
 
 extern "C" size_t f3d_periphery_workspace_size(int precision, int64_t n) {
