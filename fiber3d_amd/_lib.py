@@ -42,6 +42,14 @@ SIGNATURES = {
     "f3d_pairsum_timer_read": (ctypes.c_int, [ctypes.POINTER(ctypes.c_double),
                                               ctypes.POINTER(ctypes.c_int32)]),
     "f3d_pairsum_workspace_size": (_sz, [ctypes.c_int, ctypes.c_int, _i64, _i64]),
+    "f3d_pairsum_strided": (ctypes.c_int, [
+        ctypes.c_int, ctypes.c_int, _u32,
+        _i64, _c_p, _i64, _i64, _c_p, _i64, _i64, _c_p, _i64, _i64, _c_p,
+        _i64, _c_p, _i64, _i64,
+        _c_p, _c_p,
+        _f64, _f64, _f64,
+        _c_p, _i64, _i64,
+        _c_p, _sz, _c_p]),
     "f3d_pairsum": (ctypes.c_int, [
         ctypes.c_int, ctypes.c_int, _u32,
         _i64, _c_p, _c_p, _c_p, _c_p, _i64, _i64,

@@ -70,6 +70,15 @@ struct TwoOverR {
       !value ? 1.0 : KIND == F3D_OSEEN ? 0.5 : KIND == F3D_ROTLET ? 0.125 : 1.0 / 32.0;
 };
 
+// A call's sources: positions, normals, densities (n points of three
+// components, each with its own point and component stride) and weights.
+struct Sources {
+  const double *pos, *nrm, *den, *w;
+  long sp, sc;      // strides of pos
+  long n_sp, n_sc;  // of nrm
+  long d_sp, d_sc;  // of den
+};
+
 // Record words per source, unpadded so that a group of records loads with a
 // few wide scalar loads: 6 for Oseen and rotlet (x, y, z, f or tau), 9 for
 // the stresslet (x, y, z, n, q) and for FP64 Oseen (x, y, z, f, f/4).  FP32C
@@ -453,10 +462,8 @@ static_assert(sizeof(TargetBox) == 64, "one box per half line");
 // bits in words 0..2; the geometry of the quantisation is formed by each block.
 template <typename T, int KIND>
 __global__ void __launch_bounds__(256)
-prepare_kernel(int ns, int tiles, const double* __restrict__ pos, const double* __restrict__ nrm,
-               const double* __restrict__ den, const double* __restrict__ w, long sp, long sc,
-               const int* __restrict__ sperm, int nt, int groups, int K,
-               const double* __restrict__ tpos, long t_sp, long t_sc,
+prepare_kernel(int ns, int tiles, const Sources src, const int* __restrict__ sperm,
+               int nt, int groups, int K, const double* __restrict__ tpos, long t_sp, long t_sc,
                const int* __restrict__ tperm, const int* __restrict__ excl_lo,
                const int* __restrict__ excl_hi, int self_excl,
                const double* __restrict__ box_part, double min_extent, Geo* __restrict__ geo_out,
@@ -481,20 +488,22 @@ prepare_kernel(int ns, int tiles, const double* __restrict__ pos, const double* 
     // so a target at the padding position never meets an unregularised r = 0.
     if (valid) {
       const int o = sperm ? sperm[j] : j;  // original source index
-      const double wj = w ? w[o] : 1.0;
-      const long b = (long)o * sp;
+      const double wj = src.w ? src.w[o] : 1.0;
+      const double* __restrict__ p = src.pos + o * src.sp;
+      const double* __restrict__ d = src.den + o * src.d_sp;
 #pragma unroll
-      for (int a = 0; a < 3; ++a) x[a] = pos[b + a * sc];
+      for (int a = 0; a < 3; ++a) x[a] = p[a * src.sc];
+      const double q0 = d[0] * wj, q1 = d[src.d_sc] * wj, q2 = d[2 * src.d_sc] * wj;
       if constexpr (KIND == F3D_STRESSLET) {
-        const double n0 = nrm[b], n1 = nrm[b + sc], n2 = nrm[b + 2 * sc];
-        const double q0 = den[b] * wj, q1 = den[b + sc] * wj, q2 = den[b + 2 * sc] * wj;
+        const double* __restrict__ n = src.nrm + o * src.n_sp;
+        const double n0 = n[0], n1 = n[src.n_sc], n2 = n[2 * src.n_sc];
         r[3] = (T)n0; r[4] = (T)n1; r[5] = (T)n2;
         r[6] = (T)q0; r[7] = (T)q1; r[8] = (T)q2;
         sig += n0 * q0 + n1 * q1 + n2 * q2;
       } else {
-        r[3] = (T)(den[b] * wj);
-        r[4] = (T)(den[b + sc] * wj);
-        r[5] = (T)(den[b + 2 * sc] * wj);
+        r[3] = (T)q0;
+        r[4] = (T)q1;
+        r[5] = (T)q2;
         if constexpr (TwoOverR<T, KIND>::value && KIND == F3D_OSEEN) {
           r[6] = 0.25 * r[3];
           r[7] = 0.25 * r[4];
@@ -1076,9 +1085,8 @@ constexpr int kDirectStage = 512;
 
 template <int KIND, int K, bool MASK>
 __global__ void __launch_bounds__(256)
-pairsum_direct_kernel(int ns, const double* __restrict__ pos, const double* __restrict__ nrm,
-                      const double* __restrict__ den, const double* __restrict__ w, long s_sp,
-                      long s_sc, int nt, const double* __restrict__ tpos, long t_sp, long t_sc,
+pairsum_direct_kernel(int ns, const Sources src, int nt, const double* __restrict__ tpos,
+                      long t_sp, long t_sc,
                       const int* __restrict__ excl_lo, const int* __restrict__ excl_hi,
                       double reg2, double eps2, double factor, int lg, double* __restrict__ out,
                       long o_sp, long o_sc, int accumulate, ShellEpi epi) {
@@ -1115,16 +1123,16 @@ pairsum_direct_kernel(int ns, const double* __restrict__ pos, const double* __re
     for (int u = 0; u < PER; ++u) {
       const int j = j0 + t + 256 * u;
       if (j < ns) {
-        const long b = (long)j * s_sp;
-        const double wj = w ? w[j] : 1.0;
+        const double wj = src.w ? src.w[j] : 1.0;
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-          nx[u][c] = pos[b + c * s_sc];
+          nx[u][c] = src.pos[j * src.sp + c * src.sc];
+          const double d = src.den[j * src.d_sp + c * src.d_sc] * wj;
           if constexpr (KIND == F3D_STRESSLET) {
-            nx[u][3 + c] = nrm[b + c * s_sc];
-            nx[u][6 + c] = den[b + c * s_sc] * wj;
+            nx[u][3 + c] = src.nrm[j * src.n_sp + c * src.n_sc];
+            nx[u][6 + c] = d;
           } else {
-            nx[u][3 + c] = den[b + c * s_sc] * wj;
+            nx[u][3 + c] = d;
           }
         }
       }
@@ -1406,22 +1414,20 @@ static DirectShape direct_shape(const Plan& pl, int64_t ns, int64_t nt) {
 // Whether the output overlaps an input: the direct kernel's workgroups read
 // inputs after others have written.  (The epilogue's arrays are read at the
 // written index by the thread that writes it; its q is den.)
-static bool direct_aliases(int64_t ns, const double* pos, const double* nrm, const double* den,
-                           const double* w, int64_t s_sp, int64_t s_sc, int64_t nt,
-                           const double* tpos, int64_t t_sp, int64_t t_sc, const int32_t* lo,
-                           const int32_t* hi, const double* out, int64_t o_sp, int64_t o_sc) {
+static bool direct_aliases(int64_t ns, const Sources& s, int64_t nt, const double* tpos,
+                           int64_t t_sp, int64_t t_sc, const int32_t* lo, const int32_t* hi,
+                           const double* out, int64_t o_sp, int64_t o_sc) {
   const Span o = span_of(out, nt, o_sp, o_sc, 8);
-  return overlap(o, span_of(pos, ns, s_sp, s_sc, 8)) ||
-         overlap(o, span_of(nrm, ns, s_sp, s_sc, 8)) ||
-         overlap(o, span_of(den, ns, s_sp, s_sc, 8)) || overlap(o, span_of(w, ns, 1, 0, 8)) ||
-         overlap(o, span_of(tpos, nt, t_sp, t_sc, 8)) || overlap(o, span_of(lo, nt, 1, 0, 4)) ||
-         overlap(o, span_of(hi, nt, 1, 0, 4));
+  return overlap(o, span_of(s.pos, ns, s.sp, s.sc, 8)) ||
+         overlap(o, span_of(s.nrm, ns, s.n_sp, s.n_sc, 8)) ||
+         overlap(o, span_of(s.den, ns, s.d_sp, s.d_sc, 8)) ||
+         overlap(o, span_of(s.w, ns, 1, 0, 8)) || overlap(o, span_of(tpos, nt, t_sp, t_sc, 8)) ||
+         overlap(o, span_of(lo, nt, 1, 0, 4)) || overlap(o, span_of(hi, nt, 1, 0, 4));
 }
 
 template <typename T, int KIND>
-static int launch_pairsum(const Plan& pl, uint32_t flags, int64_t ns, const double* pos,
-                          const double* nrm, const double* den, const double* w, int64_t s_sp,
-                          int64_t s_sc, int64_t nt, const double* tpos, int64_t t_sp,
+static int launch_pairsum(const Plan& pl, uint32_t flags, int64_t ns, const Sources& src,
+                          int64_t nt, const double* tpos, int64_t t_sp,
                           int64_t t_sc, const int32_t* lo, const int32_t* hi, double eta,
                           double reg, double eps, double* out, int64_t o_sp, int64_t o_sc,
                           char* ws, const ShellEpi* epi_in, hipStream_t st) {
@@ -1431,16 +1437,14 @@ static int launch_pairsum(const Plan& pl, uint32_t flags, int64_t ns, const doub
   const bool timed = g_timer.on && g_timer.n < kTimerSlots;
   if constexpr (!kQuant) {
     const DirectShape d = direct_shape(pl, ns, nt);
-    if (d.k > 0 && !direct_aliases(ns, pos, nrm, den, w, s_sp, s_sc, nt, tpos, t_sp, t_sc, lo, hi,
-                                   out, o_sp, o_sc)) {
+    if (d.k > 0 && !direct_aliases(ns, src, nt, tpos, t_sp, t_sc, lo, hi, out, o_sp, o_sc)) {
       if (timed) F3D_HIP_CHECK(hipEventRecord(g_timer.ev[2 * g_timer.n], st));
       const dim3 grid((unsigned)ceil_div(nt, (int64_t)d.k << d.lg));
       const ShellEpi epi = epi_in ? *epi_in : ShellEpi{};
-#define F3D_PD(K, MASK)                                                                         \
-  F3D_LAUNCH((pairsum_direct_kernel<KIND, K, MASK>), grid, dim3(256), 0, st, (int)ns, pos, nrm, \
-             den, w, (long)s_sp, (long)s_sc, (int)nt, tpos, (long)t_sp, (long)t_sc, lo, hi,     \
-             reg * reg, eps * eps, factor, d.lg, out, (long)o_sp, (long)o_sc,                   \
-             (flags & F3D_ACCUMULATE) ? 1 : 0, epi)
+#define F3D_PD(K, MASK)                                                                        \
+  F3D_LAUNCH((pairsum_direct_kernel<KIND, K, MASK>), grid, dim3(256), 0, st, (int)ns, src,     \
+             (int)nt, tpos, (long)t_sp, (long)t_sc, lo, hi, reg * reg, eps * eps, factor, d.lg, \
+             out, (long)o_sp, (long)o_sc, (flags & F3D_ACCUMULATE) ? 1 : 0, epi)
       const bool mask = lo != nullptr || (flags & F3D_EXCLUDE_SELF) != 0;
       if (d.k == 1) {
         if (mask) F3D_PD(1, true);
@@ -1477,15 +1481,15 @@ static int launch_pairsum(const Plan& pl, uint32_t flags, int64_t ns, const doub
   p += align_up(sizeof(Geo), 256);
   double* box_part = reinterpret_cast<double*>(p);
   p += align_up(kBoxBlocks * 6 * sizeof(double), 256);
-  const bool same = pos == tpos && s_sp == t_sp && s_sc == t_sc && ns == nt;
+  const bool same = src.pos == tpos && src.sp == t_sp && src.sc == t_sc && ns == nt;
   const bool self_excl_flag = (flags & F3D_EXCLUDE_SELF) != 0;
   const bool sorted = pl.sort && lo == nullptr && (!self_excl_flag || same);
 
   // the quantum must resolve eps; an extent below 64 (eps + reg) is raised
   const double min_extent = 64.0 * (eps + reg) + 1e-300;
   if (kQuant || sorted)
-    F3D_LAUNCH(bbox_partial_kernel, dim3(kBoxBlocks), dim3(256), 0, st, (int)ns, pos, (long)s_sp,
-               (long)s_sc, (int)nt, tpos, (long)t_sp, (long)t_sc, box_part);
+    F3D_LAUNCH(bbox_partial_kernel, dim3(kBoxBlocks), dim3(256), 0, st, (int)ns, src.pos, src.sp,
+               src.sc, (int)nt, tpos, (long)t_sp, (long)t_sc, box_part);
   // spatial order of sources and targets (one order when they are the same points)
   const int* sperm = nullptr;
   const int* tperm = nullptr;
@@ -1497,7 +1501,7 @@ static int launch_pairsum(const Plan& pl, uint32_t flags, int64_t ns, const doub
     const SortBufs bt = sort_set(p, nt);
     p += sort_set_bytes(nt);
     int* counts = reinterpret_cast<int*>(p);
-    int rc = spatial_order(ns, pos, s_sp, s_sc, box_part, min_extent, geo_buf, bs, counts, st,
+    int rc = spatial_order(ns, src.pos, src.sp, src.sc, box_part, min_extent, geo_buf, bs, counts, st,
                            &sperm);
     if (rc != F3D_OK) return rc;
     tperm = sperm;
@@ -1510,9 +1514,8 @@ static int launch_pairsum(const Plan& pl, uint32_t flags, int64_t ns, const doub
   const bool want_sigma = epi_in != nullptr;
   const int self_excl = (flags & F3D_EXCLUDE_SELF) ? 1 : 0;
   F3D_LAUNCH((prepare_kernel<T, KIND>), dim3(kPackBlocks), dim3(256), 0, st, (int)ns,
-             pl.ns_pad / kTile, pos, nrm, den, w, (long)s_sp, (long)s_sc, sperm, (int)nt,
-             (int)target_groups(pl.K, nt), pl.K, tpos, (long)t_sp, (long)t_sc, tperm, lo, hi,
-             self_excl, (const double*)box_part, min_extent, geo_buf, tbox, gbox, rec, rec_far,
+             pl.ns_pad / kTile, src, sperm, (int)nt, (int)target_groups(pl.K, nt), pl.K, tpos,
+             (long)t_sp, (long)t_sc, tperm, lo, hi, self_excl, (const double*)box_part, min_extent, geo_buf, tbox, gbox, rec, rec_far,
              want_sigma ? sigma_part : nullptr);
 
   const dim3 grid((unsigned)ceil_div(nt, (int64_t)64 * pl.K), (unsigned)pl.Pg);
@@ -1559,9 +1562,8 @@ static int launch_pairsum(const Plan& pl, uint32_t flags, int64_t ns, const doub
 // fit_ws: shrink the source split until the workspace fits ws_bytes (the
 // allocation-free entry point, whose scratch has a fixed size) instead of
 // requiring the default plan's size.
-static int pairsum_impl(int kernel, int precision, uint32_t flags, int64_t ns, const double* pos,
-                        const double* nrm, const double* den, const double* w, int64_t s_sp,
-                        int64_t s_sc, int64_t nt, const double* tpos, int64_t t_sp, int64_t t_sc,
+static int pairsum_impl(int kernel, int precision, uint32_t flags, int64_t ns, const Sources& src,
+                        int64_t nt, const double* tpos, int64_t t_sp, int64_t t_sc,
                         const int32_t* lo, const int32_t* hi, double eta, double reg, double eps,
                         double* out, int64_t o_sp, int64_t o_sc, void* ws, size_t ws_bytes,
                         const ShellEpi* epi, void* stream, bool fit_ws = false) {
@@ -1592,8 +1594,9 @@ static int pairsum_impl(int kernel, int precision, uint32_t flags, int64_t ns, c
                ShellEpi{});
     return F3D_OK;
   }
-  F3D_REQUIRE(pos != nullptr && den != nullptr, F3D_EINVAL, "pairsum: NULL source arrays");
-  F3D_REQUIRE(kernel != F3D_STRESSLET || nrm != nullptr, F3D_EINVAL,
+  F3D_REQUIRE(src.pos != nullptr && src.den != nullptr, F3D_EINVAL,
+              "pairsum: NULL source arrays");
+  F3D_REQUIRE(kernel != F3D_STRESSLET || src.nrm != nullptr, F3D_EINVAL,
               "pairsum: stresslet needs normals");
   Plan pl;
   if (fit_ws) {
@@ -1608,8 +1611,8 @@ static int pairsum_impl(int kernel, int precision, uint32_t flags, int64_t ns, c
   F3D_REQUIRE(ws != nullptr && ws_bytes >= need, F3D_EWORKSPACE,
               "pairsum: workspace %zu bytes < required %zu", ws_bytes, need);
   char* wsc = reinterpret_cast<char*>(ws);
-#define F3D_ARGS pl, flags, ns, pos, nrm, den, w, s_sp, s_sc, nt, tpos, t_sp, t_sc, lo, hi, eta, \
-                 reg, eps, out, o_sp, o_sc, wsc, epi, st
+#define F3D_ARGS pl, flags, ns, src, nt, tpos, t_sp, t_sc, lo, hi, eta, reg, eps, out, o_sp, o_sc, \
+                 wsc, epi, st
   if (precision == F3D_F64) {
     if (kernel == F3D_OSEEN) return launch_pairsum<double, F3D_OSEEN>(F3D_ARGS);
     if (kernel == F3D_ROTLET) return launch_pairsum<double, F3D_ROTLET>(F3D_ARGS);
@@ -1715,9 +1718,23 @@ extern "C" int f3d_pairsum(int kernel, int precision, uint32_t flags, int64_t ns
                            const int32_t* excl_lo, const int32_t* excl_hi, double eta, double reg,
                            double eps, double* out, int64_t o_sp, int64_t o_sc, void* ws,
                            size_t ws_bytes, void* stream) {
-  return pairsum_impl(kernel, precision, flags, ns, src_pos, src_nrm, src_den, src_w, s_sp, s_sc,
-                      nt, trg_pos, t_sp, t_sc, excl_lo, excl_hi, eta, reg, eps, out, o_sp, o_sc,
-                      ws, ws_bytes, nullptr, stream);
+  const Sources src{src_pos, src_nrm, src_den, src_w, s_sp, s_sc, s_sp, s_sc, s_sp, s_sc};
+  return pairsum_impl(kernel, precision, flags, ns, src, nt, trg_pos, t_sp, t_sc, excl_lo, excl_hi,
+                      eta, reg, eps, out, o_sp, o_sc, ws, ws_bytes, nullptr, stream);
+}
+
+extern "C" int f3d_pairsum_strided(int kernel, int precision, uint32_t flags, int64_t ns,
+                                   const double* src_pos, int64_t s_sp, int64_t s_sc,
+                                   const double* src_nrm, int64_t n_sp, int64_t n_sc,
+                                   const double* src_den, int64_t d_sp, int64_t d_sc,
+                                   const double* src_w, int64_t nt, const double* trg_pos,
+                                   int64_t t_sp, int64_t t_sc, const int32_t* excl_lo,
+                                   const int32_t* excl_hi, double eta, double reg, double eps,
+                                   double* out, int64_t o_sp, int64_t o_sc, void* ws,
+                                   size_t ws_bytes, void* stream) {
+  const Sources src{src_pos, src_nrm, src_den, src_w, s_sp, s_sc, n_sp, n_sc, d_sp, d_sc};
+  return pairsum_impl(kernel, precision, flags, ns, src, nt, trg_pos, t_sp, t_sc, excl_lo, excl_hi,
+                      eta, reg, eps, out, o_sp, o_sc, ws, ws_bytes, nullptr, stream);
 }
 
 // ---------------------------------------------------------------------------
@@ -1764,9 +1781,9 @@ extern "C" int f3d_pairsum_noalloc(int kernel, int precision, uint32_t flags, in
   if (rc != F3D_OK) return rc;
   const size_t boxes = group_bytes(make_plan(kernel, precision, ns, nt).K, nt);
   const size_t cap = kScratchBytes + std::min(boxes, kScratchBoxes);
-  return pairsum_impl(kernel, precision, flags, ns, src_pos, src_nrm, src_den, src_w, s_sp, s_sc,
-                      nt, trg_pos, t_sp, t_sc, excl_lo, excl_hi, eta, reg, eps, out, o_sp, o_sc,
-                      ws, cap, nullptr, stream, true);
+  const Sources src{src_pos, src_nrm, src_den, src_w, s_sp, s_sc, s_sp, s_sc, s_sp, s_sc};
+  return pairsum_impl(kernel, precision, flags, ns, src, nt, trg_pos, t_sp, t_sc, excl_lo, excl_hi,
+                      eta, reg, eps, out, o_sp, o_sc, ws, cap, nullptr, stream, true);
 }
 
 extern "C" size_t f3d_periphery_workspace_size(int precision, int64_t n) {
@@ -1783,8 +1800,9 @@ extern "C" int f3d_periphery_apply(int precision, int64_t n, const double* pos,
   F3D_REQUIRE(n > 0, F3D_EINVAL, "periphery_apply: n must be positive");
   F3D_REQUIRE(nrm && w && ex && ey && ez && q, F3D_EINVAL, "periphery_apply: NULL argument");
   ShellEpi epi{nrm, w, ex, ey, ez, q, add, nullptr};
-  return pairsum_impl(F3D_STRESSLET, precision, F3D_EXCLUDE_SELF, n, pos, nrm, q, nullptr, sp, sc, n, pos, sp,
-                      sc, nullptr, nullptr, eta, reg, eps, out, sp, sc, ws, ws_bytes, &epi,
+  const Sources src{pos, nrm, q, nullptr, sp, sc, sp, sc, sp, sc};
+  return pairsum_impl(F3D_STRESSLET, precision, F3D_EXCLUDE_SELF, n, src, n, pos, sp, sc, nullptr,
+                      nullptr, eta, reg, eps, out, sp, sc, ws, ws_bytes, &epi,
                       stream);
 }
 

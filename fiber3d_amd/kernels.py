@@ -118,9 +118,13 @@ def pairsum(kernel, src_pos, src_den, trg_pos, src_nrm=None, src_w=None, excl=No
     k = {"oseen": L.OSEEN, "rotlet": L.ROTLET, "stresslet": L.STRESSLET}[kernel]
     lib = L.load()
     _ensure_tuned()
-    (sp_, sd_, sn_), (s_sp, s_sc) = _as_common([src_pos, src_den, src_nrm])
     nt = trg_pos.shape[0]
-    ns = sp_.shape[0]
+    ns = src_pos.shape[0]
+    if src_den.shape != src_pos.shape or (src_nrm is not None and src_nrm.shape != src_pos.shape):
+        (src_pos, src_den, src_nrm), _ = _as_common([src_pos, src_den, src_nrm])
+    s_sp, s_sc = _strides3(src_pos)
+    d_sp, d_sc = _strides3(src_den)
+    n_sp, n_sc = (0, 0) if src_nrm is None else _strides3(src_nrm)
     t_sp, t_sc = _strides3(trg_pos)
     if out is None:
         out = torch.empty((nt, 3), dtype=torch.float64, device=trg_pos.device)
@@ -136,10 +140,11 @@ def pairsum(kernel, src_pos, src_den, trg_pos, src_nrm=None, src_w=None, excl=No
     ws = workspace(need)
     flags = ((L.ACCUMULATE if accumulate else 0) | (L.CLAMP_NEAR if clamp_near else 0)
              | (L.EXCLUDE_SELF if exclude_self else 0))
-    rc = lib.f3d_pairsum(k, prec, flags, ns, L.ptr(sp_), L.ptr(sn_), L.ptr(sd_), L.ptr(src_w),
-                         s_sp, s_sc, nt, L.ptr(trg_pos), t_sp, t_sc, L.ptr(lo), L.ptr(hi),
-                         float(eta), float(reg), float(eps), L.ptr(out), o_sp, o_sc,
-                         L.ptr(ws), ws.numel(), _stream())
+    rc = lib.f3d_pairsum_strided(
+        k, prec, flags, ns, L.ptr(src_pos), s_sp, s_sc, L.ptr(src_nrm), n_sp, n_sc,
+        L.ptr(src_den), d_sp, d_sc, L.ptr(src_w), nt, L.ptr(trg_pos), t_sp, t_sc, L.ptr(lo),
+        L.ptr(hi), float(eta), float(reg), float(eps), L.ptr(out), o_sp, o_sc, L.ptr(ws),
+        ws.numel(), _stream())
     L.check(rc, "f3d_pairsum")
     return out
 

@@ -105,7 +105,7 @@ int f3d_lu_set_launch(int precision, int32_t factor_waves_per_cu, int32_t solve_
 int f3d_gemm_set_stream(int32_t n, int32_t enable);
 
 /*
- * Timing of the pair kernel alone (not the bounding-box, pack and reduce
+ * Timing of the pair kernel alone (not the bounding-box, prepare and reduce
  * launches around it): enable != 0 clears the record and makes every later
  * f3d_pairsum / f3d_periphery_apply record a HIP event pair around its pair
  * kernel on the caller's stream (at most 4096 launches are kept); enable == 0
@@ -155,6 +155,22 @@ int f3d_pairsum(int kernel, int precision, uint32_t flags,
                 double eta, double reg, double eps,
                 double* out, int64_t o_sp, int64_t o_sc,
                 void* ws, size_t ws_bytes, void* stream);
+
+/*
+ * f3d_pairsum with strides of their own for the normals (n_sp, n_sc) and the
+ * densities (d_sp, d_sc): positions in one layout and densities in another
+ * need no copy.
+ */
+int f3d_pairsum_strided(int kernel, int precision, uint32_t flags,
+                        int64_t ns, const double* src_pos, int64_t s_sp, int64_t s_sc,
+                        const double* src_nrm, int64_t n_sp, int64_t n_sc,
+                        const double* src_den, int64_t d_sp, int64_t d_sc,
+                        const double* src_w,
+                        int64_t nt, const double* trg_pos, int64_t t_sp, int64_t t_sc,
+                        const int32_t* excl_lo, const int32_t* excl_hi,
+                        double eta, double reg, double eps,
+                        double* out, int64_t o_sp, int64_t o_sc,
+                        void* ws, size_t ws_bytes, void* stream);
 
 /*
  * Allocation-free f3d_pairsum.  No counterpart in the reference: it is for

@@ -257,3 +257,19 @@ def test_one_launch_shell_matches_the_general_path(n, monkeypatch):
     monkeypatch.setenv("F3D_PAIRSUM_K64", "1")
     ref = sh.apply(q, add=add).cpu().numpy()
     assert rel2(got, ref) < 64 * 1e-14
+
+
+@pytest.mark.parametrize("precision,ns,nt", [("f64", 300, 70), ("f64", 5000, 3000),
+                                             ("f32c", 300, 70)])
+def test_densities_and_normals_in_their_own_layouts(precision, ns, nt):
+    """Positions, normals and densities in different layouts (in both paths of
+    FP64) give the bits of the same call on contiguous copies."""
+    print(f"case layouts {precision} ns={ns}", flush=True)
+    s, t, d, n = (_dev(a) for a in _problem(ns, ns, nt, near=False))
+    soa = d.t().contiguous().t()
+    every_other = torch.empty((2 * ns, 3), dtype=torch.float64, device="cuda")[::2].copy_(n)
+    kw = dict(eta=0.8, precision=precision)
+    a = FK.pairsum("stresslet", s, soa, t, src_nrm=every_other, **kw)
+    b = FK.pairsum("stresslet", s, d, t, src_nrm=n, **kw)
+    assert torch.equal(a, b)
+    assert torch.equal(FK.pairsum("oseen", s, soa, t, **kw), FK.pairsum("oseen", s, d, t, **kw))
