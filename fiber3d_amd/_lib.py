@@ -28,6 +28,13 @@ _u32 = ctypes.c_uint32
 _f64 = ctypes.c_double
 _sz = ctypes.c_size_t
 
+
+class GemvTerm(ctypes.Structure):
+    """f3d_gemv_term: one product of f3d_block_gemv_sum."""
+    _fields_ = [("m", _c_p), ("k", _c_p), ("m_off", _c_p), ("x_off", _c_p), ("M", _c_p),
+                ("x", _c_p), ("alpha", _f64)]
+
+
 # name -> (restype, argtypes)
 SIGNATURES = {
     "f3d_last_error": (ctypes.c_char_p, []),
@@ -107,6 +114,7 @@ SIGNATURES = {
     "f3d_gmres_solve": (ctypes.c_int, [_i64, _i32, _i32, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p]),
     "f3d_dense_gemv_batched": (ctypes.c_int, [_i64, _i32, _c_p, _c_p, _c_p, _c_p]),
     "f3d_dense_gemv_batched_f32": (ctypes.c_int, [_i64, _i32, _c_p, _c_p, _c_p, _c_p]),
+    "f3d_block_gemv_sum": (ctypes.c_int, [_i64, _i32, _i32, _c_p, _c_p, _c_p, _f64, _c_p]),
     "f3d_block_gemv_batched": (ctypes.c_int, [
         _i64, _i32, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _f64, _f64, _c_p]),
 }

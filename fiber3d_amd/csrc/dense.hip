@@ -822,8 +822,11 @@ lu_solve_kernel(const int* __restrict__ n_arr, const long* __restrict__ a_off,
 }
 
 // ---------------------------------------------------------------------------
-// y_b = alpha M_b x_b + beta y_b, M_b column-major m x k, m <= 64 kSlots: a
-// workgroup of four waves per block.  A lane has row lane of each 64-row
+// y_b = sum over terms of alpha M_b x_b, plus beta y_b; M_b column-major m x k, m
+// <= 64 kSlots: a workgroup of four waves per block, all terms in one launch
+// (a fiber's rows of the operator have four: A and the three Q_c; in launches
+// of their own these took 22 + 3 x 7.5 us for 1000 fibers of 32 nodes, here
+// 40.9, and 6 + 3 x 4.6 us for 32 fibers, here 9.2).  A lane has row lane of each 64-row
 // segment (R 64), or, for m <= 32, row lane % 32 of every other column (R 32).
 // The waves take groups of columns in turn, 16 loads of a lane in flight; the
 // four sums meet in LDS in a fixed order.
@@ -834,18 +837,21 @@ lu_solve_kernel(const int* __restrict__ n_arr, const long* __restrict__ a_off,
 // blocks of 128 x 128 6.1 us for 18, of 114 x 32 3.9 for 10.
 constexpr int kGemvThreads = 256;
 
+// acc += alpha M x for the lane's rows
 template <int R, int SL>
 __device__ __forceinline__ void block_gemv_cols(const double* __restrict__ M,
                                                 const double* __restrict__ x, int m, int kk,
-                                                int wv, int lane, double (&acc)[SL]) {
+                                                double alpha, int wv, int lane,
+                                                double (&acc)[SL]) {
   constexpr int C = 64 / R;    // columns side by side in a wave
   constexpr int U = 16 / SL;   // steps whose loads are in flight together
   const int sub = R == 64 ? 0 : lane / R;
   int row[SL];
+  double sum[SL];
 #pragma unroll
   for (int s = 0; s < SL; ++s) {
-    acc[s] = 0.0;
-    row[s] = min(lane % R + 64 * s, m - 1);  // (rows past m are not written)
+    sum[s] = 0.0;
+    row[s] = min(lane % R + 64 * s, m - 1);
   }
   for (int j0 = wv * (U * C); j0 < kk; j0 += 4 * U * C) {
     double v[U][SL], xv[U];
@@ -860,29 +866,45 @@ __device__ __forceinline__ void block_gemv_cols(const double* __restrict__ M,
     for (int u = 0; u < U; ++u) {
       const bool in = j0 + u * C + sub < kk;  // past the end: adds nothing
 #pragma unroll
-      for (int s = 0; s < SL; ++s) acc[s] = in ? fma(v[u][s], xv[u], acc[s]) : acc[s];
+      for (int s = 0; s < SL; ++s) sum[s] = in ? fma(v[u][s], xv[u], sum[s]) : sum[s];
     }
   }
-  if (R == 32) acc[0] += __shfl_xor(acc[0], 32, 64);
+#pragma unroll
+  for (int s = 0; s < SL; ++s)  // (a term may have fewer rows than the block)
+    acc[s] = lane % R + 64 * s < m ? fma(alpha, sum[s], acc[s]) : acc[s];
 }
 
-__global__ void __launch_bounds__(kGemvThreads)
-block_gemv_kernel(const int* __restrict__ m_arr, const int* __restrict__ k_arr,
-                  const long* __restrict__ m_off, const long* __restrict__ x_off,
-                  const long* __restrict__ y_off, const double* __restrict__ M,
-                  const double* __restrict__ x, double* __restrict__ y, double alpha,
-                  double beta) {
-  __shared__ double red[4][64 * kSlots];
+struct GemvTerms {
+  f3d_gemv_term t[F3D_GEMV_TERMS];
+};
+
+__global__ void __launch_bounds__(kGemvThreads * F3D_GEMV_TERMS)
+block_gemv_kernel(int terms, const GemvTerms tt, const long* __restrict__ y_off,
+                  double* __restrict__ y, double beta) {
+  __shared__ double red[4 * F3D_GEMV_TERMS][64 * kSlots];
   const int b = blockIdx.x;
-  const int t = threadIdx.x, lane = t & 63;
+  const int t = threadIdx.x, lane = t & 63, groups = blockDim.x / kGemvThreads;
   const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int m = m_arr[b], kk = k_arr[b];
-  if (m <= 0 || m > 64 * kSlots || kk < 0) return;
-  const double* __restrict__ Mb = M + m_off[b];
-  const double* __restrict__ xb = x + x_off[b];
+  int m = 0;  // rows of the block: of its tallest term
+  for (int q = 0; q < terms; ++q) {
+    const int mq = tt.t[q].m[b];
+    if (mq > 64 * kSlots || tt.t[q].k[b] < 0) return;
+    m = max(m, mq);
+  }
+  if (m <= 0) return;
   auto sums = [&](auto R, auto SL) __attribute__((always_inline)) {
     double acc[SL.value];
-    block_gemv_cols<R.value, SL.value>(Mb, xb, m, kk, wv, lane, acc);
+#pragma unroll
+    for (int s = 0; s < SL.value; ++s) acc[s] = 0.0;
+#pragma unroll 1
+    for (int q = wv / 4; q < terms; q += groups) {
+      const f3d_gemv_term& g = tt.t[q];
+      const int mq = g.m[b];
+      if (mq > 0)
+        block_gemv_cols<R.value, SL.value>(g.M + g.m_off[b], g.x + g.x_off[b], mq, g.k[b],
+                                           g.alpha, wv % 4, lane, acc);
+    }
+    if (R.value == 32) acc[0] += __shfl_xor(acc[0], 32, 64);
 #pragma unroll
     for (int s = 0; s < SL.value; ++s) red[wv][64 * s + lane] = acc[s];
   };
@@ -893,9 +915,11 @@ block_gemv_kernel(const int* __restrict__ m_arr, const int* __restrict__ k_arr,
   else sums(integral_constant<int, 64>{}, integral_constant<int, 4>{});
   __syncthreads();
   if (t >= m) return;
-  const double v = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
+  double v = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
+  for (int g = 1; g < groups; ++g)
+    v += (red[4 * g][t] + red[4 * g + 1][t]) + (red[4 * g + 2][t] + red[4 * g + 3][t]);
   double* __restrict__ yb = y + y_off[b];
-  yb[t] = beta == 0.0 ? alpha * v : fma(alpha, v, beta * yb[t]);
+  yb[t] = beta == 0.0 ? v : fma(beta, yb[t], v);
 }
 
 // ---------------------------------------------------------------------------
@@ -1146,14 +1170,32 @@ extern "C" int f3d_block_gemv_batched(int64_t nb, int32_t mmax, const int32_t* m
                                       const int64_t* x_off, const int64_t* y_off,
                                       const double* M, const double* x, double* y, double alpha,
                                       double beta, void* stream) {
+  const f3d_gemv_term term{m, k, m_off, x_off, M, x, alpha};
+  return f3d_block_gemv_sum(nb, mmax, 1, &term, y_off, y, beta, stream);
+}
+
+extern "C" int f3d_block_gemv_sum(int64_t nb, int32_t mmax, int32_t terms,
+                                  const f3d_gemv_term* term, const int64_t* y_off, double* y,
+                                  double beta, void* stream) {
   F3D_REQUIRE(nb >= 0 && nb < (1ll << 31), F3D_EINVAL, "block_gemv: bad batch count");
   F3D_REQUIRE(mmax >= 1 && mmax <= 64 * kSlots, F3D_EINVAL,
               "block_gemv: mmax=%d outside [1,%d]", mmax, 64 * kSlots);
+  F3D_REQUIRE(terms >= 1 && terms <= F3D_GEMV_TERMS && term, F3D_EINVAL,
+              "block_gemv: %d terms outside [1,%d]", terms, F3D_GEMV_TERMS);
   if (nb == 0) return F3D_OK;
-  F3D_REQUIRE(m && k && m_off && x_off && y_off && M && x && y, F3D_EINVAL,
-              "block_gemv: NULL argument");
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  F3D_LAUNCH(block_gemv_kernel, dim3((unsigned)nb), dim3(kGemvThreads), 0, st, m, k, (const long*)m_off,
-             (const long*)x_off, (const long*)y_off, M, x, y, alpha, beta);
+  F3D_REQUIRE(y && y_off, F3D_EINVAL, "block_gemv: NULL argument");
+  GemvTerms tt{};
+  for (int q = 0; q < terms; ++q) {
+    const f3d_gemv_term& g = term[q];
+    F3D_REQUIRE(g.m && g.k && g.m_off && g.x_off && g.M && g.x, F3D_EINVAL,
+                "block_gemv: NULL argument");
+    tt.t[q] = g;
+  }
+  // Four waves a term where the blocks leave CUs idle (32 blocks: 9.2 us for 12.8 with
+  // the terms one after the other); elsewhere four waves a block, since the
+  // waves of short terms would only hold their places (1000 blocks: 40.9 us for 48.2).
+  const int groups = nb <= num_cus() ? terms : 1;
+  F3D_LAUNCH(block_gemv_kernel, dim3((unsigned)nb), dim3(kGemvThreads * groups), 0,
+             reinterpret_cast<hipStream_t>(stream), terms, tt, (const long*)y_off, y, beta);
   return F3D_OK;
 }

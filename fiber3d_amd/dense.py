@@ -137,6 +137,21 @@ class BlockGemv:
             buf[o:o + M.size] = np.asarray(M, np.float64).T.ravel()
         return torch.from_numpy(buf).to(device())
 
+    @staticmethod
+    def sum(terms, y, beta=0.0):
+        """y_b = sum of alpha M_b x_b over terms (gemv, M, x, alpha), plus beta
+        y_b, in one launch; the first term's gemv has the rows of y and the
+        others no more."""
+        first = terms[0][0]
+        p = lambda t: t.data_ptr()
+        arr = (L.GemvTerm * len(terms))(*(
+            L.GemvTerm(p(g.m), p(g.k), p(g.m_off), p(g.x_off), p(M), p(x), float(alpha))
+            for g, M, x, alpha in terms))
+        rc = L.load().f3d_block_gemv_sum(first.nb, first.mmax, len(terms), arr,
+                                         L.ptr(first.y_off), L.ptr(y), float(beta), _stream())
+        L.check(rc, "f3d_block_gemv_sum")
+        return y
+
     def __call__(self, M, x, y, alpha=1.0, beta=0.0):
         rc = L.load().f3d_block_gemv_batched(
             self.nb, self.mmax, L.ptr(self.m), L.ptr(self.k), L.ptr(self.m_off), L.ptr(self.x_off),

@@ -920,9 +920,8 @@ class FiberSystem:
         if B is not None:
             B.rows(x, out, nper3)
         res = out[self.fib0:]
-        self.gA(self.A_buf, XT, res)
-        for c in range(3):
-            self.gQ[c](self.Q_buf[c], self.v_soa, res, alpha=-1.0, beta=1.0)
+        BlockGemv.sum([(self.gA, self.A_buf, XT, 1.0)]
+                      + [(self.gQ[c], self.Q_buf[c], self.v_soa, -1.0) for c in range(3)], res)
         if self.att:
             self._link_rows(x, out, vsoa)
         # minus ends clamped to the cortex: flow term of their tension

@@ -346,6 +346,25 @@ int f3d_block_gemv_batched(int64_t nb, int32_t mmax, const int32_t* m, const int
                            double beta, void* stream);
 
 /*
+ * y_b = sum over the terms of alpha * M_b x_b, plus beta * y_b: up to
+ * F3D_GEMV_TERMS products of the form above into the same rows in one launch.
+ * A term may have fewer rows than the block (the tallest term's); it then adds
+ * to the first m[b] of them.  No x may alias y.
+ */
+#define F3D_GEMV_TERMS 4
+typedef struct {
+  const int32_t* m;
+  const int32_t* k;
+  const int64_t* m_off;
+  const int64_t* x_off;
+  const double* M;
+  const double* x;
+  double alpha;
+} f3d_gemv_term;
+int f3d_block_gemv_sum(int64_t nb, int32_t mmax, int32_t terms, const f3d_gemv_term* term,
+                       const int64_t* y_off, double* y, double beta, void* stream);
+
+/*
  * y_b = M_b x_b for `count` dense ROW-major m x m FP64 matrices stored
  * back to back (M + b*m*m), x and y of length count*m (y must not alias x).
  * Applies the shell preconditioner's dense inverse, the same linear map as the

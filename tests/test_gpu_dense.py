@@ -209,6 +209,39 @@ def test_block_gemv_edges(beta):
         assert (np.abs(got[yo:yo + m] - ref) <= 260 * 2.3e-16 * scale + 1e-300).all(), (m, k)
 
 
+@pytest.mark.parametrize("beta", [0.0, -0.5])
+def test_block_gemv_sum(beta):
+    """Four products into the same rows, the later terms with fewer rows (none,
+    up to a segment's edge, all) than the block; tolerance as above."""
+    print(f"case block gemv sum beta={beta}", flush=True)
+    rng = np.random.default_rng(12)
+    ms = np.array([20, 32, 33, 64, 66, 128, 130, 256])
+    rows = [ms, np.maximum(ms - 14, 1), np.minimum(ms, 32), np.minimum(ms, 64)]
+    ks = [ms, np.array([5, 8, 8, 16, 17, 32, 33, 64]), ms, np.array([1, 0, 3, 260, 9, 15, 16, 7])]
+    alphas = [1.0, -1.0, 0.5, 2.0]
+    y_off = np.concatenate([[0], np.cumsum(ms)[:-1]])
+    terms, host = [], []
+    for m, k, a in zip(rows, ks, alphas):
+        mats = [rng.normal(size=(mb, kb)) for mb, kb in zip(m, k)]
+        x_off = np.concatenate([[0], np.cumsum(k)[:-1]])
+        x = rng.normal(size=int(k.sum()))
+        g = BlockGemv(m, k, x_off, y_off)
+        terms.append((g, g.pack(mats), torch.from_numpy(x).cuda(), a))
+        host.append((mats, x_off, x, a))
+    y0 = rng.normal(size=int(ms.sum()))
+    y = torch.from_numpy(y0.copy()).cuda()
+    BlockGemv.sum(terms, y, beta=beta)
+    got = y.cpu().numpy()
+    for b, (m, yo) in enumerate(zip(ms, y_off)):
+        ref, scale = beta * y0[yo:yo + m], np.abs(beta * y0[yo:yo + m])
+        for mats, x_off, x, a in host:
+            M = mats[b]
+            xb = x[x_off[b]:x_off[b] + M.shape[1]]
+            ref[:M.shape[0]] += a * (M @ xb)
+            scale[:M.shape[0]] += np.abs(a) * (np.abs(M) @ np.abs(xb))
+        assert (np.abs(got[yo:yo + m] - ref) <= 2 * 260 * 2.3e-16 * scale).all(), b
+
+
 def test_batched_lu_on_real_fiber_blocks_config2_shape():
     """Workload 2 shape: fibers with N in {16, 24, 32, 48, 64} (n = 4N up to
     256), A_sq assembled from the fiber discretisation; FP32 LU + FP64
