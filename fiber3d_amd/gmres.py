@@ -54,12 +54,13 @@ applied to the combination rather than to each basis vector.
 `measure_inner=True` returns the largest such difference relative to ||H y||
 as `inner_err`, the quantity `inner_rel_err` must bound.
 """
-import ctypes
 import math
 from dataclasses import dataclass
 
 import numpy as np
 import torch
+
+from .kernels import _stream
 
 
 @dataclass
@@ -140,21 +141,18 @@ class GmresContext:
     def reset(self):
         self.graphs = {}
 
-    def _stream(self):
-        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-
     def begin(self, r):
         L = self.L
         L.check(L.load().f3d_gmres_begin(self.n, self.m, L.ptr(r), L.ptr(self.V), L.ptr(self.ws),
-                                         self._stream()), "f3d_gmres_begin")
+                                         _stream()), "f3d_gmres_begin")
 
     def _step_eager(self, op):
         L, lib = self.L, self.L.load()
         L.check(lib.f3d_gmres_current(self.n, self.m, L.ptr(self.V), L.ptr(self.xin),
-                                      L.ptr(self.ws), self._stream()), "f3d_gmres_current")
+                                      L.ptr(self.ws), _stream()), "f3d_gmres_current")
         op(self.xin, self.w)
         L.check(lib.f3d_gmres_arnoldi(self.n, self.m, L.ptr(self.V), L.ptr(self.w),
-                                      L.ptr(self.ws), self._stream()), "f3d_gmres_arnoldi")
+                                      L.ptr(self.ws), _stream()), "f3d_gmres_arnoldi")
 
     def step(self, op, key=None):
         """One Arnoldi step with op(x, out) = A P^-1 x; replayed from a
@@ -198,7 +196,7 @@ class GmresContext:
         L = self.L
         L.check(L.load().f3d_gmres_solve(self.n, self.m, int(k), L.ptr(self.V), L.ptr(self.upd),
                                          L.ptr(r), L.ptr(self.r_upd if r is not None else None),
-                                         L.ptr(self.ws), self._stream()), "f3d_gmres_solve")
+                                         L.ptr(self.ws), _stream()), "f3d_gmres_solve")
         return self.upd
 
 
