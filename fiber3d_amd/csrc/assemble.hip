@@ -43,6 +43,8 @@
 // 0.51 ms less, without the matrix instructions the same.
 #include "common.h"
 
+#include <algorithm>
+
 namespace f3d {
 
 constexpr int kAsmNmax = 64;
@@ -66,13 +68,14 @@ __device__ __forceinline__ void swap_rows(double& x, double& y) {
 }
 
 // xs, xss, xsss = D_1 X, D_2 X, D_3 X of every fiber and its weights: a lane per
-// (fiber, component) with the coordinates in registers, kDerivRows rows of D
-// per wave, whose entries are wave-uniform (scalar loads).  xsss goes to the
+// (fiber, component) with the coordinates in registers, up to kDerivRows rows of
+// D per wave (one where few fibers leave CUs idle: 25 us with 8, 5 with one for 32
+// fibers of 32 nodes), whose entries are wave-uniform (scalar loads).  xsss goes to the
 // start of the fiber's force rows, which are written last.
 constexpr int kDerivRows = 8;
 template <int NMAX>
 __global__ void __launch_bounds__(64)
-fiber_deriv_kernel(int nfib, int N, const long* __restrict__ node0,
+fiber_deriv_kernel(int nfib, int N, int rows, const long* __restrict__ node0,
                    const double* __restrict__ length, const long* __restrict__ f_off,
                    const double* __restrict__ X, const double* __restrict__ D0,
                    const double* __restrict__ w0, double* __restrict__ xs,
@@ -86,7 +89,7 @@ fiber_deriv_kernel(int nfib, int N, const long* __restrict__ node0,
   double x[NMAX];
 #pragma unroll
   for (int q = 0; q < NMAX; ++q) x[q] = X[(nd + min(q, N - 1)) * 3 + c];
-  const int k0 = blockIdx.y * kDerivRows, k1 = min(k0 + kDerivRows, N);
+  const int k0 = blockIdx.y * rows, k1 = min(k0 + rows, N);
   for (int k = k0; k < k1; ++k) {
     const double* __restrict__ d = D0 + k * N;
     double e1 = 0.0, e2 = 0.0, e3 = 0.0;
@@ -135,6 +138,7 @@ fiber_assemble_kernel(int nfib, int N, const long* __restrict__ node0,
   const int t = threadIdx.x, lane = t & 63;
   const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
   const int g = lane >> 4, c16 = lane & 15;
+  const int part = blockIdx.y, parts = gridDim.y;
   const int nx = N - 4, nt = N - 2, n4 = 4 * N, nq = n4 - 14;
   const int NN = N * N;
   for (int e = t; e < NMAX * NMAX; e += kAsmThreads) {
@@ -157,14 +161,13 @@ fiber_assemble_kernel(int nfib, int N, const long* __restrict__ node0,
   // the tile's rows of D_1 .. D_4: steps lo .. lo + ks - 1 hold its non-zeros
   // and the diagonal
   int lo = KS, hi = 0;
+#pragma unroll 4
   for (int st = 0; st < KS; ++st) {
     const int k = 4 * st + g;
-    bool any = false;
-    if (k < N && jj < N) {
-      any = k == jj;
-#pragma unroll
-      for (int d = 0; d < 4; ++d) any = any || D0[d * NN + k * N + jj] != 0.0;
-    }
+    const bool in = k < N && jj < N;
+    const double* __restrict__ d = D0 + (in ? k * N + jj : 0);
+    const double e1 = d[0], e2 = d[NN], e3 = d[2 * NN], e4 = d[3 * NN];
+    const bool any = in & ((k == jj) | (e1 != 0.0) | (e2 != 0.0) | (e3 != 0.0) | (e4 != 0.0));
     if (__ballot(any) != 0ull) {
       lo = min(lo, st);
       hi = st + 1;
@@ -211,7 +214,7 @@ fiber_assemble_kernel(int nfib, int N, const long* __restrict__ node0,
     double* __restrict__ Af = Aout + a_off[f];
     // ---- projected products: p = 4 a + b < 16 is block (a, b) of A_sq's
     // projected rows; p = 16 + c is the tension part of Q_c.
-    for (int p = first; p < 19; p += share) {
+    for (int p = first + share * part; p < 19; p += share * parts) {
       const int a = p < 16 ? p & 3 : 4 + (p - 16), b = p < 16 ? p >> 2 : 0;
       const bool tens = a >= 3;
       const int rows = tens ? nt : nx;
@@ -309,7 +312,7 @@ fiber_assemble_kernel(int nfib, int N, const long* __restrict__ node0,
 
     // ---- 14 boundary rows of every column (force- and torque-free ends):
     // four columns per wave, a lane per row
-    for (int j0 = 4 * wv; j0 < n4; j0 += 16) {
+    for (int j0 = 4 * (wv + 4 * part); j0 < n4; j0 += 16 * parts) {
       const int j = j0 + g, r = c16;
       if (j < n4 && r < 14) {
         const int b = (j >= N) + (j >= 2 * N) + (j >= 3 * N), jb = j - b * N;
@@ -334,7 +337,7 @@ fiber_assemble_kernel(int nfib, int N, const long* __restrict__ node0,
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       double* __restrict__ Q = (c == 0 ? Q0 : (c == 1 ? Q1 : Q2)) + q_off[3 * f + c];
-      for (int j = wv; j < N; j += 4) {
+      for (int j = wv + 4 * part; j < N; j += 4 * parts) {
 #pragma unroll
         for (int b = 0; b < 3; ++b)
           if (lane < nx) Q[j * nq + b * nx + lane] = b == c ? sPX[j * NMAX + lane] : 0.0;
@@ -529,12 +532,16 @@ extern "C" int f3d_fiber_assemble(int64_t nfib, int32_t N, const int64_t* node0,
   const int64_t most = 2 * (int64_t)num_cus();
   const unsigned grid = (unsigned)(nfib < most ? nfib : most);
   const unsigned fgrid = (unsigned)(nfib < 4 * most ? nfib : 4 * most);
-  const dim3 dgrid((unsigned)ceil_div(3 * nfib, 64), (unsigned)ceil_div(N, kDerivRows));
+  const int64_t dwaves = ceil_div(3 * nfib, (int64_t)64);
+  const int rows = (int)std::min<int64_t>(kDerivRows, ceil_div(dwaves * N, 2 * most));
+  const dim3 dgrid((unsigned)dwaves, (unsigned)ceil_div(N, rows));
+  // few fibers: several workgroups share one, by products and columns
+  const unsigned parts = nfib * 4 <= most ? 4 : (nfib * 2 <= most ? 2 : 1);
 #define F3D_ASM(NM)                                                                             \
-  F3D_LAUNCH(fiber_deriv_kernel<NM>, dgrid, dim3(64), 0, st, (int)nfib, (int)N,                 \
+  F3D_LAUNCH(fiber_deriv_kernel<NM>, dgrid, dim3(64), 0, st, (int)nfib, (int)N, rows,           \
              (const long*)node0, length, (const long*)f_off, X, D0, w0, xs_out, xss_out, w_out, \
              F_out);                                                                            \
-  F3D_LAUNCH(fiber_assemble_kernel<NM>, dim3(grid), dim3(kAsmThreads), 0, st, (int)nfib, (int)N, \
+  F3D_LAUNCH(fiber_assemble_kernel<NM>, dim3(grid, parts), dim3(kAsmThreads), 0, st, (int)nfib, (int)N, \
              (const long*)node0, length, (const long*)a_off, (const long*)f_off,                \
              (const long*)q_off, (const double*)xs_out, (const double*)xss_out,                 \
              (const double*)F_out, D0, PX, PT, E, dt, c0, c1, penalty, A_out, Q0, Q1, Q2);      \

@@ -199,7 +199,8 @@ def test_hip_assembly_matches_torch_assembly(N):
 @pytest.mark.parametrize("N,nfib,dense", [(12, 7, False), (16, 3, False), (17, 5, True),
                                           (31, 5, False), (32, 9, True), (33, 3, False),
                                           (47, 3, True), (48, 2, False), (49, 3, True),
-                                          (63, 2, False), (64, 3, True), (20, 1101, False)])
+                                          (63, 2, False), (64, 3, True), (20, 1101, False),
+                                          (24, 200, False)])
 def test_hip_assembly_at_tile_edges(N, nfib, dense):
     """Assembly and right-hand side at the edges of the 16-column tiles and of
     the two kernel sizes, with more fibers than workgroups, and with derivative
