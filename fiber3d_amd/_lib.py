@@ -114,6 +114,7 @@ SIGNATURES = {
     "f3d_gmres_solve": (ctypes.c_int, [_i64, _i32, _i32, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p]),
     "f3d_dense_gemv_batched": (ctypes.c_int, [_i64, _i32, _c_p, _c_p, _c_p, _c_p]),
     "f3d_dense_gemv_batched_f32": (ctypes.c_int, [_i64, _i32, _c_p, _c_p, _c_p, _c_p]),
+    "f3d_fiber_ends": (ctypes.c_int, [_i64] + [_c_p] * 4 + [_f64] + [_c_p] * 5),
     "f3d_block_gemv_sum": (ctypes.c_int, [_i64, _i32, _i32, _c_p, _c_p, _c_p, _f64, _c_p]),
     "f3d_block_gemv_batched": (ctypes.c_int, [
         _i64, _i32, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _f64, _f64, _c_p]),

@@ -507,6 +507,29 @@ fiber_rhs_kernel(int nfib, int N, const long* __restrict__ node0,
   }
 }
 
+// ---------------------------------------------------------------------------
+// Plus-end forces F_end x_s(L): the force at every node (zero but at the ends),
+// and the ends' positions, forces and weights as compact arrays for the explicit
+// flows.  A wave per fiber.  Seven gathers and fills of a few KB, 5 us each, in
+// one launch.
+__global__ void __launch_bounds__(64)
+fiber_end_kernel(const long* __restrict__ end_idx, const double* __restrict__ X,
+                 const double* __restrict__ xs, const double* __restrict__ w, double end_force,
+                 double* __restrict__ force, double* __restrict__ Xe, double* __restrict__ fe,
+                 double* __restrict__ we) {
+  const int f = blockIdx.x;
+  const long last = end_idx[f], first = f ? end_idx[f - 1] + 1 : 0;
+  for (long e = first * 3 + threadIdx.x; e < last * 3; e += 64) force[e] = 0.0;
+  if (threadIdx.x < 3) {
+    const int c = threadIdx.x;
+    const double v = end_force * xs[last * 3 + c];
+    force[last * 3 + c] = v;
+    fe[f * 3l + c] = v;
+    Xe[f * 3l + c] = X[last * 3 + c];
+    if (c == 0) we[f] = w[last];
+  }
+}
+
 }  // namespace f3d
 
 using namespace f3d;
@@ -583,5 +606,18 @@ extern "C" int f3d_fiber_rhs(int64_t nfib, int32_t N, const int64_t* node0, cons
     F3D_RHS(64);
   }
 #undef F3D_RHS
+  return F3D_OK;
+}
+
+extern "C" int f3d_fiber_ends(int64_t nfib, const int64_t* end_idx, const double* X,
+                              const double* xs, const double* w, double end_force, double* force,
+                              double* Xe, double* fe, double* we, void* stream) {
+  F3D_REQUIRE(nfib >= 0 && nfib < (1ll << 31), F3D_EINVAL, "fiber_ends: bad fiber count");
+  if (nfib == 0) return F3D_OK;
+  F3D_REQUIRE(end_idx && X && xs && w && force && Xe && fe && we, F3D_EINVAL,
+              "fiber_ends: NULL argument");
+  F3D_LAUNCH(fiber_end_kernel, dim3((unsigned)nfib), dim3(64), 0,
+             reinterpret_cast<hipStream_t>(stream), (const long*)end_idx, X, xs, w, end_force,
+             force, Xe, fe, we);
   return F3D_OK;
 }

@@ -812,11 +812,21 @@ class FiberSystem:
         # explicit force: plus end along the end tangent.  Only the end nodes
         # carry force, so only they are sources of the explicit flows (the
         # zero-force nodes add exact zeros to the reference's all-node sums).
-        force = torch.zeros((self.npts, 3), dtype=torch.float64, device=dev)
         last = self.end_idx
-        force[last] = self.end_force * self.xs[last]
+        if self.assembly == "hip":
+            force = torch.empty((self.npts, 3), dtype=torch.float64, device=dev)
+            Xe, fe = (torch.empty((self.nfib, 3), dtype=torch.float64, device=dev)
+                      for _ in range(2))
+            we = torch.empty(self.nfib, dtype=torch.float64, device=dev)
+            rc = L.load().f3d_fiber_ends(
+                self.nfib, L.ptr(last), L.ptr(self.X), L.ptr(self.xs), L.ptr(self.weights),
+                float(self.end_force), L.ptr(force), L.ptr(Xe), L.ptr(fe), L.ptr(we), _stream())
+            L.check(rc, "f3d_fiber_ends")
+        else:
+            force = torch.zeros((self.npts, 3), dtype=torch.float64, device=dev)
+            force[last] = self.end_force * self.xs[last]
+            Xe, fe, we = self.X[last], force[last], self.weights[last]
         self.force = force
-        Xe, fe, we = self.X[last], force[last], self.weights[last]
         pp = self.pair_precision_rhs = "f64"
         vff = pairsum("oseen", Xe, fe, self.X, src_w=we, excl=self.excl_end,
                       eta=self.eta, reg=self.reg, eps=self.eps, precision=pp)
@@ -835,7 +845,7 @@ class FiberSystem:
                           eta=self.eta, reg=self.reg, eps=self.eps, precision=pp)
             if B is not None:
                 B.explicit(self.shell.pos, out=vfs, accumulate=True)
-            rhs[:3 * self.nper] = -vfs.reshape(-1)
+            torch.neg(vfs.reshape(-1), out=rhs[:3 * self.nper])
         dt, c0, c1, p = self.dt, self.c0, self.c1, self.penalty
         if self.assembly == "hip":
             # fused per-fiber RHS rows, one launch per node count

@@ -332,6 +332,17 @@ int f3d_fiber_rhs(int64_t nfib, int32_t N, const int64_t* node0, const double* l
                   double* rhs, void* stream);
 
 /*
+ * Plus-end forces end_force * x_s(L) of nfib fibers whose nodes lie one fiber
+ * after another, end_idx[f] the last node of fiber f: force (npts x 3, AoS,
+ * zero except at the ends), and per fiber the end's position Xe, force fe (nfib
+ * x 3) and weight we, the sources of the explicit flows of
+ * python/tstep/tstep.py:794-846.
+ */
+int f3d_fiber_ends(int64_t nfib, const int64_t* end_idx, const double* X, const double* xs,
+                   const double* w, double end_force, double* force, double* Xe, double* fe,
+                   double* we, void* stream);
+
+/*
  * y_b = alpha * M_b x_b + beta * y_b for a batch of dense COLUMN-major blocks
  * of shape m[b] x k[b] (leading dimension m[b]) stored at M + m_off[b]; x at
  * x_off[b], y at y_off[b] (y must not alias x).  m[b] <= mmax <= 1024.
