@@ -2,9 +2,13 @@
 and the BF16 GEMM.
 
 Pair sums: for each (kernel, precision) and each tuned problem size
-(n_targets, n_sources) of a grid of powers of two, it times f3d_pairsum over
-the launch shapes -- targets per lane K in {1, 2, 4} and the wavefront count
-the source split aims for -- and keeps the fastest.  apply() installs the
+(n_targets, n_sources) of a grid of powers of two, it times f3d_pairsum (there
+and at three quarters of it) over the launch shapes -- targets per lane K in
+{1, 2, 4} and the wavefront count the source split aims for -- and keeps the
+fastest.  FP32C sums depend on their shape at the 1e-8 level (K groups the
+targets of the near/far test, the split the compensated partial sums): the saved
+table holds FP32C shapes that were tuned on powers of four only, and sizes in
+between (the entries without a rate) take the nearest of those.  apply() installs the
 fastest shape of the nearest tuned size (in log2 n_targets + log2 n_sources)
 into every size bucket of the library (f3d_pairsum_set_launch_bucket), and
 the 65536 x 65536 shape as the (kernel, precision) default.  The large
@@ -34,8 +38,8 @@ PRECS = {"f64": L.F64, "f32c": L.F32C}
 LG_MIN, LG_MAX = 8, 22          # size buckets of the library (log2 sizes)
 KS = (1, 2, 4)
 WAVES = (2048, 4096, 8192, 16384, 32768)
-GRID_NT = (4096, 16384, 65536)
-GRID_NS = (1024, 4096, 16384, 65536)
+GRID_NT = (4096, 8192, 16384, 32768, 65536, 262144)
+GRID_NS = (1024, 2048, 4096, 8192, 16384, 32768, 65536)
 LU_WAVES = {"f64": (1, 2, 4), "f32c": (2, 4, 8)}
 
 
@@ -136,6 +140,32 @@ def apply(path=CACHE, table=None):
     return table
 
 
+def _time_queued(fn, reps, replays=3):
+    """Seconds per call of fn on the device: `reps` calls in one recorded graph,
+    the fastest of `replays` (host work does not count, nor do the launches
+    of calls that follow each other)."""
+    import torch
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        fn()
+        stream.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=stream):
+            for _ in range(reps):
+                fn()
+    g.replay()
+    a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    best = None
+    for _ in range(replays):
+        a.record()
+        g.replay()
+        b.record()
+        b.synchronize()
+        t = a.elapsed_time(b) * 1e-3 / reps
+        best = t if best is None else min(best, t)
+    return best
+
+
 def _time(fn, min_s=0.02, max_reps=200):
     """Seconds per call: one untimed call, then enough calls for ~min_s."""
     import torch
@@ -177,10 +207,16 @@ def tune_pairsum(kernels=("oseen", "stresslet", "rotlet"), precisions=("f32c", "
                     for k in ks:
                         for w in waves:
                             set_launch_bucket(kernel, precision, lg(nt), lg(ns), k, w)
-                            kw = dict(src_nrm=NR[:ns] if kernel == "stresslet" else None,
-                                      precision=precision, out=out[:nt])
-                            t = _time(lambda: pairsum(kernel, X[:ns], F[:ns], X[:nt], **kw))
-                            rate = nt * ns / t / 1e9
+                            t = pairs = 0.0
+                            # the bucket's largest sizes and three quarters of them
+                            for t_, s_ in ((nt, ns), (3 * nt // 4, 3 * ns // 4)):
+                                kw = dict(src_nrm=NR[:s_] if kernel == "stresslet" else None,
+                                          precision=precision, out=out[:t_])
+                                reps = max(1, min(10, int(2e9 / (t_ * s_))))
+                                t += _time_queued(
+                                    lambda: pairsum(kernel, X[:s_], F[:s_], X[:t_], **kw), reps)
+                                pairs += t_ * s_
+                            rate = pairs / t / 1e9
                             if best is None or rate > best[0]:
                                 best = (rate, k, w)
                     set_launch_bucket(kernel, precision, lg(nt), lg(ns), best[1], best[2])
