@@ -58,48 +58,51 @@ struct TileOperand {
 // KC (K contiguous): row tid / 4, 16 consecutive k.  Otherwise (rows
 // contiguous): two items of two k and four rows each.
 template <bool KC>
-__device__ __forceinline__ void tile_load(const TileOperand& o, bool vec, int r0, int k0, int kend,
-                                          float (&v)[16]) {
+__device__ __forceinline__ void tile_place(int w, int& r, int& k) {
   const int tid = threadIdx.x;
   if constexpr (KC) {
-    const int r = r0 + (tid >> 2), k = k0 + 16 * (tid & 3);
-    const float* __restrict__ p = o.p + (long)min(r, o.R - 1) * o.sr + (long)k * o.sk;
-    const bool in = r < o.R;
-    if (vec && in && k + 16 <= kend) {
+    r = tid >> 2;
+    k = 16 * (tid & 3) + w;
+  } else {
+    const int item = tid + 256 * (w >> 3);
+    r = 4 * (item & 15) + (w & 3);
+    k = 2 * (item >> 4) + ((w >> 2) & 1);
+  }
+}
+
+// A chunk inside the operand takes float4 loads; at its edges, and where rows are
+// not aligned, every value has a clamped load of its own, all sixteen in flight
+// (a branch per value, or per quad, made the compiler wait inside), and
+// tile_mask drops what lies outside when the chunk is used.
+template <bool KC>
+__device__ __forceinline__ void tile_load(const TileOperand& o, bool whole, int r0, int k0,
+                                          int kend, float (&v)[16]) {
+  int r, k;
+  if (whole) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float4 f = reinterpret_cast<const float4*>(p)[q];
-        v[4 * q] = f.x; v[4 * q + 1] = f.y; v[4 * q + 2] = f.z; v[4 * q + 3] = f.w;
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 16; ++i) v[i] = in && k + i < kend ? p[(long)i * o.sk] : 0.0f;
+    for (int q = 0; q < 4; ++q) {
+      tile_place<KC>(4 * q, r, k);
+      const float4 f = *reinterpret_cast<const float4*>(o.p + (r0 + r) * o.sr + (k0 + k) * o.sk);
+      v[4 * q] = f.x; v[4 * q + 1] = f.y; v[4 * q + 2] = f.z; v[4 * q + 3] = f.w;
     }
   } else {
 #pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      const int item = tid + 256 * e;
-      const int r = r0 + 4 * (item & 15), k = k0 + 2 * (item >> 4);
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int w = 8 * e + 4 * h;
-        const float* __restrict__ p = o.p + (long)min(k + h, kend - 1) * o.sk + (long)r * o.sr;
-        const bool in = k + h < kend;
-        float4 f;
-        if (vec && in && r + 4 <= o.R) {
-          f = *reinterpret_cast<const float4*>(p);
-        } else {
-          f.x = in && r < o.R ? p[0] : 0.0f;
-          f.y = in && r + 1 < o.R ? p[o.sr] : 0.0f;
-          f.z = in && r + 2 < o.R ? p[2 * o.sr] : 0.0f;
-          f.w = in && r + 3 < o.R ? p[3 * o.sr] : 0.0f;
-        }
-        v[w] = f.x;
-        v[w + 1] = f.y;
-        v[w + 2] = f.z;
-        v[w + 3] = f.w;
-      }
+    for (int w = 0; w < 16; ++w) {
+      tile_place<KC>(w, r, k);
+      v[w] = o.p[min(r0 + r, o.R - 1) * o.sr + min(k0 + k, kend - 1) * o.sk];
     }
+  }
+}
+
+template <bool KC>
+__device__ __forceinline__ void tile_mask(const TileOperand& o, bool whole, int r0, int k0,
+                                          int kend, float (&v)[16]) {
+  if (whole) return;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) {
+    int r, k;
+    tile_place<KC>(w, r, k);
+    v[w] = r0 + r < o.R && k0 + k < kend ? v[w] : 0.0f;
   }
 }
 
@@ -151,11 +154,16 @@ __device__ __forceinline__ f32x16_t tile_product(TileShared& sh, const TileOpera
 #pragma unroll
   for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
   float ra[16], rb[16];
+  const bool wa = va && m0 + kMT <= A.R, wb = vb && n0 + kNT <= B.R;
   auto load = [&](int k0) __attribute__((always_inline)) {
-    tile_load<AKC>(A, va, m0, k0, kend, ra);
-    tile_load<BKC>(B, vb, n0, k0, kend, rb);
+    const bool in = k0 + kKT <= kend;
+    tile_load<AKC>(A, wa && in, m0, k0, kend, ra);
+    tile_load<BKC>(B, wb && in, n0, k0, kend, rb);
   };
-  auto store = [&](int buf) __attribute__((always_inline)) {
+  auto store = [&](int buf, int k0) __attribute__((always_inline)) {
+    const bool in = k0 + kKT <= kend;
+    tile_mask<AKC>(A, wa && in, m0, k0, kend, ra);
+    tile_mask<BKC>(B, wb && in, n0, k0, kend, rb);
     tile_store<AKC>(sh.a[buf], ra);
     tile_store<BKC>(sh.b[buf], rb);
     if constexpr (SUM) {
@@ -164,25 +172,28 @@ __device__ __forceinline__ f32x16_t tile_product(TileShared& sh, const TileOpera
     }
   };
   if (kbeg >= kend) return acc;
-  load(kbeg);
-  store(0);
-  __syncthreads();
-  int buf = 0;
-  for (int k0 = kbeg; k0 < kend; k0 += kKT, buf ^= 1) {
+  // One copy of the loads and of the stores: the first pass of the loop has no
+  // product yet.  (A kernel's instructions are fetched from L2 when it starts,
+  // and short products run them about once.)
+  const int row = 32 * wm + (lane & 31), col = 32 * wn + (lane & 31);
+  int buf = 1;
+#pragma unroll 1
+  for (int k0 = kbeg - kKT; k0 < kend; k0 += kKT, buf ^= 1) {
     const bool more = k0 + kKT < kend;
     if (more) load(k0 + kKT);  // in flight during the MFMAs
-    const int row = 32 * wm + (lane & 31), col = 32 * wn + (lane & 31);
+    if (k0 >= kbeg) {
 #pragma unroll
-    for (int ks = 0; ks < kKT; ks += 16) {
-      const int kofs = ks + 8 * (lane >> 5);
-      const bf16x8_t a =
-          __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(&sh.a[buf][row][kofs]));
-      const bf16x8_t b =
-          __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(&sh.b[buf][col][kofs]));
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+      for (int ks = 0; ks < kKT; ks += 16) {
+        const int kofs = ks + 8 * (lane >> 5);
+        const bf16x8_t a =
+            __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(&sh.a[buf][row][kofs]));
+        const bf16x8_t b =
+            __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(&sh.b[buf][col][kofs]));
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
+      }
     }
-    if (more) store(buf ^ 1);
-    __syncthreads();
+    if (more) store(buf ^ 1, k0 + kKT);
+    lds_barrier();
   }
   return acc;
 }
@@ -196,29 +207,46 @@ gemm_bf16_kernel(TileOperand A, TileOperand B, int K, int kchunk, float* __restr
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int m0 = blockIdx.y * kMT, n0 = blockIdx.x * kNT;
   const int kbeg = blockIdx.z * kchunk;
-  float unused[4];
-  const f32x16_t acc =
-      tile_product<AKC, BKC, false>(sh, A, B, m0, n0, kbeg, min(K, kbeg + kchunk), unused);
   // C layout of the 32 x 32 MFMA: register i of lane l holds
   // row 8*(i/4) + 4*(l/32) + i%4, column l%32.
   const int n = n0 + 32 * (wave & 1) + (lane & 31);
+  const int mb = m0 + 32 * (wave >> 1) + 4 * (lane >> 5);
+  // What the epilogue reads comes before the product: read row by row among its
+  // stores, each value waited for the stores of the row before (9 us, of the 10
+  // that a small layer took).
+  float bn = 0.0f, z[16];
+  if (EPI == EPI_BIAS_RELU || EPI == EPI_BIAS) {
+    if (bias) bn = bias[min(n, B.R - 1)];
+  }
+  if (EPI == EPI_RELU_GRAD) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int m = mb + 8 * (i >> 2) + (i & 3);
+      z[i] = Zin[(long)min(m, A.R - 1) * scm + (long)min(n, B.R - 1) * scn];
+    }
+  }
+  float unused[4];
+  const f32x16_t acc =
+      tile_product<AKC, BKC, false>(sh, A, B, m0, n0, kbeg, min(K, kbeg + kchunk), unused);
+  if (n >= B.R) return;
+  const long c0 = (long)mb * scm + (long)n * scn;
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
-    const int m = m0 + 32 * (wave >> 1) + 8 * (i >> 2) + 4 * (lane >> 5) + (i & 3);
-    if (m >= A.R || n >= B.R) continue;
+    const int q = 8 * (i >> 2) + (i & 3);
+    if (mb + q >= A.R) break;  // (rows rise with i)
     float v = alpha * acc[i];
-    const long ci = (long)m * scm + (long)n * scn;
+    const long ci = c0 + q * scm;
     if (EPI == EPI_ATOMIC) {
       atomicAdd(&C[ci], v);
     } else if (EPI == EPI_BIAS_RELU || EPI == EPI_BIAS) {
-      if (bias) v += bias[n];
+      if (bias) v += bn;
       if (EPI == EPI_BIAS_RELU) {
         if (Z) Z[ci] = v;
         v = v > 0.0f ? v : 0.0f;
       }
       C[ci] = v;
     } else if (EPI == EPI_RELU_GRAD) {
-      C[ci] = Zin[ci] > 0.0f ? v : 0.0f;
+      C[ci] = z[i] > 0.0f ? v : 0.0f;
     } else {
       C[ci] = v;
     }
@@ -662,8 +690,9 @@ extern "C" int f3d_gemm_bf16(int epi, int64_t M, int64_t N, int64_t K, int32_t k
   // the streaming paths: row-major A (unit K stride) and C (unit N stride),
   // N in {128, 256}, 16 < K <= 256, no K split, from kStreamRows rows on.
   // Fewer rows leave CUs idle or pay B's set-up for a block or two: at 256 x
-  // 256, 8192 rows take 15 us tiled, 26 streaming, 39 resident; 32768 rows 39,
-  // 33, 47; 65536 rows 73, 61, 55; 262144 rows 288, 253, 130.  (At K = 4 the
+  // 256, 8192 rows take 12 us tiled, 26 streaming, 39 resident; 32768 rows 32,
+  // 33, 47; 49152 rows 50 tiled, 50 resident; 65536 rows 73, 61, 55; 262144 rows
+  // 288, 253, 130.  (At K = 4 the
   // tiled kernel is the fastest at every size: 174 against 220 us at 262144.)
   const int mode = (N == 128 || N == 256) ? g_gemm_stream[N == 256 ? 1 : 0] : 0;
   const bool stream_ok = epi != EPI_ATOMIC && ksplit == 1 && sak == 1 && scn == 1 && mode > 0 &&
