@@ -333,14 +333,18 @@ fiber_assemble_kernel(int nfib, int N, const long* __restrict__ node0,
         Af[(long)j * n4 + (n4 - 14) + r] = v;
       }
     }
-    // ---- identity part of Q_c: rows [0, 3 nx), P_X in row block c --------
+    // ---- identity part of Q_c: rows [0, 3 nx), P_X in row block c (streamed past
+    // L2, like the force rows: 41 and 27 us of 4096 fibers x 64; the products are
+    // not, their pieces of lines meet in L2: +140 us) --------
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       double* __restrict__ Q = (c == 0 ? Q0 : (c == 1 ? Q1 : Q2)) + q_off[3 * f + c];
       for (int j = wv + 4 * part; j < N; j += 4 * parts) {
 #pragma unroll
         for (int b = 0; b < 3; ++b)
-          if (lane < nx) Q[j * nq + b * nx + lane] = b == c ? sPX[j * NMAX + lane] : 0.0;
+          if (lane < nx)
+            __builtin_nontemporal_store(b == c ? sPX[j * NMAX + lane] : 0.0,
+                                        &Q[j * nq + b * nx + lane]);
       }
     }
   }
@@ -391,8 +395,9 @@ fiber_force_kernel(int nfib, int N, const long* __restrict__ node0,
       for (int a = 0; a < 3; ++a) {
         double* __restrict__ Fa = Fb + a * (4 * N * N) + j * N;
 #pragma unroll
-        for (int b = 0; b < 3; ++b) Fa[b * (N * N)] = b == a ? v4 : 0.0;
-        Fa[3 * (N * N)] = xa[a] * c1[q] + (i == j ? xxa[a] : 0.0);
+        for (int b = 0; b < 3; ++b)
+          __builtin_nontemporal_store(b == a ? v4 : 0.0, &Fa[b * (N * N)]);
+        __builtin_nontemporal_store(xa[a] * c1[q] + (i == j ? xxa[a] : 0.0), &Fa[3 * (N * N)]);
       }
     }
   }
