@@ -874,7 +874,7 @@ extern "C" int f3d_mlp_forward(int64_t M, int32_t n_in, int32_t width, int32_t n
                                const float* b3, float* H1, float* H2, float* Y, void* stream) {
   F3D_REQUIRE(M >= 0 && n_in >= 1 && width >= 1 && n_out >= 1, F3D_EINVAL, "mlp_forward: bad sizes");
   if (M == 0) return F3D_OK;
-  F3D_REQUIRE(X && W1 && b1 && W2 && b2 && W3 && b3 && H1 && H2 && Y, F3D_EINVAL,
+  F3D_REQUIRE(X && W1 && W2 && W3 && H1 && H2 && Y, F3D_EINVAL,
               "mlp_forward: NULL argument");
   int rc = f3d_gemm_bf16(EPI_BIAS_RELU, M, width, n_in, 1, X, sxm, sxk, W1, width, 1, H1, width, 1,
                          b1, nullptr, nullptr, 1.0f, stream);

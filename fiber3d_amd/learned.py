@@ -63,18 +63,35 @@ class MLP:
         self.v = [torch.zeros_like(p) for p in self.params]
         self.t = 0
         self.n_in, self.n_out, self.width = n_in, n_out, width
+        self.shapes = [(n_in, width), (width, width), (width, n_out)]
+
+    def _weight(self, k):
+        """Weight k as the fused passes read it: FP32 rows of its layer's
+        shape, one after another (a copy of a strided weight)."""
+        w = self.W[k]
+        assert w.dtype == torch.float32 and tuple(w.shape) == self.shapes[k], (w.dtype, w.shape)
+        return w.contiguous()
+
+    def _bias(self, k):
+        b = self.b[k]
+        if b is None:
+            return None
+        assert b.dtype == torch.float32 and b.numel() >= self.shapes[k][1], (b.dtype, b.shape)
+        return b.contiguous()
 
     def forward(self, X, keep=False):
         M, dev = X.shape[0], X.device
         assert X.dtype == torch.float32 and X.shape[1] == self.n_in
-        H1 = torch.empty((M, self.width), device=dev)
+        W, b = [self._weight(k) for k in range(3)], [self._bias(k) for k in range(3)]
+        for t in (*W, *b):
+            assert t is None or t.device == dev, (t.device, dev)
+        H1 = torch.empty((M, self.width), dtype=torch.float32, device=dev)
         H2 = torch.empty_like(H1)
-        Y = torch.empty((M, self.n_out), device=dev)
+        Y = torch.empty((M, self.n_out), dtype=torch.float32, device=dev)
         p = L.ptr
         rc = L.load().f3d_mlp_forward(
-            M, self.n_in, self.width, self.n_out, p(X), X.stride(0), X.stride(1), p(self.W[0]),
-            p(self.b[0]), p(self.W[1]), p(self.b[1]), p(self.W[2]), p(self.b[2]), p(H1), p(H2),
-            p(Y), _stream())
+            M, self.n_in, self.width, self.n_out, p(X), X.stride(0), X.stride(1), p(W[0]),
+            p(b[0]), p(W[1]), p(b[1]), p(W[2]), p(b[2]), p(H1), p(H2), p(Y), _stream())
         L.check(rc, "f3d_mlp_forward")
         if keep:
             self._cache = (X, H1, H2)
@@ -83,16 +100,20 @@ class MLP:
     def backward(self, dY):
         """Gradients of the loss wrt all parameters, given dL/dY."""
         X, H1, H2 = self._cache
-        M = X.shape[0]
+        M, dev = X.shape[0], X.device
         assert dY.dtype == torch.float32 and dY.shape == (M, self.n_out)
+        W2, W3 = self._weight(1), self._weight(2)
+        for t in (dY, W2, W3):
+            assert t.device == dev, (t.device, dev)
         lib = L.load()
-        grads = [torch.empty_like(q) for q in self.params]
+        grads = [torch.empty(s, dtype=torch.float32, device=dev)
+                 for s in self.shapes + [s[1:] for s in self.shapes]]
         need = lib.f3d_mlp_workspace_size(M, self.n_in, self.width, self.n_out)
-        ws = torch.empty(need, dtype=torch.uint8, device=X.device)
+        ws = torch.empty(need, dtype=torch.uint8, device=dev)
         p = L.ptr
         rc = lib.f3d_mlp_backward(
             M, self.n_in, self.width, self.n_out, p(X), X.stride(0), X.stride(1), p(H1), p(H2),
-            p(dY), dY.stride(0), dY.stride(1), p(self.W[1]), p(self.W[2]),
+            p(dY), dY.stride(0), dY.stride(1), p(W2), p(W3),
             *(p(g) for g in grads), p(ws), need, _stream())
         L.check(rc, "f3d_mlp_backward")
         return grads

@@ -202,3 +202,42 @@ def test_adam_and_mse_against_fp64():
     Y = net.forward(X)
     loss = net.train_step(X, T, lr=0.0)
     assert abs(loss - float(((Y.double() - T.double()) ** 2).mean())) <= 1e-6 * loss
+
+
+def test_mlp_passes_take_any_layout_and_check_types():
+    """A strided weight (and bias) acts as the dense copy of its values, in the
+    forward and the backward pass, also when the process's default type is
+    FP64; a layer without a bias adds none; a weight of another type or shape
+    is refused."""
+    print("case mlp layouts", flush=True)
+    rng = np.random.default_rng(8)
+    X = torch.from_numpy(rng.normal(size=(300, 5)).astype(np.float32)).cuda()
+    dY = torch.from_numpy(rng.normal(size=(300, 2)).astype(np.float32)).cuda()
+
+    def passes(net):
+        return [net.forward(X, keep=True)] + net.backward(dY)
+    net, dense = LG.MLP(5, 2, seed=6), LG.MLP(5, 2, seed=6)
+    for k in range(3):
+        w = torch.from_numpy(rng.normal(size=net.W[k].shape).astype(np.float32)).cuda() / 16
+        b = torch.from_numpy(rng.normal(size=net.b[k].shape).astype(np.float32)).cuda()
+        dense.W[k], dense.b[k] = w, b
+        net.W[k] = w.t().contiguous().t()
+        net.b[k] = torch.stack([b, -b], 1)[:, 0]
+    want = passes(dense)
+    assert all(torch.equal(a, b) for a, b in zip(passes(net), want))
+    torch.set_default_dtype(torch.float64)
+    try:
+        assert all(torch.equal(a, b) for a, b in zip(passes(net), want))
+    finally:
+        torch.set_default_dtype(torch.float32)
+    net.b[1], dense.b[1] = None, torch.zeros_like(dense.b[1])
+    assert torch.equal(net.forward(X), dense.forward(X))
+    for k in range(3):
+        for bad in (dense.W[k].double(), dense.W[k][:-1], dense.W[k].cpu()):
+            net.W[k] = bad
+            with pytest.raises(AssertionError):
+                net.forward(X)
+            if k:
+                with pytest.raises(AssertionError):
+                    net.backward(dY)
+        net.W[k] = dense.W[k]
