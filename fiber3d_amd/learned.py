@@ -119,14 +119,33 @@ class MLP:
         return grads
 
     def adam(self, grads, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8):
+        """One Adam step.  Tensors that the fused launch can address (dense FP32 of
+        one shape on the current device) take it together; any other follows the same
+        formulas through torch, which converts, broadcasts or refuses it."""
         self.t += 1
-        k = len(self.params)
-        grads = [g.contiguous() for g in grads]
+        fused = []
+        for q in zip(self.params, grads, self.m, self.v):
+            p, g = q[0], q[1].contiguous()
+            if p.is_cuda and p.device.index == torch.cuda.current_device() and all(
+                    t.dtype == torch.float32 and t.device == p.device and t.shape == p.shape
+                    and t.is_contiguous() for t in (p, g, *q[2:])):
+                fused.append((p, g, *q[2:]))
+            else:
+                self._adam_torch(*q, lr, b1, b2, eps)
+        if not fused:
+            return
+        k = len(fused)
         ptrs = lambda ts: (ctypes.c_void_p * k)(*(t.data_ptr() for t in ts))
-        sizes = (ctypes.c_int64 * k)(*(q.numel() for q in self.params))
-        rc = L.load().f3d_adam(k, sizes, ptrs(self.params), ptrs(grads), ptrs(self.m),
-                               ptrs(self.v), lr, b1, b2, eps, self.t, _stream())
+        p, g, m, v = zip(*fused)
+        sizes = (ctypes.c_int64 * k)(*(t.numel() for t in p))
+        rc = L.load().f3d_adam(k, sizes, ptrs(p), ptrs(g), ptrs(m), ptrs(v), lr, b1, b2, eps,
+                               self.t, _stream())
         L.check(rc, "f3d_adam")
+
+    def _adam_torch(self, p, g, m, v, lr, b1, b2, eps):
+        m.mul_(b1).add_(g, alpha=1 - b1)
+        v.mul_(b2).addcmul_(g, g, value=1 - b2)
+        p.sub_(lr * (m / (1 - b1**self.t)) / ((v / (1 - b2**self.t)).sqrt() + eps))
 
     def train_step(self, X, target, lr=1e-3):
         Y = self.forward(X, keep=True)

@@ -241,3 +241,52 @@ def test_mlp_passes_take_any_layout_and_check_types():
                 with pytest.raises(AssertionError):
                     net.backward(dY)
         net.W[k] = dense.W[k]
+
+
+def _adam_ref(p, g, m, v, t, lr):
+    g = g.astype(np.float64)
+    m = 0.9 * m + 0.1 * g
+    v = 0.999 * v + 0.001 * g * g
+    return p - lr * (m / (1 - 0.9 ** t)) / (np.sqrt(v / (1 - 0.999 ** t)) + 1e-8), m, v
+
+
+@pytest.mark.parametrize("odd", ["f64_grad", "strided_param", "strided_moment", "row_grad"])
+def test_adam_on_tensors_of_any_layout(odd):
+    """Gradients of another type or a broadcast shape, and parameters or
+    moments that are views, take the same step as dense ones, and what lies
+    beside a view stays as it is."""
+    print(f"case adam {odd}", flush=True)
+    rng = np.random.default_rng(14)
+    net = LG.MLP(4, 3, width=32, seed=3)
+    room = torch.full((32, 64), 5.0, device="cuda")
+    if odd == "strided_param":
+        room[:, ::2] = net.params[1]
+        net.params[1] = room[:, ::2]
+    if odd == "strided_moment":
+        net.m[1] = room[:, ::2].zero_()
+    P = [p.cpu().double().numpy() for p in net.params]
+    m, v = [np.zeros_like(p) for p in P], [np.zeros_like(p) for p in P]
+    for t in (1, 2):
+        G = [rng.normal(size=p.shape).astype(np.float32) for p in P]
+        if odd == "row_grad":
+            G[1] = G[1][:1]
+        g = [torch.from_numpy(q).cuda() for q in G]
+        if odd == "f64_grad":
+            g = [q.double() for q in g]
+        net.adam(g, lr=1e-2)
+        for k, q in enumerate(G):
+            P[k], m[k], v[k] = _adam_ref(P[k], np.broadcast_to(q, P[k].shape), m[k], v[k], t, 1e-2)
+    for p, r in zip(net.params, P):
+        np.testing.assert_allclose(p.cpu().double().numpy(), r, rtol=0, atol=3e-6)
+    assert bool((room[:, 1::2] == 5.0).all())
+
+
+def test_adam_refuses_tensors_it_cannot_use():
+    """A gradient of the wrong shape or in host memory is an error."""
+    print("case adam refused", flush=True)
+    for bad in (lambda g: g[:-1], lambda g: g.cpu()):
+        net = LG.MLP(4, 3, width=32, seed=3)
+        g = [torch.ones_like(p) for p in net.params]
+        g[1] = bad(g[1])
+        with pytest.raises(RuntimeError):
+            net.adam(g)
