@@ -149,16 +149,22 @@ class MLP:
 
     def train_step(self, X, target, lr=1e-3):
         Y = self.forward(X, keep=True)
-        assert torch.result_type(Y, target) == torch.float32
-        target = target.to(Y.dtype).expand_as(Y).contiguous()
-        lib = L.load()
-        dY = torch.empty_like(Y)
-        loss = torch.empty((), device=Y.device)
-        need = lib.f3d_mse_workspace_size()
-        ws = torch.empty(need, dtype=torch.uint8, device=Y.device)
-        rc = lib.f3d_mse(Y.numel(), L.ptr(Y), L.ptr(target), L.ptr(dY), L.ptr(loss), L.ptr(ws),
-                         need, _stream())
-        L.check(rc, "f3d_mse")
+        if (isinstance(target, torch.Tensor) and target.dtype == torch.float32
+                and target.device == Y.device and target.shape == Y.shape and Y.numel()):
+            target = target.contiguous()
+            lib = L.load()
+            dY = torch.empty_like(Y)
+            loss = torch.empty((), dtype=torch.float32, device=Y.device)
+            need = lib.f3d_mse_workspace_size()
+            ws = torch.empty(need, dtype=torch.uint8, device=Y.device)
+            rc = lib.f3d_mse(Y.numel(), L.ptr(Y), L.ptr(target), L.ptr(dY), L.ptr(loss), L.ptr(ws),
+                             need, _stream())
+            L.check(rc, "f3d_mse")
+        else:
+            # torch broadcasts and converts the target, or refuses it
+            diff = Y - target
+            loss = (diff * diff).mean()
+            dY = (2.0 / diff.numel()) * diff
         self.adam(self.backward(dY), lr=lr)
         return float(loss)  # waits for the device once the whole step is queued
 

@@ -290,3 +290,31 @@ def test_adam_refuses_tensors_it_cannot_use():
         g[1] = bad(g[1])
         with pytest.raises(RuntimeError):
             net.adam(g)
+
+
+def test_train_step_takes_the_targets_that_torch_subtracts():
+    """Targets that broadcast, of another type, one number or one value in host
+    memory train as the full FP32 tensor does; those that torch cannot subtract
+    from the output are refused."""
+    print("case train_step targets", flush=True)
+    rng = np.random.default_rng(21)
+    X = torch.from_numpy(rng.normal(size=(70, 3)).astype(np.float32)).cuda()
+    row = torch.tensor([1.5, -0.25], device="cuda")
+    full = row.expand(70, 2)
+
+    def params(target):
+        net = LG.MLP(3, 2, width=32, seed=4)
+        loss = net.train_step(X, target, lr=1e-2)
+        return loss, [p.cpu() for p in net.params]
+    for target, same in ((row, full), (full.half(), full), (full.t().contiguous().t(), full),
+                         (2.0, torch.full((70, 2), 2.0, device="cuda")),
+                         (torch.tensor(2.0), torch.full((70, 2), 2.0, device="cuda"))):
+        (la, pa), (lb, pb) = params(target), params(same.contiguous())
+        assert abs(la - lb) <= 1e-6 * lb
+        for a, b in zip(pa, pb):
+            torch.testing.assert_close(a, b, rtol=0, atol=2e-6)
+    for bad in (full.cpu(), full > 0):
+        with pytest.raises(RuntimeError):
+            params(bad)
+    with pytest.raises(AssertionError):
+        params(full.double())
