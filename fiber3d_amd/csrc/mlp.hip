@@ -916,7 +916,9 @@ extern "C" int f3d_mlp_backward(int64_t M, int32_t n_in, int32_t width, int32_t 
                                 size_t ws_bytes, void* stream) {
   F3D_REQUIRE(M >= 0 && M < (1ll << 31) && n_in >= 1 && width >= 1 && n_out >= 1, F3D_EINVAL,
               "mlp_backward: bad sizes");
-  F3D_REQUIRE(X && H1 && H2 && dY && W2 && W3 && gW1 && gW2 && gW3 && gb1 && gb2 && gb3, F3D_EINVAL,
+  // (no samples: zero gradients, and arrays of no elements may have no address)
+  F3D_REQUIRE(M == 0 || (X && H1 && H2 && dY), F3D_EINVAL, "mlp_backward: NULL argument");
+  F3D_REQUIRE(W2 && W3 && gW1 && gW2 && gW3 && gb1 && gb2 && gb3, F3D_EINVAL,
               "mlp_backward: NULL argument");
   const size_t need = f3d_mlp_workspace_size(M, n_in, width, n_out);
   F3D_REQUIRE(ws != nullptr && ws_bytes >= need, F3D_EWORKSPACE,
@@ -926,12 +928,14 @@ extern "C" int f3d_mlp_backward(int64_t M, int32_t n_in, int32_t width, int32_t 
   float* dZ1 = dZ2 + (size_t)M * width;
   float* part = dZ1 + (size_t)M * width;
   // dZ = (dOut W^T) where the layer's ReLU was open
-  int rc = f3d_gemm_bf16(EPI_RELU_GRAD, M, width, n_out, 1, dY, sym, syk, W3, 1, n_out, dZ2, width,
-                         1, nullptr, nullptr, H2, 1.0f, stream);
-  if (rc != F3D_OK) return rc;
-  rc = f3d_gemm_bf16(EPI_RELU_GRAD, M, width, width, 1, dZ2, width, 1, W2, 1, width, dZ1, width, 1,
-                     nullptr, nullptr, H1, 1.0f, stream);
-  if (rc != F3D_OK) return rc;
+  if (M > 0) {
+    int rc = f3d_gemm_bf16(EPI_RELU_GRAD, M, width, n_out, 1, dY, sym, syk, W3, 1, n_out, dZ2,
+                           width, 1, nullptr, nullptr, H2, 1.0f, stream);
+    if (rc != F3D_OK) return rc;
+    rc = f3d_gemm_bf16(EPI_RELU_GRAD, M, width, width, 1, dZ2, width, 1, W2, 1, width, dZ1, width,
+                       1, nullptr, nullptr, H1, 1.0f, stream);
+    if (rc != F3D_OK) return rc;
+  }
   GradPlan p;
   grad_slices(M, &p.kchunk, &p.slices);
   p.K = (int)M;

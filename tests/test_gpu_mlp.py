@@ -318,3 +318,13 @@ def test_train_step_takes_the_targets_that_torch_subtracts():
             params(bad)
     with pytest.raises(AssertionError):
         params(full.double())
+
+
+def test_mlp_passes_of_no_samples():
+    """An empty batch has an empty output and zero gradients."""
+    print("case mlp no samples", flush=True)
+    net = LG.MLP(5, 2, width=64, seed=6)
+    Y = net.forward(torch.empty((0, 5), device="cuda"), keep=True)
+    assert Y.shape == (0, 2)
+    for g, p in zip(net.backward(torch.empty((0, 2), device="cuda")), net.params):
+        assert g.shape == p.shape and not bool(g.any())
