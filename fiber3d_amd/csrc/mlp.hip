@@ -768,10 +768,9 @@ namespace f3d {
 // FP64, per block and then over the blocks in a fixed order.
 constexpr int kMseBlocks = 64;
 __global__ void __launch_bounds__(256)
-mse_kernel(int64_t n, const float* __restrict__ y, const float* __restrict__ t,
+mse_kernel(int64_t n, const float* __restrict__ y, const float* __restrict__ t, float c,
            float* __restrict__ dy, double* __restrict__ part) {
   __shared__ double red[4];
-  const float c = 2.0f / (float)n;
   double s = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
     const float d = y[i] - t[i];
@@ -831,7 +830,9 @@ extern "C" int f3d_mse(int64_t n, const float* y, const float* t, float* dy, flo
               "mse: workspace %zu bytes < required %zu", ws_bytes, f3d_mse_workspace_size());
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   double* part = reinterpret_cast<double*>(ws);
-  F3D_LAUNCH(mse_kernel, dim3(kMseBlocks), dim3(256), 0, st, n, y, t, dy, part);
+  // (2 / n rounded once: the FP32 value of n is not n from 2^24 on)
+  F3D_LAUNCH(mse_kernel, dim3(kMseBlocks), dim3(256), 0, st, n, y, t, (float)(2.0 / (double)n), dy,
+             part);
   F3D_LAUNCH(mse_final_kernel, dim3(1), dim3(kMseBlocks), 0, st, n, (const double*)part, loss);
   return F3D_OK;
 }

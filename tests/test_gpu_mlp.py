@@ -328,3 +328,19 @@ def test_mlp_passes_of_no_samples():
     assert Y.shape == (0, 2)
     for g, p in zip(net.backward(torch.empty((0, 2), device="cuda")), net.params):
         assert g.shape == p.shape and not bool(g.any())
+
+
+@pytest.mark.parametrize("n", [1, 3, 2 ** 24 + 1])
+def test_mse_gradient_factor_is_rounded_once(n):
+    """dy = fl(2 / n) (y - t), also where n itself is not an FP32 number."""
+    from fiber3d_amd import _lib as L
+    from fiber3d_amd.kernels import _stream
+    print(f"case mse factor n={n}", flush=True)
+    y, t = torch.rand(n, device="cuda"), torch.rand(n, device="cuda")
+    dy, loss = torch.empty_like(y), torch.empty((), device="cuda")
+    ws = torch.empty(L.load().f3d_mse_workspace_size(), dtype=torch.uint8, device="cuda")
+    L.check(L.load().f3d_mse(n, L.ptr(y), L.ptr(t), L.ptr(dy), L.ptr(loss), L.ptr(ws), ws.numel(),
+                             _stream()), "f3d_mse")
+    assert torch.equal(dy, (2.0 / n) * (y - t))
+    ref = float(((y - t).double() ** 2).mean())
+    assert abs(float(loss) - ref) <= 1e-6 * ref
