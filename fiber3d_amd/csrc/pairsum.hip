@@ -857,7 +857,7 @@ pairsum_kernel(const T* __restrict__ rec, const T* __restrict__ rec_far,
     hi[k] = 0;
     if ((excl_lo != nullptr || self_excl) && sl < nt) {
       lo[k] = self_excl ? sl : excl_lo[i];
-      hi[k] = self_excl ? sl + 1 : excl_hi[i];
+      hi[k] = self_excl ? sl + 1 : max(excl_hi[i], lo[k]);  // (reversed: empty)
     }
   }
 
@@ -1111,7 +1111,7 @@ pairsum_direct_kernel(int ns, const Sources src, int nt, const double* __restric
     lo[q] = hi[q] = 0;
     if (MASK) {
       lo[q] = excl_lo ? excl_lo[i] : i;
-      hi[q] = excl_lo ? excl_hi[i] : i + 1;
+      hi[q] = excl_lo ? max(excl_hi[i], lo[q]) : i + 1;  // (reversed: empty)
     }
     ax[q] = ay[q] = az[q] = 0.0;
   }

@@ -142,7 +142,8 @@ size_t f3d_pairsum_workspace_size(int kernel, int precision, int64_t ns, int64_t
  *   trg_pos   [nt] target positions
  *   excl_lo/excl_hi [nt] optional int32 half-open source-index range
  *             [lo_i, hi_i) whose pairs are EXCLUDED for target i (same-fiber
- *             exclusion, or lo=i,hi=i+1 to drop the self term); both NULL or
+ *             exclusion, or lo=i,hi=i+1 to drop the self term; none where
+ *             hi_i <= lo_i); both NULL or
  *             both set.  Replaces the add-then-subtract of the per-fiber self
  *             block (tstep_utils.py:703-729, :812-851).
  *   out       [nt] result, scaled by the kernel constant

@@ -273,3 +273,24 @@ def test_densities_and_normals_in_their_own_layouts(precision, ns, nt):
     b = FK.pairsum("stresslet", s, d, t, src_nrm=n, **kw)
     assert torch.equal(a, b)
     assert torch.equal(FK.pairsum("oseen", s, soa, t, **kw), FK.pairsum("oseen", s, d, t, **kw))
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32c"])
+@pytest.mark.parametrize("ns", [1000, 4096, 4097])
+@pytest.mark.parametrize("kind", ["oseen", "stresslet"])
+def test_reversed_exclusion_ranges_are_empty(kind, ns, prec):
+    """A range with hi < lo excludes nothing, whichever kernel takes the call
+    and whatever the ranges of the targets beside it."""
+    from fiber3d_amd.kernels import pairsum
+    print(f"case reversed ranges {kind} {ns} {prec}", flush=True)
+    rng = np.random.default_rng(ns)
+    X, F, T = (torch.from_numpy(rng.normal(size=(n, 3))).cuda() for n in (ns, ns, 130))
+    lo = torch.from_numpy(rng.integers(0, ns, 130).astype(np.int32)).cuda()
+    empty, rev = lo.clone(), lo - 1 - torch.arange(130, dtype=torch.int32, device="cuda")
+    empty[::3] += 40
+    rev[::3] = empty[::3]
+    kw = dict(src_nrm=F if kind == "stresslet" else None, precision=prec)
+    want = pairsum(kind, X, F, T, excl=(lo, empty), **kw)
+    assert torch.equal(pairsum(kind, X, F, T, excl=(lo, rev), **kw), want)
+    none = pairsum(kind, X, F, T, excl=(lo, lo - 1), **kw)
+    assert torch.equal(none, pairsum(kind, X, F, T, excl=(lo, lo), **kw))
