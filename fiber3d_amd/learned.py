@@ -65,33 +65,33 @@ class MLP:
         self.n_in, self.n_out, self.width = n_in, n_out, width
         self.shapes = [(n_in, width), (width, width), (width, n_out)]
 
-    def _weight(self, k):
-        """Weight k as the fused passes read it: FP32 rows of its layer's
-        shape, one after another (a copy of a strided weight)."""
-        w = self.W[k]
-        assert w.dtype == torch.float32 and tuple(w.shape) == self.shapes[k], (w.dtype, w.shape)
-        return w.contiguous()
-
-    def _bias(self, k):
-        b = self.b[k]
-        if b is None:
-            return None
-        assert b.dtype == torch.float32 and b.numel() >= self.shapes[k][1], (b.dtype, b.shape)
-        return b.contiguous()
+    def _dense(self, k, dev):
+        """Weight k (k < 3) or bias k - 3 as the fused passes read it: FP32 rows
+        of its layer's shape, one after another, on device index dev (a copy of
+        a strided one).  A bias may be None, or longer than its layer."""
+        if k < 3:
+            t = self.W[k]
+            ok = t.shape == self.shapes[k]
+        else:
+            t = self.b[k - 3]
+            if t is None:
+                return None
+            ok = t.numel() >= self.shapes[k - 3][1]
+        assert ok and t.dtype is torch.float32 and t.get_device() == dev, (k, t.shape, t.dtype,
+                                                                          t.device)
+        return t.contiguous()
 
     def forward(self, X, keep=False):
-        M, dev = X.shape[0], X.device
-        assert X.dtype == torch.float32 and X.shape[1] == self.n_in
-        W, b = [self._weight(k) for k in range(3)], [self._bias(k) for k in range(3)]
-        for t in (*W, *b):
-            assert t is None or t.device == dev, (t.device, dev)
-        H1 = torch.empty((M, self.width), dtype=torch.float32, device=dev)
+        M, dev = X.shape[0], X.get_device()
+        assert dev >= 0 and X.dtype == torch.float32 and X.shape[1] == self.n_in
+        W1, W2, W3, b1, b2, b3 = (self._dense(k, dev) for k in range(6))
+        H1 = X.new_empty((M, self.width))
         H2 = torch.empty_like(H1)
-        Y = torch.empty((M, self.n_out), dtype=torch.float32, device=dev)
+        Y = X.new_empty((M, self.n_out))
         p = L.ptr
         rc = L.load().f3d_mlp_forward(
-            M, self.n_in, self.width, self.n_out, p(X), X.stride(0), X.stride(1), p(W[0]),
-            p(b[0]), p(W[1]), p(b[1]), p(W[2]), p(b[2]), p(H1), p(H2), p(Y), _stream())
+            M, self.n_in, self.width, self.n_out, p(X), X.stride(0), X.stride(1), p(W1),
+            p(b1), p(W2), p(b2), p(W3), p(b3), p(H1), p(H2), p(Y), _stream())
         L.check(rc, "f3d_mlp_forward")
         if keep:
             self._cache = (X, H1, H2)
@@ -100,16 +100,15 @@ class MLP:
     def backward(self, dY):
         """Gradients of the loss wrt all parameters, given dL/dY."""
         X, H1, H2 = self._cache
-        M, dev = X.shape[0], X.device
-        assert dY.dtype == torch.float32 and dY.shape == (M, self.n_out)
-        W2, W3 = self._weight(1), self._weight(2)
-        for t in (dY, W2, W3):
-            assert t.device == dev, (t.device, dev)
+        M, dev = X.shape[0], X.get_device()
+        assert dY.dtype == torch.float32 and dY.shape == (M, self.n_out) and dY.get_device() == dev
+        W2, W3 = (self._dense(k, dev) for k in (1, 2))
         lib = L.load()
-        grads = [torch.empty(s, dtype=torch.float32, device=dev)
-                 for s in self.shapes + [s[1:] for s in self.shapes]]
+        # (dense whatever the parameters' layouts: the kernels write rows)
+        grads = ([X.new_empty(self.shapes[0]), torch.empty_like(W2), torch.empty_like(W3)]
+                 + [X.new_empty(s[1:]) for s in self.shapes])
         need = lib.f3d_mlp_workspace_size(M, self.n_in, self.width, self.n_out)
-        ws = torch.empty(need, dtype=torch.uint8, device=dev)
+        ws = X.new_empty(-(-need // 4))
         p = L.ptr
         rc = lib.f3d_mlp_backward(
             M, self.n_in, self.width, self.n_out, p(X), X.stride(0), X.stride(1), p(H1), p(H2),
@@ -124,14 +123,17 @@ class MLP:
         formulas through torch, which converts, broadcasts or refuses it."""
         self.t += 1
         fused = []
-        for q in zip(self.params, grads, self.m, self.v):
-            p, g = q[0], q[1].contiguous()
-            if p.is_cuda and p.device.index == torch.cuda.current_device() and all(
-                    t.dtype == torch.float32 and t.device == p.device and t.shape == p.shape
-                    and t.is_contiguous() for t in (p, g, *q[2:])):
-                fused.append((p, g, *q[2:]))
+        f32 = torch.float32
+        here = torch.cuda.current_device() if torch.cuda.is_initialized() else -2
+        for p, grad, m, v in zip(self.params, grads, self.m, self.v):
+            g = grad.contiguous()
+            if (p.dtype is f32 and g.dtype is f32 and m.dtype is f32 and v.dtype is f32
+                    and here == p.get_device() == g.get_device() == m.get_device()
+                    == v.get_device() and p.shape == g.shape == m.shape == v.shape
+                    and p.is_contiguous() and m.is_contiguous() and v.is_contiguous()):
+                fused.append((p, g, m, v))
             else:
-                self._adam_torch(*q, lr, b1, b2, eps)
+                self._adam_torch(p, grad, m, v, lr, b1, b2, eps)
         if not fused:
             return
         k = len(fused)
@@ -154,9 +156,9 @@ class MLP:
             target = target.contiguous()
             lib = L.load()
             dY = torch.empty_like(Y)
-            loss = torch.empty((), dtype=torch.float32, device=Y.device)
+            loss = Y.new_empty(())
             need = lib.f3d_mse_workspace_size()
-            ws = torch.empty(need, dtype=torch.uint8, device=Y.device)
+            ws = Y.new_empty(-(-need // 4))
             rc = lib.f3d_mse(Y.numel(), L.ptr(Y), L.ptr(target), L.ptr(dY), L.ptr(loss), L.ptr(ws),
                              need, _stream())
             L.check(rc, "f3d_mse")
