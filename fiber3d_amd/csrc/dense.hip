@@ -627,24 +627,43 @@ __device__ __forceinline__ void forward_segment(const T* __restrict__ L, int n, 
       });
 }
 
+// backward_segment where a pivot of the segment is zero, infinite, NaN or outside
+// 2^-400 .. 2^400: a division per column, one column at a time, for any number
+// of slots above.
+template <typename T>
+__device__ __forceinline__ void backward_segment_divide(const T* __restrict__ U, int n, int k0,
+                                                        int lane, double& cur,
+                                                        double (&next)[kSlots - 1]) {
+#pragma unroll 1
+  for (int j = min(64, n - k0) - 1; j >= 0; --j) {
+    const T* __restrict__ col = U + (long)(k0 + j) * n;
+    const double u = (double)col[k0 + min(lane, j)];
+    const double wk = readlane_f64(cur, j) / readlane_f64(u, j);
+    cur = lane == j ? wk : (lane < j ? fma(-u, wk, cur) : cur);
+#pragma unroll
+    for (int m = 1; m < kSlots; ++m)
+      if (64 * m <= k0) next[m - 1] = fma(-(double)col[k0 - 64 * m + lane], wk, next[m - 1]);
+  }
+}
+
 // w_k /= U(k, k); w_i -= U(i, k) w_k, i < k, for the columns of cur's segment
 // from the last to k0; next[m - 1]: slot m above.  Every row's quotient comes
 // from its reciprocal r = 1 / U(i, i), three operations on the chain where a
 // division takes about twelve: q = w r, then q + r (w - q U), the correctly
-// rounded quotient while nothing over- or underflows (Markstein).  A q that is
-// not finite stays as it is, and so does every q of a pivot outside
-// 2^-400 .. 2^400 (zero, infinite and NaN pivots among them).
+// rounded quotient while nothing over- or underflows (Markstein); a q that is
+// not finite stays as it is.  Returns whether the segment has a pivot outside
+// 2^-400 .. 2^400, whose reciprocal may do either: its results are to be dropped.
+// (The answer comes after the columns, not before them: asked before, a solve of
+// 1000 blocks of order 128 waits for the diagonal, 22.6 -> 23.0 us.)
 template <typename T, int NB>
-__device__ __forceinline__ void backward_segment(const T* __restrict__ U, int n, int k0, int lane,
+__device__ __forceinline__ bool backward_segment(const T* __restrict__ U, int n, int k0, int lane,
                                                  double& cur, double (&next)[kSlots - 1]) {
   const int cnt = min(64, n - k0);
+  const double dg = (double)U[(long)min(k0 + lane, n - 1) * (n + 1)];
   unsigned off[NB + 1];
 #pragma unroll
   for (int m = 1; m <= NB; ++m) off[m] = (unsigned)(k0 - 64 * m + lane) * (unsigned)sizeof(T);
-  const double dg = (double)U[(long)min(k0 + lane, n - 1) * (n + 1)];
   const double rc = 1.0 / dg;
-  const bool safe = fabs(dg) > 0x1p-400 && fabs(dg) < 0x1p400;
-  const double ds = safe ? dg : 0.0, rr = safe ? rc : 0.0;
   stream_chunks<T, NB + 1>(
       cnt, cur,
       [&](int j0, T (&r)[chunk_cols(NB + 1)][NB + 1]) __attribute__((always_inline)) {
@@ -657,13 +676,14 @@ __device__ __forceinline__ void backward_segment(const T* __restrict__ U, int n,
           if (decltype(tail)::value && j0 + u >= cnt) break;
           const int j = cnt - 1 - (j0 + u);
           const double q = cur * rc;
-          const double t = fma(fma(-q, ds, cur), rr, q);
+          const double t = fma(fma(-q, dg, cur), rc, q);
           const double wk = readlane_f64(isfinite(q) ? t : q, j);
           cur = lane == j ? wk : (lane < j ? fma(-(double)r[u][0], wk, cur) : cur);
 #pragma unroll
           for (int m = 1; m <= NB; ++m) next[m - 1] = fma(-(double)r[u][m], wk, next[m - 1]);
         }
       });
+  return __ballot(!(fabs(dg) > 0x1p-400 && fabs(dg) < 0x1p400)) != 0ull;
 }
 
 // w <- U^-1 L^-1 w (the factor's L unit lower, U upper, column-major), FP64
@@ -688,10 +708,18 @@ __device__ __forceinline__ void trsv_lu(const T* __restrict__ L, int n, int lane
 #pragma unroll
   for (int m = 0; m < kSlots - 1; ++m) next[m] = sw[64 * max(ns - 2 - m, 0) + lane];
   for (int s = ns - 1; s >= 0; --s) {
-    if (s == 3) backward_segment<T, 3>(L, n, 64 * s, lane, cur, next);
-    else if (s == 2) backward_segment<T, 2>(L, n, 64 * s, lane, cur, next);
-    else if (s == 1) backward_segment<T, 1>(L, n, 64 * s, lane, cur, next);
-    else backward_segment<T, 0>(L, n, 64 * s, lane, cur, next);
+    const double cur0 = cur, next0[kSlots - 1] = {next[0], next[1], next[2]};
+    bool wide;
+    if (s == 3) wide = backward_segment<T, 3>(L, n, 64 * s, lane, cur, next);
+    else if (s == 2) wide = backward_segment<T, 2>(L, n, 64 * s, lane, cur, next);
+    else if (s == 1) wide = backward_segment<T, 1>(L, n, 64 * s, lane, cur, next);
+    else wide = backward_segment<T, 0>(L, n, 64 * s, lane, cur, next);
+    if (wide) {
+      cur = cur0;
+#pragma unroll
+      for (int m = 0; m < kSlots - 1; ++m) next[m] = next0[m];
+      backward_segment_divide<T>(L, n, 64 * s, lane, cur, next);
+    }
     sw[64 * s + lane] = cur;
     cur = next[0];
     next[0] = next[1];

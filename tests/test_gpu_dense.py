@@ -349,3 +349,24 @@ def test_dense_gemv_batched_f32_entries(count, m, offset):
     torch.cuda.synchronize()
     ref = np.einsum("bij,bj->bi", M32.astype(np.float64), x.reshape(count, m)).ravel()
     assert rel2(y.cpu().numpy(), ref) < 1e-13
+
+
+@pytest.mark.parametrize("n", [1, 64, 65, 130, 256])
+def test_lu_solve_divides_by_pivots_beyond_the_reciprocal(n):
+    """Upper triangular factors with pivots whose reciprocal over- or
+    underflows, or whose quotients are the subnormal numbers: every entry is the
+    correctly rounded quotient of its right-hand side (the rest of the factor is
+    zero, so that nothing else rounds), in every segment of the rows."""
+    print(f"case lu solve quotients at the ends of the range n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    d = np.ldexp(rng.uniform(1.0, 2.0, n) * rng.choice([-1.0, 1.0], n),
+                 rng.choice([-1070, -1030, -1022, -700, -401, -3, 0, 401, 1000, 1023], n))
+    q = np.ldexp(rng.uniform(1.0, 2.0, n), rng.integers(-30, 30, n))
+    with np.errstate(over="ignore", under="ignore"):
+        x = np.clip(d * q, -1e308, 1e308)
+        ref = x / d
+    bs = BlockSet([n])
+    lu = BatchedLU(bs, bs.pack([np.eye(n)]), precision="f64", refine=0)
+    lu.lu64.copy_(torch.from_numpy(np.diag(d).ravel()))
+    y = lu.solve(torch.from_numpy(x).cuda()).cpu().numpy()
+    np.testing.assert_array_equal(y, ref)
