@@ -176,7 +176,7 @@ gm_current_kernel(int64_t n, const double* __restrict__ V, double* __restrict__ 
     xin[i] = vj[i];
 }
 
-// partial dots part[k * nc + c] = sum over chunk c of V_k . w, k = 0..j;
+// partial dots part[k * nc + c] = sum over chunks c, c + nc, .. of V_k . w, k = 0..j;
 // the last block sums them into h (add: h += the sums)
 __global__ void __launch_bounds__(kGb)
 gm_dots_kernel(int64_t n, int m, const double* __restrict__ V, const double* __restrict__ w,
@@ -188,11 +188,15 @@ gm_dots_kernel(int64_t n, int m, const double* __restrict__ V, const double* __r
   if ((int)blockIdx.y > j) return;
   const int nc = gridDim.x;
   const int c = blockIdx.x;
-  const int64_t i0 = (int64_t)c * kGchunk;
-  const int64_t i1 = i0 + kGchunk < n ? i0 + kGchunk : n;
   for (int k = blockIdx.y; k <= j; k += gridDim.y) {
     const double* __restrict__ vk = V + (int64_t)k * n;
-    const double s = block_sum(strided_dot(vk, w, i0 + threadIdx.x, i1, kGb), red);
+    // (more than kGmaxBlocks chunks: a block takes several)
+    double t = 0.0;
+    for (int64_t i0 = (int64_t)c * kGchunk; i0 < n; i0 += (int64_t)nc * kGchunk) {
+      const int64_t i1 = i0 + kGchunk < n ? i0 + kGchunk : n;
+      t += strided_dot(vk, w, i0 + threadIdx.x, i1, kGb);
+    }
+    const double s = block_sum(t, red);
     if (threadIdx.x == 0) p.part[(int64_t)k * nc + c] = s;
   }
   if (last_block(&p.ctl[cnt], nc * min((int)gridDim.y, j + 1))) {

@@ -106,3 +106,22 @@ def test_steps_at_chunk_edges(n):
     assert dev.info == 0 and dev.iterations == host.iterations
     # a residual of 1e-12 |b| and a smallest eigenvalue of 1: |x - b/d| <= 1e-12 |b|
     assert rel2(dev.x.cpu().numpy(), (b / d).cpu().numpy()) < 2.1e-12
+
+
+@pytest.mark.parametrize("n", [1024 * 4096, 1024 * 4096 + 1, 2 * 1024 * 4096 + 5000])
+def test_steps_of_vectors_beyond_one_chunk_per_block(n):
+    """The dot products' grid ends at 1024 blocks: vectors of more chunks than
+    that are summed whole, so the basis stays orthonormal (to n eps of the FP64
+    products that check it)."""
+    print(f"case gmres many chunks n={n}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    d = 1.0 + torch.rand(n, dtype=torch.float64, device="cuda", generator=g)
+    b = torch.zeros(n, dtype=torch.float64, device="cuda")
+    b[-1000:] = torch.randn(1000, dtype=torch.float64, device="cuda", generator=g)
+    ctx = GmresContext(n, 4, b.device)
+    ctx.begin(b)
+    for _ in range(3):
+        ctx.step(lambda x, out: torch.mul(d, x, out=out))
+    V = ctx.V[:4].cpu().numpy()
+    gram = V @ V.T
+    assert np.abs(gram - np.eye(4)).max() <= n * 2.0 ** -53
