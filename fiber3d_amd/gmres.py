@@ -227,7 +227,8 @@ def _gmres_host(matvec, b, precond, tol, restart, maxiter, x0, inner, callback, 
     # iterations continue to `target` (<= tol) once started; a guess (or any
     # restart) whose FP64 residual is already <= tol is accepted as it is
     t_it = tol if target is None else min(float(target), tol)
-    Pinv = precond if precond is not None else (lambda v, out=None: v.clone())
+    Pinv = precond if precond is not None else (
+        lambda v, out=None: v.clone() if out is None else out.copy_(v))
     op = inner if inner is not None else matvec
     inner_cycles = 0
     measured = None

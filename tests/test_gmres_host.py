@@ -185,3 +185,11 @@ def test_target_below_tolerance():
     near = torch.from_numpy(x * (1 + 1e-12))
     res = gmres(mv, bt, pc, tol=1e-8, target=1e-11, x0=near)
     assert res.iterations == 0 and res.guess_used and res.residual <= 1e-8
+
+
+def test_without_a_preconditioner():
+    """precond=None is the identity, in every product and in the update."""
+    A, b, mv, _, bt = _system(seed=5)
+    res = gmres(mv, bt, None, tol=1e-11, restart=20)
+    assert res.info == 0
+    assert np.linalg.norm(b - A @ res.x.numpy()) / np.linalg.norm(b) <= 1.01e-11
