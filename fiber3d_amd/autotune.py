@@ -145,9 +145,11 @@ def _time_queued(fn, reps, replays=3):
     the fastest of `replays` (host work does not count, nor do the launches
     of calls that follow each other)."""
     import torch
-    stream = torch.cuda.Stream()
+    from .kernels import recording_stream
+    stream = recording_stream()
     with torch.cuda.stream(stream):
         fn()
+        recording_stream()  # (its recorded work's workspace)
         stream.synchronize()
         g = torch.cuda.CUDAGraph()
         with torch.cuda.graph(g, stream=stream):

@@ -60,7 +60,7 @@ from dataclasses import dataclass
 import numpy as np
 import torch
 
-from .kernels import _stream
+from .kernels import _stream, recording_stream
 
 
 @dataclass
@@ -172,7 +172,7 @@ class GmresContext:
             torch.cuda.current_stream().synchronize()
             ctl = self.ctl.clone()
             graph = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(graph):
+            with torch.cuda.graph(graph, stream=recording_stream()):
                 self._step_eager(op)
             # recording ran nothing: replay it for this step
             self.ctl.copy_(ctl)

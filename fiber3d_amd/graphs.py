@@ -12,11 +12,14 @@ The recorded kernels hold the device addresses of everything the operator
 reads: positions, weights, assembled blocks, LU factors and the pair-sum
 workspace. A graph is therefore valid only until those tensors are replaced.
 The time stepper drops its graphs whenever it re-assembles the system.
-Recording runs the operator twice on a side stream first. That warms caches
-and grows the shared pair-sum workspace to its final size, so nothing is
-allocated inside the recording.
+Recording runs the operator twice on the recording stream first. That warms
+caches and grows that stream's pair-sum workspace to its final size, so nothing
+is allocated inside the recording. Graphs share that workspace: replay them in
+order.
 """
 import torch
+
+from .kernels import recording_stream
 
 
 class CapturedOperator:
@@ -30,15 +33,16 @@ class CapturedOperator:
         self.keep = tuple(keep)
         self.x = torch.zeros(n, dtype=dtype, device=device)
         self.y = torch.zeros(n, dtype=dtype, device=device)
-        side = torch.cuda.Stream(device=device)
+        side = recording_stream()
         side.wait_stream(torch.cuda.current_stream(device))
         with torch.cuda.stream(side):
             for _ in range(warmup):
                 fn(self.x, self.y)
+            recording_stream()  # (its recorded work's workspace)
         torch.cuda.current_stream(device).wait_stream(side)
         torch.cuda.synchronize(device)
         self.graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(self.graph):
+        with torch.cuda.graph(self.graph, stream=side):
             fn(self.x, self.y)
         self.replays = 0
 

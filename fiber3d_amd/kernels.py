@@ -12,6 +12,7 @@ A module-level precision (``set_precision``) selects FP64 (default, parity
 path) or FP32-compensated evaluation for the drop-in names.
 """
 import ctypes
+import threading
 
 import numpy as np
 import torch
@@ -55,11 +56,25 @@ def _ensure_tuned():
 # with, and freeing the buffer would hand that memory to other tensors.
 _ws_retired = []
 
+# Held from the look-up of a workspace to the end of the call that launches with
+# it: a sum is several launches, and those of two threads on one stream must
+# not interleave.
+_ws_lock = threading.RLock()
 
-def workspace(nbytes, tag="default"):
-    """A cached device byte buffer of at least nbytes (grown by >= 1.5x on
-    demand; a replaced buffer is retired, never freed)."""
-    key = (tag, torch.cuda.current_device())
+
+def workspace(nbytes, tag="default", at=None):
+    """The device byte buffer (at least nbytes) of the current stream (`at`, where
+    the caller has it): sums queued on different streams are not ordered, so
+    each stream has its own, and recorded work another than the stream's eager
+    work (graphs that share one: those recorded on one stream; replay them in
+    order).  Grown by >= 1.5x on demand; a replaced buffer is retired, never
+    freed."""
+    if _capturing():
+        tag = ("recorded", tag)
+    return _buffer((tag, at or _here()), nbytes)
+
+
+def _buffer(key, nbytes):
     buf = _ws.get(key)
     if buf is None or buf.numel() < nbytes:
         size = max(int(nbytes), 256)
@@ -71,15 +86,43 @@ def workspace(nbytes, tag="default"):
     return buf
 
 
+_recording = {}
+
+
+def recording_stream():
+    """The stream on which HIP graphs are recorded, one per device.  Its recorded
+    work has a workspace as large as the current stream's, so that recording
+    what has run here allocates none."""
+    dev = torch.cuda.current_device()
+    with _ws_lock:
+        if dev not in _recording:
+            _recording[dev] = torch.cuda.Stream()
+        side = _recording[dev]
+        mine = _ws.get(("default", _here()))
+        if mine is not None:
+            with torch.cuda.stream(side):
+                _buffer((("recorded", "default"), _here()), mine.numel())
+    return side
+
+
+_capturing = getattr(torch._C, "_cuda_isCurrentStreamCapturing",
+                     torch.cuda.is_current_stream_capturing)
+
+
 # the current stream's handle without a Stream object (0.3 us instead of 2.9,
 # of the 14 us of host work that bounded a small sum)
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
+def _here():
+    """(device index, raw handle) of the current stream."""
+    dev = torch.cuda.current_device()
+    return dev, (torch.cuda.current_stream().cuda_stream if _raw_stream is None
+                 else _raw_stream(dev))
+
+
 def _stream():
-    if _raw_stream is None:
-        return ctypes_stream(torch.cuda.current_stream())
-    return ctypes.c_void_p(_raw_stream(torch.cuda.current_device()))
+    return ctypes.c_void_p(_here()[1])
 
 
 def ctypes_stream(s):
@@ -150,14 +193,16 @@ def pairsum(kernel, src_pos, src_den, trg_pos, src_nrm=None, src_w=None, excl=No
         assert src_w.dtype == torch.float64 and src_w.numel() == ns and src_w.is_contiguous()
     prec = _PREC[precision]
     need = lib.f3d_pairsum_workspace_size(k, prec, ns, nt)
-    ws = workspace(need)
     flags = ((L.ACCUMULATE if accumulate else 0) | (L.CLAMP_NEAR if clamp_near else 0)
              | (L.EXCLUDE_SELF if exclude_self else 0))
-    rc = lib.f3d_pairsum_strided(
-        k, prec, flags, ns, src_pos.data_ptr(), s_sp, s_sc, _addr(src_nrm), n_sp, n_sc,
-        src_den.data_ptr(), d_sp, d_sc, _addr(src_w), nt, trg_pos.data_ptr(), t_sp, t_sc,
-        _addr(lo), _addr(hi), float(eta), float(reg), float(eps), out.data_ptr(), o_sp, o_sc,
-        ws.data_ptr(), ws.numel(), _stream())
+    at = _here()
+    with _ws_lock:
+        ws = workspace(need, at=at)
+        rc = lib.f3d_pairsum_strided(
+            k, prec, flags, ns, src_pos.data_ptr(), s_sp, s_sc, _addr(src_nrm), n_sp, n_sc,
+            src_den.data_ptr(), d_sp, d_sc, _addr(src_w), nt, trg_pos.data_ptr(), t_sp, t_sc,
+            _addr(lo), _addr(hi), float(eta), float(reg), float(eps), out.data_ptr(), o_sp, o_sc,
+            ws.data_ptr(), ws.numel(), at[1])
     L.check(rc, "f3d_pairsum")
     return out
 
@@ -174,10 +219,12 @@ def periphery_apply(pos, nrm, w, ex, ey, ez, q, add=None, eta=1.0, reg=5e-3, eps
     elif _strides3(out) != (sp, sc):
         raise ValueError("out must share the layout of the inputs")
     prec = _PREC[precision]
-    ws = workspace(lib.f3d_periphery_workspace_size(prec, n))
-    rc = lib.f3d_periphery_apply(prec, n, L.ptr(pos), L.ptr(nrm), L.ptr(w), L.ptr(ex), L.ptr(ey),
-                                 L.ptr(ez), L.ptr(q), L.ptr(add), sp, sc, float(eta), float(reg),
-                                 float(eps), L.ptr(out), L.ptr(ws), ws.numel(), _stream())
+    with _ws_lock:
+        ws = workspace(lib.f3d_periphery_workspace_size(prec, n))
+        rc = lib.f3d_periphery_apply(
+            prec, n, L.ptr(pos), L.ptr(nrm), L.ptr(w), L.ptr(ex), L.ptr(ey), L.ptr(ez), L.ptr(q),
+            L.ptr(add), sp, sc, float(eta), float(reg), float(eps), L.ptr(out), L.ptr(ws),
+            ws.numel(), _stream())
     L.check(rc, "f3d_periphery_apply")
     return out
 

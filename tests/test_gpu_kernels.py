@@ -294,3 +294,68 @@ def test_reversed_exclusion_ranges_are_empty(kind, ns, prec):
     assert torch.equal(pairsum(kind, X, F, T, excl=(lo, rev), **kw), want)
     none = pairsum(kind, X, F, T, excl=(lo, lo - 1), **kw)
     assert torch.equal(none, pairsum(kind, X, F, T, excl=(lo, lo), **kw))
+
+
+def _sums(count, ns=20000, nt=3000):
+    """Calls of pairsum (general path, several launches each) on data of their
+    own, with the results of serial runs."""
+    rng = np.random.default_rng(count)
+    calls = []
+    for k in range(count):
+        X, F, T = (torch.from_numpy(rng.normal(size=(n, 3))).cuda() for n in (ns + k, ns + k, nt))
+        kw = dict(src_nrm=F) if k % 2 else {}
+        calls.append(lambda kind=("oseen", "stresslet")[k % 2], X=X, F=F, T=T, kw=kw:
+                     FK.pairsum(kind, X, F, T, precision=("f64", "f32c")[k // 2 % 2], **kw))
+    want = [c() for c in calls]
+    torch.cuda.synchronize()
+    return calls, want
+
+
+def test_sums_on_several_streams_do_not_share_a_workspace():
+    """Sums queued on different streams at once, and graphs recorded on one stream
+    while it runs sums of its own, give what serial runs give."""
+    print("case sums on several streams", flush=True)
+    calls, want = _sums(4)
+    streams = [torch.cuda.Stream() for _ in calls]
+    for _ in range(5):
+        got = [None] * len(calls)
+        for s in streams:
+            s.wait_stream(torch.cuda.current_stream())
+        for k, (c, s) in enumerate(zip(calls, streams)):
+            with torch.cuda.stream(s):
+                got[k] = c()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+    # recorded on streams[0], replayed on the current stream beside eager sums there
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=streams[0]):
+        out = calls[1]()
+    for _ in range(5):
+        out.zero_()
+        streams[0].wait_stream(torch.cuda.current_stream())
+        graph.replay()
+        with torch.cuda.stream(streams[0]):
+            eager = calls[0]()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want[1]) and torch.equal(eager, want[0])
+
+
+def test_sums_from_several_threads_on_one_stream():
+    """A sum's launches are queued together: those of another thread on the same
+    stream come before or after."""
+    print("case sums from several threads", flush=True)
+    import threading
+    calls, want = _sums(4, ns=6000, nt=1000)
+    got = [[] for _ in calls]
+
+    def work(k):
+        for _ in range(20):
+            got[k].append(calls[k]())
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(len(calls))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for g, w in zip(got, want):
+        assert len(g) == 20 and all(torch.equal(a, w) for a in g)
