@@ -1283,6 +1283,12 @@ struct KernelTimer {
 };
 static KernelTimer g_timer;
 
+// The sizes that a sum accepts; a plan is made for these only (its counts are
+// 32-bit).
+static bool sizes_ok(int64_t ns, int64_t nt) {
+  return ns >= 0 && nt >= 0 && ns < (1ll << 30) && nt < (1ll << 30);
+}
+
 static Plan make_plan(int kernel, int precision, int64_t ns, int64_t nt) {
   Plan pl;
   const int kk = (kernel >= 0 && kernel < 3) ? kernel : 0;
@@ -1669,8 +1675,7 @@ extern "C" int f3d_pairsum_plan(int kernel, int precision, int64_t ns, int64_t n
               "pairsum_plan: unknown kernel %d", kernel);
   F3D_REQUIRE(precision == F3D_F64 || precision == F3D_F32C, F3D_EINVAL,
               "pairsum_plan: unknown precision %d", precision);
-  F3D_REQUIRE(ns >= 0 && nt >= 0 && ns < (1ll << 30) && nt < (1ll << 30), F3D_EINVAL,
-              "pairsum_plan: bad sizes");
+  F3D_REQUIRE(sizes_ok(ns, nt), F3D_EINVAL, "pairsum_plan: bad sizes");
   F3D_REQUIRE(out != nullptr, F3D_EINVAL, "pairsum_plan: NULL output");
   const Plan pl = make_plan(kernel, precision, ns, nt);
   out[0] = pl.K;
@@ -1707,7 +1712,7 @@ extern "C" int f3d_pairsum_timer_read(double* total_ms, int32_t* launches) {
 }
 
 extern "C" size_t f3d_pairsum_workspace_size(int kernel, int precision, int64_t ns, int64_t nt) {
-  if (precision != F3D_F64 && precision != F3D_F32C) return 0;
+  if ((precision != F3D_F64 && precision != F3D_F32C) || !sizes_ok(ns, nt)) return 0;
   return pairsum_ws(kernel, precision, ns, nt);
 }
 
@@ -1776,6 +1781,8 @@ extern "C" int f3d_pairsum_noalloc(int kernel, int precision, uint32_t flags, in
                                    int64_t t_sc, const int32_t* excl_lo, const int32_t* excl_hi,
                                    double eta, double reg, double eps, double* out, int64_t o_sp,
                                    int64_t o_sc, void* stream) {
+  F3D_REQUIRE(sizes_ok(ns, nt), F3D_EINVAL, "pairsum_noalloc: bad sizes ns=%lld nt=%lld",
+              (long long)ns, (long long)nt);
   void* ws = nullptr;
   const int rc = scratch_for_current_device(&ws);
   if (rc != F3D_OK) return rc;
@@ -1787,7 +1794,7 @@ extern "C" int f3d_pairsum_noalloc(int kernel, int precision, uint32_t flags, in
 }
 
 extern "C" size_t f3d_periphery_workspace_size(int precision, int64_t n) {
-  if (precision != F3D_F64 && precision != F3D_F32C) return 0;
+  if ((precision != F3D_F64 && precision != F3D_F32C) || !sizes_ok(n, n)) return 0;
   return pairsum_ws(F3D_STRESSLET, precision, n, n);
 }
 

@@ -117,7 +117,7 @@ int f3d_gemm_set_stream(int32_t n, int32_t enable);
 int f3d_pairsum_timer(int enable);
 int f3d_pairsum_timer_read(double* total_ms, int32_t* launches);
 
-/* Bytes of workspace f3d_pairsum needs for these sizes. */
+/* Bytes of workspace f3d_pairsum needs for these sizes (0 for sizes it refuses). */
 size_t f3d_pairsum_workspace_size(int kernel, int precision, int64_t ns, int64_t nt);
 
 /*

@@ -113,3 +113,28 @@ def test_bench_refuses_more_than_one_gpu():
                        capture_output=True, text=True, timeout=300)
     assert r.returncode != 0
     assert "one GPU" in (r.stdout + r.stderr)
+
+
+def test_sizes_beyond_the_range_are_refused_before_a_plan_is_made():
+    """Sizes whose padded 32-bit counts wrap round (to zero at 2^32 - 63 and 2^32)
+    ask for no workspace and are refused; in a process of its own, since a
+    plan for them divides by zero."""
+    import subprocess
+    import sys
+    code = ("import ctypes\n"
+            "from fiber3d_amd import _lib as L\n"
+            "lib, n = L.load(), None\n"
+            "for big in (-1, 2**30, 2**31, 2**32 - 63, 2**32, 2**40):\n"
+            "    for prec in (L.F64, L.F32C):\n"
+            "        for ns, nt in ((big, 10), (10, big)):\n"
+            "            assert lib.f3d_pairsum_workspace_size(0, prec, ns, nt) == 0\n"
+            "            rc = lib.f3d_pairsum_noalloc(0, prec, 0, ns, n, n, n, n, 3, 1, nt, n, 3,\n"
+            "                                         1, n, n, 1.0, 5e-3, 1e-5, n, 3, 1, n)\n"
+            "            assert rc == L.EINVAL, (rc, ns, nt)\n"
+            "        assert lib.f3d_periphery_workspace_size(prec, big) == 0\n"
+            "assert lib.f3d_pairsum_workspace_size(0, L.F64, 2**30 - 1, 10) > 0\n"
+            "print('ok')\n")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", code], cwd=root, capture_output=True, text=True,
+                       timeout=300)
+    assert r.returncode == 0 and r.stdout == "ok\n", (r.returncode, r.stderr)
