@@ -144,14 +144,14 @@ def _addr(t):
 
 
 def _as_common(ts):
-    """Make a list of (N,3) tensors (None allowed) share one (sp, sc)."""
+    """Make a list of (N,3) tensors (None allowed) share one (sp, sc) and device."""
     ref = next(t for t in ts if t is not None)
     st = _strides3(ref)
     out = []
     for t in ts:
         if t is None:
             out.append(None)
-        elif _strides3(t) != st:
+        elif _strides3(t) != st or t.device != ref.device:
             out.append(torch.empty_strided(ref.shape, ref.stride(), dtype=ref.dtype,
                                            device=ref.device).copy_(t))
         else:
@@ -176,7 +176,10 @@ def pairsum(kernel, src_pos, src_den, trg_pos, src_nrm=None, src_w=None, excl=No
     _ensure_tuned()
     nt = trg_pos.shape[0]
     ns = src_pos.shape[0]
-    if src_den.shape != src_pos.shape or (src_nrm is not None and src_nrm.shape != src_pos.shape):
+    dev = src_pos.get_device()
+    if (src_den.shape != src_pos.shape or src_den.get_device() != dev
+            or (src_nrm is not None and (src_nrm.shape != src_pos.shape
+                                         or src_nrm.get_device() != dev))):
         (src_pos, src_den, src_nrm), _ = _as_common([src_pos, src_den, src_nrm])
     s_sp, s_sc = _strides3(src_pos)
     d_sp, d_sc = _strides3(src_den)

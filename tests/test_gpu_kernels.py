@@ -359,3 +359,17 @@ def test_sums_from_several_threads_on_one_stream():
     torch.cuda.synchronize()
     for g, w in zip(got, want):
         assert len(g) == 20 and all(torch.equal(a, w) for a in g)
+
+
+@pytest.mark.parametrize("ns", [100, 5000])
+def test_densities_and_normals_in_host_memory_are_copied(ns):
+    """Densities and normals on the host, in either layout, act as their
+    copies on the positions' device."""
+    print(f"case host densities {ns}", flush=True)
+    rng = np.random.default_rng(ns)
+    X, F, N = (torch.from_numpy(rng.normal(size=(ns, 3))) for _ in range(3))
+    T = torch.from_numpy(rng.normal(size=(64, 3))).cuda()
+    soa = lambda t: t.t().contiguous().t()
+    want = FK.pairsum("stresslet", X.cuda(), F.cuda(), T, src_nrm=N.cuda())
+    for f, n in ((soa(F), N.cuda()), (F, N), (F.cuda(), soa(N))):
+        assert torch.equal(FK.pairsum("stresslet", X.cuda(), f, T, src_nrm=n), want)
