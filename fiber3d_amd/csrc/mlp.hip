@@ -339,7 +339,6 @@ grad_reduce_kernel(GradPlan p, const float* __restrict__ ws) {
 // every A fragment across the wave's two column tiles and every B fragment
 // across its two row tiles.
 constexpr int kSM = 128;  // rows per workgroup
-constexpr int kStreamRows = 49152;  // fewer rows take the tiled kernel
 constexpr int kSK = 32;   // K chunk
 constexpr int kSP = kSK + 8;  // LDS row pitch (bf16 elements): 80 B, 16-byte aligned
 
@@ -658,6 +657,33 @@ gemm_bf16_resident_kernel(int M, int N, int K, const float* __restrict__ A, long
 
 using namespace f3d;
 
+// Rows from which the row-block kernels are the faster ones.  Fewer leave CUs
+// idle or pay B's set-up for a block or two; the tiled kernel's time grows
+// faster with the rows, and faster still where its last 64-deep chunk of K is
+// partial.  us, N = 256, resident against tiled: K = 256, 8192 rows 38 / 11,
+// 32768 47 / 31, 49152 51 / 49, 262144 132 / 288; K = 128, 49151 32 / 32; K = 32, 4096
+// 8.1 / 7.2, 8192 8.9 / 10.3, 49151 18 / 40; K = 96, 8192 16 / 12, 16384 18.5 / 19.8,
+// 49151 27 / 48; K = 144, 24576 29 / 26, 32768 31 / 33; K = 16, 4096 6.0 / 6.2, 262144
+// 65 / 118.  N = 128 crosses near the same rows (K = 32, 8192 7.2 / 7.2; K = 96,
+// 16384 11.9 / 11.9; K = 144, 32768 18.5 / 19).
+constexpr int kStreamRows = 49152;
+static int64_t resident_rows(int64_t K) {
+  const int64_t part = K % 64;
+  if (part == 0) return kStreamRows;
+  return part == 32 ? 128 * K : std::min(256 * K, 20480 + 64 * K);
+}
+// The streaming kernel takes any K and alignment; at N = 256 a CU has one
+// workgroup of it, so its time is that of 128 rows a CU up to there: 32768 rows of K
+// = 130 (250), 28 us for 34 (38 for 49), but 48 for 41 (67 for 59) at 40000.  From
+// 7/8 of that on, where the tiled kernel has a partial chunk or a long one, and
+// B's rows are contiguous or its set-up little beside the products.  (K <= 16: the
+// tiled kernel at every size: K = 4, 262144 rows 97 / 88.)
+static bool stream_fills(int64_t M, int64_t N, int64_t K, bool b_rows) {
+  const int64_t full = (int64_t)kSM * num_cus();
+  return N == 256 && M <= full && 8 * M > 7 * full && (K % 64 != 0 || K > 128) &&
+         (b_rows || K > 128);
+}
+
 // Kernel for the per-node layers N = 128 / N = 256 (set by the autotuner
 // through f3d_gemm_set_stream): 0 tiled, 1 streaming, 2 resident-weight.
 static int g_gemm_stream[2] = {2, 2};
@@ -687,19 +713,17 @@ extern "C" int f3d_gemm_bf16(int epi, int64_t M, int64_t N, int64_t K, int32_t k
   if (M == 0 || N == 0) return F3D_OK;
   F3D_REQUIRE(A && B && C, F3D_EINVAL, "gemm_bf16: NULL operand");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  // the streaming paths: row-major A (unit K stride) and C (unit N stride),
-  // N in {128, 256}, 16 < K <= 256, no K split, from kStreamRows rows on.
-  // Fewer rows leave CUs idle or pay B's set-up for a block or two: at 256 x
-  // 256, 8192 rows take 12 us tiled, 26 streaming, 39 resident; 32768 rows 32,
-  // 33, 47; 49152 rows 50 tiled, 50 resident; 65536 rows 73, 61, 55; 262144 rows
-  // 288, 253, 130.  (At K = 4 the
-  // tiled kernel is the fastest at every size: 174 against 220 us at 262144.)
+  // the row-block kernels: row-major A (unit K stride) and C (unit N stride), N
+  // in {128, 256}, K <= 256, no K split; the resident one also needs K a
+  // multiple of 16 and 16-byte rows of A
   const int mode = (N == 128 || N == 256) ? g_gemm_stream[N == 256 ? 1 : 0] : 0;
-  const bool stream_ok = epi != EPI_ATOMIC && ksplit == 1 && sak == 1 && scn == 1 && mode > 0 &&
-                         K > 16 && K <= 256 && M >= kStreamRows;
-  // the resident-weight path also needs K a multiple of 16 and 16-byte rows of A
-  const bool resident_ok = stream_ok && mode == 2 && K > 0 && K % 16 == 0 && sam % 4 == 0 &&
-                           (reinterpret_cast<uintptr_t>(A) & 15) == 0;
+  const bool rows_ok = epi != EPI_ATOMIC && ksplit == 1 && sak == 1 && scn == 1 && mode > 0 &&
+                       K <= 256 && M >= kSM;
+  const bool resident = mode == 2 && K > 0 && K % 16 == 0 && sam % 4 == 0 &&
+                        (reinterpret_cast<uintptr_t>(A) & 15) == 0;
+  const bool resident_ok = rows_ok && resident && M >= resident_rows(K);
+  const bool stream_ok =
+      rows_ok && K > 16 && (M >= kStreamRows || (!resident && stream_fills(M, N, K, sbn == 1)));
   if (resident_ok) {
     const int RM = N == 256 ? 32 : 64;
     const int64_t nblocks = ceil_div(M, (int64_t)RM);

@@ -344,3 +344,53 @@ def test_mse_gradient_factor_is_rounded_once(n):
     assert torch.equal(dy, (2.0 / n) * (y - t))
     ref = float(((y - t).double() ** 2).mean())
     assert abs(float(loss) - ref) <= 1e-6 * ref
+
+
+def _layer(M, N, K, epi, form, seed, mode, in_place=False):
+    """One gemm call in a mode of f3d_gemm_set_stream; its results against FP64
+    products of the BF16-rounded operands, element by element: FP32
+    accumulation over K terms (2 K eps of the absolute products)."""
+    from fiber3d_amd import _lib as L
+    from fiber3d_amd import autotune
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    A = rnd(M, K + 3)[:, :K] if form == "strided" else rnd(M, K)
+    B, bias, zin = rnd(K, N), rnd(N), rnd(M, N)
+    b16 = lambda t: t.bfloat16().double()
+    pre, mag = b16(A) @ b16(B), b16(A).abs() @ b16(B).abs()
+    code = {"store": LG.EPI_STORE, "bias_relu": LG.EPI_BIAS_RELU, "bias": LG.EPI_BIAS,
+            "relu_grad": LG.EPI_RELU_GRAD}[epi]
+    if epi.startswith("bias"):
+        pre, mag = pre + bias.double(), mag + bias.double().abs()
+    want = pre.clamp(min=0) if epi == "bias_relu" else (
+        pre * (zin > 0) if epi == "relu_grad" else pre)
+    C = A if in_place else torch.full((M, N), 7.0, device="cuda")
+    Z = torch.full((M, N), 7.0, device="cuda") if epi == "bias_relu" and not in_place else None
+    L.check(L.load().f3d_gemm_set_stream(N, mode), "f3d_gemm_set_stream")
+    try:
+        LG.gemm(A, B.t().contiguous() if form == "transB" else B, C, code, transB=form == "transB",
+                bias=bias if epi.startswith("bias") else None, Z=Z,
+                Zin=zin if epi == "relu_grad" else None)
+        torch.cuda.synchronize()
+    finally:
+        autotune.apply()
+    bound = 2 * (K + 2) * 2.0 ** -24 * mag
+    assert bool(((C.double() - want).abs() <= bound).all()), mode
+    if Z is not None:
+        assert bool(((Z.double() - pre).abs() <= bound).all()), mode
+
+
+@pytest.mark.parametrize("N", [128, 256])
+@pytest.mark.parametrize("epi", ["store", "bias_relu", "bias", "relu_grad"])
+@pytest.mark.parametrize("M,K,form", [(4097, 16, "dense"), (4159, 32, "transB"), (12289, 96, "dense"),
+                                      (49153, 23, "dense"), (49280, 50, "transB"),
+                                      (49153, 48, "strided"), (49159, 64, "transB"),
+                                      (32768, 100, "dense"), (32767, 250, "transB")])
+def test_row_block_kernels_with_every_epilogue(M, K, form, epi, N):
+    """The resident and streaming kernels where the dispatch takes them (a K
+    that is not a multiple of 16 or of 4, or rows that are not aligned, goes to
+    the streaming kernel in both modes), with every epilogue, the
+    pre-activations, transposed weights and partial last row blocks."""
+    print(f"case row blocks {M}x{N}x{K} {form} {epi}", flush=True)
+    for mode in (2, 1):
+        _layer(M, N, K, epi, form, M + K, mode)
