@@ -684,6 +684,15 @@ static bool stream_fills(int64_t M, int64_t N, int64_t K, bool b_rows) {
          (b_rows || K > 128);
 }
 
+// Whether row-major a (M x K, row stride sa) and c (M x N, row stride sc) share
+// memory.
+static bool meets_rows(const float* a, int64_t M, int64_t K, int64_t sa, const float* c, int64_t N,
+                       int64_t sc) {
+  const int64_t a0 = std::min<int64_t>(0, (M - 1) * sa), a1 = std::max<int64_t>(0, (M - 1) * sa) + K;
+  const int64_t c0 = std::min<int64_t>(0, (M - 1) * sc), c1 = std::max<int64_t>(0, (M - 1) * sc) + N;
+  return K > 0 && a + a0 < c + c1 && c + c0 < a + a1;
+}
+
 // Kernel for the per-node layers N = 128 / N = 256 (set by the autotuner
 // through f3d_gemm_set_stream): 0 tiled, 1 streaming, 2 resident-weight.
 static int g_gemm_stream[2] = {2, 2};
@@ -721,9 +730,14 @@ extern "C" int f3d_gemm_bf16(int epi, int64_t M, int64_t N, int64_t K, int32_t k
                        K <= 256 && M >= kSM;
   const bool resident = mode == 2 && K > 0 && K % 16 == 0 && sam % 4 == 0 &&
                         (reinterpret_cast<uintptr_t>(A) & 15) == 0;
-  const bool resident_ok = rows_ok && resident && M >= resident_rows(K);
+  // Calls that only they can take: C or Z over A (a row block reads all of its
+  // rows before it writes them, where a tile of the tiled kernel may be
+  // written while another still reads).
+  const bool must = meets_rows(A, M, K, sam, C, N, scm) ||
+                    (Z && meets_rows(A, M, K, sam, Z, N, scm));
+  const bool resident_ok = rows_ok && resident && (must || M >= resident_rows(K));
   const bool stream_ok =
-      rows_ok && K > 16 && (M >= kStreamRows || (!resident && stream_fills(M, N, K, sbn == 1)));
+      rows_ok && (must || (K > 16 && (M >= kStreamRows || (!resident && stream_fills(M, N, K, sbn == 1)))));
   if (resident_ok) {
     const int RM = N == 256 ? 32 : 64;
     const int64_t nblocks = ceil_div(M, (int64_t)RM);

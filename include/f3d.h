@@ -438,6 +438,8 @@ int f3d_gmres_solve(int64_t n, int32_t m, int32_t k, const double* V, double* up
  *   0 store; 1 + bias[n], store pre-activation to Z (nullable), ReLU;
  *   2 multiply by ReLU'(Zin) (Zin > 0); 3 atomic add (C pre-zeroed; the only
  *   mode allowed with ksplit > 1); 4 + bias[n].
+ * C may be Zin.  C (or Z) may be A only for N <= 64, or for N = 128 or 256 with at
+ * least 128 rows, unit sak and scn, K <= 256 and a row-block kernel enabled.
  */
 int f3d_gemm_bf16(int epi, int64_t M, int64_t N, int64_t K, int32_t ksplit, const float* A,
                   int64_t sam, int64_t sak, const float* B, int64_t sbk, int64_t sbn, float* C,

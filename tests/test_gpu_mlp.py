@@ -394,3 +394,12 @@ def test_row_block_kernels_with_every_epilogue(M, K, form, epi, N):
     print(f"case row blocks {M}x{N}x{K} {form} {epi}", flush=True)
     for mode in (2, 1):
         _layer(M, N, K, epi, form, M + K, mode)
+
+
+@pytest.mark.parametrize("N", [128, 256])
+@pytest.mark.parametrize("M", [128, 1000, 4096])
+def test_layers_in_place(M, N):
+    """An N x N layer whose output is its input's storage."""
+    print(f"case layer in place {M}x{N}", flush=True)
+    for mode in (2, 1):
+        _layer(M, N, N, "bias_relu", "dense", M + N, mode, in_place=True)
