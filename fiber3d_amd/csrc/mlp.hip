@@ -684,6 +684,9 @@ static bool stream_fills(int64_t M, int64_t N, int64_t K, bool b_rows) {
          (b_rows || K > 128);
 }
 
+// Row tiles of the tiled kernel's grid (its y extent).
+constexpr int64_t kTiledRowTiles = 65535;
+
 // Whether row-major a (M x K, row stride sa) and c (M x N, row stride sc) share
 // memory.
 static bool meets_rows(const float* a, int64_t M, int64_t K, int64_t sa, const float* c, int64_t N,
@@ -732,9 +735,10 @@ extern "C" int f3d_gemm_bf16(int epi, int64_t M, int64_t N, int64_t K, int32_t k
                         (reinterpret_cast<uintptr_t>(A) & 15) == 0;
   // Calls that only they can take: C or Z over A (a row block reads all of its
   // rows before it writes them, where a tile of the tiled kernel may be
-  // written while another still reads).
+  // written while another still reads), and more rows than its grid has.
   const bool must = meets_rows(A, M, K, sam, C, N, scm) ||
-                    (Z && meets_rows(A, M, K, sam, Z, N, scm));
+                    (Z && meets_rows(A, M, K, sam, Z, N, scm)) ||
+                    ceil_div(M, (int64_t)kMT) > kTiledRowTiles;
   const bool resident_ok = rows_ok && resident && (must || M >= resident_rows(K));
   const bool stream_ok =
       rows_ok && (must || (K > 16 && (M >= kStreamRows || (!resident && stream_fills(M, N, K, sbn == 1)))));

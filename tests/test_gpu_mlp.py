@@ -403,3 +403,16 @@ def test_layers_in_place(M, N):
     print(f"case layer in place {M}x{N}", flush=True)
     for mode in (2, 1):
         _layer(M, N, N, "bias_relu", "dense", M + N, mode, in_place=True)
+
+
+def test_more_rows_than_the_tiled_grid_has():
+    """A short K, which the tiled kernel takes, with more row tiles than a grid's y
+    extent: the rows go to a row-block kernel."""
+    print("case rows beyond the tiled grid", flush=True)
+    M, N, K = 64 * 65536 + 1, 128, 4
+    A, B = torch.randn(M, K, device="cuda"), torch.randn(K, N, device="cuda")
+    C = torch.full((M, N), 7.0, device="cuda")
+    LG.gemm(A, B, C)
+    for rows in (slice(0, 1000), slice(M // 2, M // 2 + 1000), slice(M - 1000, M)):
+        want = A[rows].bfloat16().double() @ B.bfloat16().double()
+        assert rel2(C[rows].cpu().numpy(), want.cpu().numpy()) < 1e-6
