@@ -1,24 +1,24 @@
-"""Autotuner of the launch shapes: pair sums per size bucket, the batched LU
-and the BF16 GEMM.
+"""Autotuner of the launch shapes: pair sums per size bucket and the BF16
+GEMM.
 
 Pair sums: for each (kernel, precision) and each tuned problem size
 (n_targets, n_sources) of a grid of powers of two, it times f3d_pairsum (there
 and at three quarters of it) over the launch shapes -- targets per lane K in
 {1, 2, 4} and the wavefront count the source split aims for -- and keeps the
 fastest.  FP32C sums depend on their shape at the 1e-8 level (K groups the
-targets of the near/far test, the split the compensated partial sums): the saved
-table holds FP32C shapes that were tuned on powers of four only, and sizes in
-between (the entries without a rate) take the nearest of those.  apply() installs the
+targets of the near/far test, the split the compensated partial sums), so their
+shapes are tuned on powers of four only, over fewer wavefront counts, and the
+sizes in between (the entries without a rate) take the nearest of those: a finer
+grid would change sums of those sizes.  apply() installs the
 fastest shape of the nearest tuned size (in log2 n_targets + log2 n_sources)
 into every size bucket of the library (f3d_pairsum_set_launch_bucket), and
 the 65536 x 65536 shape as the (kernel, precision) default.  The large
 fiber -> fiber Oseen sum (262144 nodes, exclusion ranges) is tuned on its
 own layout, bucket 18/18.
 
-Batched LU (f3d_lu_set_launch): waves per CU and solve staging, timed on
-fiber blocks of the shapes the stepper factors (the waves-per-CU entry is
-checked and stored, but no launch depends on either any more).  BF16 GEMM (f3d_gemm_set_stream): resident-weight,
-streaming or tiled kernel for the per-node layers (N = 128, 256).
+BF16 GEMM (f3d_gemm_set_stream): resident-weight, streaming or tiled kernel for
+the per-node layers (N = 128, 256).  Batched LU (f3d_lu_set_launch): a table's
+entry is checked and passed on, but no launch depends on it, and none is tuned.
 
 The table lives in fiber3d_amd/tuning.json; the kernels module calls apply()
 at import when it exists.  validate() checks a table's shape and ranges.
@@ -37,10 +37,15 @@ KERNELS = {"oseen": L.OSEEN, "rotlet": L.ROTLET, "stresslet": L.STRESSLET}
 PRECS = {"f64": L.F64, "f32c": L.F32C}
 LG_MIN, LG_MAX = 8, 22          # size buckets of the library (log2 sizes)
 KS = (1, 2, 4)
-WAVES = (2048, 4096, 8192, 16384, 32768)
+WAVES = {"f64": (2048, 4096, 8192, 12288, 16384, 24576, 32768, 65536),
+         "f32c": (2048, 4096, 8192, 16384, 32768)}
 GRID_NT = (4096, 8192, 16384, 32768, 65536, 262144)
 GRID_NS = (1024, 2048, 4096, 8192, 16384, 32768, 65536)
-LU_WAVES = {"f64": (1, 2, 4), "f32c": (2, 4, 8)}
+# the sizes of the grid whose shapes are timed
+TUNED = {"f64": (GRID_NT, GRID_NS),
+         "f32c": ((4096, 16384, 65536), (1024, 4096, 16384, 65536))}
+LU_LAUNCH = {"f64": {"factor_waves_per_cu": 4, "solve_staged": 0},
+             "f32c": {"factor_waves_per_cu": 8, "solve_staged": 0}}
 
 
 def set_launch(kernel, precision, k, waves):
@@ -79,6 +84,18 @@ def expand_buckets(tuned):
     pts = sorted(tuned)
     return {(a, b): tuned[_nearest(pts, a, b)]
             for a in range(LG_MIN, LG_MAX + 1) for b in range(LG_MIN, LG_MAX + 1)}
+
+
+def fill_grid(rated):
+    """The entries of every size of the grid: the timed ones ({"16/12": entry}),
+    and in between the shape of the nearest of them."""
+    pts = {tuple(int(s) for s in size.split("/")): v for size, v in rated.items()}
+    near = {}
+    for nt in GRID_NT:
+        for ns in GRID_NS:
+            v = pts[_nearest(sorted(pts), lg(nt), lg(ns))]
+            near[f"{lg(nt)}/{lg(ns)}"] = {"k": v["k"], "waves": v["waves"]}
+    return {**near, **rated}
 
 
 def validate(table):
@@ -186,14 +203,15 @@ def _time(fn, min_s=0.02, max_reps=200):
 
 
 def tune_pairsum(kernels=("oseen", "stresslet", "rotlet"), precisions=("f32c", "f64"),
-                 grid_nt=GRID_NT, grid_ns=GRID_NS, ks=KS, waves=WAVES, seed=0, log=None):
-    """Fastest (K, waves) per (kernel, precision) and tuned size; the
-    65536 x 65536 entry is also the (kernel, precision) default."""
+                 ks=KS, seed=0, log=None):
+    """Fastest (K, waves) per (kernel, precision) and tuned size, the grid's other
+    sizes filled from them; the 65536 x 65536 entry is also the (kernel,
+    precision) default."""
     import torch
     from .kernels import pairsum
 
     rng = np.random.default_rng(seed)
-    nmax = max(max(grid_nt), max(grid_ns))
+    nmax = max(GRID_NT + GRID_NS)
     X = torch.from_numpy(rng.uniform(0, 1, (nmax, 3))).cuda()
     F = torch.from_numpy(rng.normal(size=(nmax, 3))).cuda()
     NR = torch.nn.functional.normalize(torch.from_numpy(rng.normal(size=(nmax, 3))), dim=1).cuda()
@@ -203,11 +221,12 @@ def tune_pairsum(kernels=("oseen", "stresslet", "rotlet"), precisions=("f32c", "
         for precision in precisions:
             key = f"{kernel}/{precision}"
             buckets[key] = {}
+            grid_nt, grid_ns = TUNED[precision]
             for nt in grid_nt:
                 for ns in grid_ns:
                     best = None
                     for k in ks:
-                        for w in waves:
+                        for w in WAVES[precision]:
                             set_launch_bucket(kernel, precision, lg(nt), lg(ns), k, w)
                             t = pairs = 0.0
                             # the bucket's largest sizes and three quarters of them
@@ -228,10 +247,11 @@ def tune_pairsum(kernels=("oseen", "stresslet", "rotlet"), precisions=("f32c", "
                         log(f"{key} nt={nt} ns={ns}: {ent}")
                     if nt == ns == 65536:
                         defaults[key] = dict(ent)
+            buckets[key] = fill_grid(buckets[key])
     return defaults, buckets
 
 
-def tune_pairsum_fibers(precisions=("f32c", "f64"), ks=KS, waves=WAVES, log=None):
+def tune_pairsum_fibers(precisions=("f32c", "f64"), ks=KS, log=None):
     """The fiber -> fiber Oseen sum of the large workload (4096 fibers x 64
     nodes in a ball of radius 14, each fiber's own nodes excluded): its
     spatially compact tiles and exclusion ranges (the given order is kept)
@@ -256,7 +276,7 @@ def tune_pairsum_fibers(precisions=("f32c", "f64"), ks=KS, waves=WAVES, log=None
     for precision in precisions:
         best = None
         for k in ks:
-            for w in waves:
+            for w in WAVES[precision]:
                 set_launch_bucket("oseen", precision, lg(n), lg(n), k, w)
                 t = _time(lambda: pairsum("oseen", X, F, X, excl=excl, precision=precision,
                                           out=out), min_s=0.05, max_reps=5)
@@ -268,52 +288,6 @@ def tune_pairsum_fibers(precisions=("f32c", "f64"), ks=KS, waves=WAVES, log=None
         res[f"oseen/{precision}"] = {f"{lg(n)}/{lg(n)}": ent}
         if log:
             log(f"oseen/{precision} fibers n={n}: {ent}")
-    return res
-
-
-def _lu_workload(seed=0):
-    """Fiber blocks of the stepper's shapes: 1000 fibers of 32 nodes
-    (n = 128) and 512 of 64 nodes (n = 256), A_sq from the discretisation."""
-    from . import configs
-    from .system import FiberSystem
-    out = []
-    for nfib, N in ((1000, 32), (512, 64)):
-        spec = configs.FiberSpec(nfib, N, 1.0, 6.0)
-        S = FiberSystem(configs.make_fibers(spec, seed), None, lu_precision="f64")
-        out.append(S)
-    return out
-
-
-def tune_lu(log=None):
-    import torch
-    from .dense import BatchedLU
-
-    systems = _lu_workload()
-    res = {}
-    for prec in ("f64", "f32c"):
-        best = None
-        for w in LU_WAVES[prec]:
-            L.check(L.load().f3d_lu_set_launch(PRECS[prec], w, 1), "f3d_lu_set_launch")
-            lus = [BatchedLU(S.bs, S.A_buf, precision=prec, refine=0) for S in systems]
-            t = _time(lambda: [lu.factor() for lu in lus])
-            if best is None or t < best[0]:
-                best = (t, w)
-        timings = {}
-        for staged in (1, 0):
-            L.check(L.load().f3d_lu_set_launch(PRECS[prec], best[1], staged),
-                    "f3d_lu_set_launch")
-            lus = [BatchedLU(S.bs, S.A_buf, precision=prec, refine=0) for S in systems]
-            xs = [torch.randn(S.bs.nrows, dtype=torch.float64, device="cuda") for S in systems]
-            ys = [torch.empty_like(x) for x in xs]
-            timings[staged] = _time(lambda: [lu.solve(x, out=y)
-                                             for lu, x, y in zip(lus, xs, ys)])
-        staged = 1 if timings[1] <= timings[0] else 0
-        L.check(L.load().f3d_lu_set_launch(PRECS[prec], best[1], staged), "f3d_lu_set_launch")
-        res[prec] = {"factor_waves_per_cu": best[1], "factor_ms": round(best[0] * 1e3, 4),
-                     "solve_staged": staged, "solve_ms_staged": round(timings[1] * 1e3, 4),
-                     "solve_ms_streaming": round(timings[0] * 1e3, 4)}
-        if log:
-            log(f"lu {prec}: {res[prec]}")
     return res
 
 
@@ -342,7 +316,13 @@ def tune_gemm(M=262144, K=256, log=None):
     return res
 
 
-PARTS = ("pairsum", "fibers", "lu", "gemm")
+PARTS = ("pairsum", "fibers", "gemm")
+
+
+PROBLEM = (f"pair sums: unit-cube points, n_targets x n_sources over {list(GRID_NT)} x "
+           f"{list(GRID_NS)} (FP64) and {list(TUNED['f32c'][0])} x {list(TUNED['f32c'][1])} "
+           "(FP32C, other sizes from the nearest), and the 262144-node fiber -> fiber Oseen sum "
+           "with exclusion ranges (bucket 18/18); GEMM: 262144 x 256 x N")
 
 
 def tune_all(path=CACHE, log=print, parts=PARTS, base=None):
@@ -361,15 +341,11 @@ def tune_all(path=CACHE, log=print, parts=PARTS, base=None):
     if "fibers" in parts:
         for k, b in tune_pairsum_fibers(log=log).items():
             table.setdefault("pairsum_buckets", {}).setdefault(k, {}).update(b)
-    if "lu" in parts:
-        table["lu"] = tune_lu(log=log)
+    table["lu"] = {p: dict(v) for p, v in LU_LAUNCH.items()}
     if "gemm" in parts:
         table["gemm"] = tune_gemm(log=log)
     table["device"] = torch.cuda.get_device_name(0)
-    table["problem"] = ("pair sums: unit-cube points, n_targets x n_sources over "
-                        f"{list(GRID_NT)} x {list(GRID_NS)}, and the 262144-node fiber -> "
-                        "fiber Oseen sum with exclusion ranges (bucket 18/18); LU: 1000 "
-                        "blocks of order 128 and 512 of order 256; GEMM: 262144 x 256 x N")
+    table["problem"] = PROBLEM
     validate(table)
     if path:
         with open(path, "w") as fh:

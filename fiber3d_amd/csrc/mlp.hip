@@ -661,7 +661,7 @@ using namespace f3d;
 // idle or pay B's set-up for a block or two; the tiled kernel's time grows
 // faster with the rows, and faster still where its last 64-deep chunk of K is
 // partial.  us, N = 256, resident against tiled: K = 256, 8192 rows 38 / 11,
-// 32768 47 / 31, 49152 51 / 49, 262144 132 / 288; K = 128, 49151 32 / 32; K = 32, 4096
+// 32768 47 / 31, 49152 51 / 49, 262144 134 / 231; K = 128, 49151 32 / 32; K = 32, 4096
 // 8.1 / 7.2, 8192 8.9 / 10.3, 49151 18 / 40; K = 96, 8192 16 / 12, 16384 18.5 / 19.8,
 // 49151 27 / 48; K = 144, 24576 29 / 26, 32768 31 / 33; K = 16, 4096 6.0 / 6.2, 262144
 // 65 / 118.  N = 128 crosses near the same rows (K = 32, 8192 7.2 / 7.2; K = 96,

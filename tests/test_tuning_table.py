@@ -101,3 +101,21 @@ def test_bucket_reset_returns_to_the_default():
     assert AT.plan("rotlet", "f32c", 4096, 4096)[0] == 4
     AT.set_launch_bucket("rotlet", "f32c", 12, 12, 0, 0)
     assert AT.plan("rotlet", "f32c", 4096, 4096)[0] == 1
+
+
+def test_tuner_can_produce_the_saved_table():
+    """Every saved shape is one the tuner tries at a size it times; the grid's other
+    sizes have the shape that the tuner fills in; no section describes launches
+    that nothing chooses."""
+    t = _saved()
+    for key, buckets in t["pairsum_buckets"].items():
+        prec = key.split("/")[1]
+        rated = {s: v for s, v in buckets.items() if "gpairs_s" in v}
+        for v in [*rated.values(), t["pairsum"][key]]:
+            assert v["k"] in AT.KS and v["waves"] in AT.WAVES[prec], (key, v)
+        grid = {s: v for s, v in rated.items() if s != "18/18"}
+        nts, nss = AT.TUNED[prec]
+        assert set(grid) == {f"{AT.lg(nt)}/{AT.lg(ns)}" for nt in nts for ns in nss}
+        assert AT.fill_grid(grid) == {s: v for s, v in buckets.items() if s != "18/18"}
+    assert t["lu"] == AT.LU_LAUNCH and "lu" not in AT.PARTS
+    assert t["problem"] == AT.PROBLEM
