@@ -137,9 +137,13 @@ class MLP:
         if not fused:
             return
         k = len(fused)
-        ptrs = lambda ts: (ctypes.c_void_p * k)(*(t.data_ptr() for t in ts))
-        p, g, m, v = zip(*fused)
-        sizes = (ctypes.c_int64 * k)(*(t.numel() for t in p))
+        p, g, m, v = ([t.data_ptr() for t in ts] for ts in zip(*fused))
+        if len({*p, *m, *v}) < 3 * k:  # shared storage: one after the other
+            for q in fused:
+                self._adam_torch(*q, lr, b1, b2, eps)
+            return
+        ptrs = lambda ts: (ctypes.c_void_p * k)(*ts)
+        sizes = (ctypes.c_int64 * k)(*(q[0].numel() for q in fused))
         rc = L.load().f3d_adam(k, sizes, ptrs(p), ptrs(g), ptrs(m), ptrs(v), lr, b1, b2, eps,
                                self.t, _stream())
         L.check(rc, "f3d_adam")

@@ -416,3 +416,17 @@ def test_more_rows_than_the_tiled_grid_has():
     for rows in (slice(0, 1000), slice(M // 2, M // 2 + 1000), slice(M - 1000, M)):
         want = A[rows].bfloat16().double() @ B.bfloat16().double()
         assert rel2(C[rows].cpu().numpy(), want.cpu().numpy()) < 1e-6
+
+
+def test_adam_on_shared_parameters():
+    """A parameter listed twice takes both of its steps, one after the other."""
+    print("case adam shared", flush=True)
+    rng = np.random.default_rng(5)
+    net = LG.MLP(4, 3, width=4096, seed=3)
+    net.params[4] = net.params[3]
+    G = [rng.normal(size=p.shape).astype(np.float32) for p in net.params]
+    net.adam([torch.from_numpy(q).cuda() for q in G], lr=1e-2)
+    want = np.zeros(4096)
+    for q in (G[3], G[4]):
+        want = _adam_ref(want, q, np.zeros(4096), np.zeros(4096), 1, 1e-2)[0]
+    np.testing.assert_allclose(net.params[3].cpu().double().numpy(), want, rtol=0, atol=3e-6)
