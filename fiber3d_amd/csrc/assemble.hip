@@ -1,5 +1,6 @@
-// Batched per-fiber assembly of the implicit fiber system (FP64), one
-// 256-thread workgroup per fiber, for fibers of one node count N (5..64).
+// Batched per-fiber assembly of the implicit fiber system (FP64) for fibers of
+// one node count N (5..64): persistent 256-thread workgroups, or up to four per
+// fiber where there are few.
 //
 // Reference: fiber.form_linear_operator (python/fiber/fiber.py:322-447),
 // apply_BC_rectangular with force- and torque-free ends (:810-961),

@@ -6,7 +6,8 @@
 //     (lu_factor_f32_mfma_kernel below), two 256-thread workgroups per CU;
 //   * forward/backward substitution with optional FP64 iterative refinement,
 //     one wavefront per block;
-//   * column-major block GEMV, one wavefront per block.
+//   * column-major block GEMV, sums of up to four products, one workgroup per
+//     block.
 //
 // Reference: scipy.linalg.lu_factor / lu_solve per fiber in
 // python/tstep/tstep_utils.py:1405-1419 and python/tstep/tstep.py:985-988;

@@ -447,19 +447,11 @@ int f3d_gemm_bf16(int epi, int64_t M, int64_t N, int64_t K, int32_t ksplit, cons
                   float alpha, void* stream);
 
 /*
- * The learned guess's net in -> width -> width -> out (ReLU; FP32 weights
- * W1 (n_in x width), W2 (width x width), W3 (width x n_out), row-major) over M
- * samples as whole passes, no reference counterpart.  X has strides (sxm, sxk);
- * H1, H2 (M x width) and Y (M x n_out) are row-major: the layers' outputs
- * after their ReLUs, and the net's output.  backward: the gradients of a loss
- * with dL/dY = dY (strides sym, syk), summed over the samples in a fixed
- * order; ws: f3d_mlp_workspace_size bytes.
- */
-/*
- * (continued) mse: loss[0] = mean (y - t)^2 over n values and dy =
- * 2 (y - t) / n (ws: f3d_mse_workspace_size bytes).  adam: step t (1-based) of
- * Adam on count tensors given by host arrays of sizes and device pointers,
- * parameters and moments updated in place.
+ * Mean squared error and its gradient: loss[0] = mean (y - t)^2 over n values and
+ * dy = 2 (y - t) / n (ws: f3d_mse_workspace_size bytes).  adam: step t (1-based) of
+ * Adam on count FP32 tensors given by host arrays of sizes and device pointers
+ * (no two may share memory), parameters and moments updated in place.  No
+ * reference counterpart.
  */
 size_t f3d_mse_workspace_size(void);
 int f3d_mse(int64_t n, const float* y, const float* t, float* dy, float* loss, void* ws,
@@ -467,6 +459,15 @@ int f3d_mse(int64_t n, const float* y, const float* t, float* dy, float* loss, v
 int f3d_adam(int32_t count, const int64_t* sizes, float* const* p, const float* const* g,
              float* const* m, float* const* v, double lr, double b1, double b2, double eps,
              int64_t t, void* stream);
+/*
+ * The learned guess's net in -> width -> width -> out (ReLU; FP32 weights
+ * W1 (n_in x width), W2 (width x width), W3 (width x n_out), row-major) over M
+ * samples as whole passes, no reference counterpart.  X has strides (sxm, sxk);
+ * H1, H2 (M x width) and Y (M x n_out) are row-major: the layers' outputs
+ * after their ReLUs, and the net's output; a bias may be NULL.  backward: the
+ * gradients of a loss with dL/dY = dY (strides sym, syk), summed over the
+ * samples in a fixed order (zero for M = 0); ws: f3d_mlp_workspace_size bytes.
+ */
 size_t f3d_mlp_workspace_size(int64_t M, int32_t n_in, int32_t width, int32_t n_out);
 int f3d_mlp_forward(int64_t M, int32_t n_in, int32_t width, int32_t n_out, const float* X,
                     int64_t sxm, int64_t sxk, const float* W1, const float* b1, const float* W2,
