@@ -22,7 +22,7 @@ import numpy as np
 import torch
 
 from . import _lib as L
-from .kernels import _stream
+from .kernels import _addr, _stream
 
 EPI_STORE, EPI_BIAS_RELU, EPI_RELU_GRAD, EPI_ATOMIC, EPI_BIAS = 0, 1, 2, 3, 4
 
@@ -88,7 +88,7 @@ class MLP:
         H1 = X.new_empty((M, self.width))
         H2 = torch.empty_like(H1)
         Y = X.new_empty((M, self.n_out))
-        p = L.ptr
+        p = _addr
         rc = L.load().f3d_mlp_forward(
             M, self.n_in, self.width, self.n_out, p(X), X.stride(0), X.stride(1), p(W1),
             p(b1), p(W2), p(b2), p(W3), p(b3), p(H1), p(H2), p(Y), _stream())
@@ -109,7 +109,7 @@ class MLP:
                  + [X.new_empty(s[1:]) for s in self.shapes])
         need = lib.f3d_mlp_workspace_size(M, self.n_in, self.width, self.n_out)
         ws = X.new_empty(-(-need // 4))
-        p = L.ptr
+        p = _addr
         rc = lib.f3d_mlp_backward(
             M, self.n_in, self.width, self.n_out, p(X), X.stride(0), X.stride(1), p(H1), p(H2),
             p(dY), dY.stride(0), dY.stride(1), p(W2), p(W3),
@@ -163,8 +163,8 @@ class MLP:
             loss = Y.new_empty(())
             need = lib.f3d_mse_workspace_size()
             ws = Y.new_empty(-(-need // 4))
-            rc = lib.f3d_mse(Y.numel(), L.ptr(Y), L.ptr(target), L.ptr(dY), L.ptr(loss), L.ptr(ws),
-                             need, _stream())
+            rc = lib.f3d_mse(Y.numel(), _addr(Y), _addr(target), _addr(dY), _addr(loss),
+                             _addr(ws), need, _stream())
             L.check(rc, "f3d_mse")
         else:
             # torch broadcasts and converts the target, or refuses it
