@@ -43,12 +43,17 @@ _tuned = False
 
 
 def _ensure_tuned():
-    """Install the saved launch-shape table (fiber3d_amd/tuning.json) once."""
+    """Install the saved launch-shape table (fiber3d_amd/tuning.json) once; other
+    threads' first sums wait for it."""
     global _tuned
     if not _tuned:
-        _tuned = True
-        from . import autotune
-        autotune.apply()
+        with _ws_lock:
+            if not _tuned:
+                from . import autotune
+                try:
+                    autotune.apply()
+                finally:
+                    _tuned = True
 
 
 # Workspace buffers replaced by a larger one stay allocated for the life of

@@ -119,3 +119,29 @@ def test_tuner_can_produce_the_saved_table():
         assert AT.fill_grid(grid) == {s: v for s, v in buckets.items() if s != "18/18"}
     assert t["lu"] == AT.LU_LAUNCH and "lu" not in AT.PARTS
     assert t["problem"] == AT.PROBLEM
+
+
+def test_the_first_sums_of_all_threads_wait_for_the_table(monkeypatch):
+    """Whichever thread's sum comes first installs the table; no other goes on before
+    it is there."""
+    import threading
+    import time
+    from fiber3d_amd import kernels as FK
+    installed, seen = [], []
+
+    def slow():
+        time.sleep(0.2)
+        installed.append(1)
+
+    def first_sum():
+        FK._ensure_tuned()
+        seen.append(len(installed))
+    monkeypatch.setattr(FK, "_tuned", False)
+    monkeypatch.setattr(AT, "apply", slow)
+    threads = [threading.Thread(target=first_sum) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert seen == [1, 1, 1, 1]
+    monkeypatch.undo()
