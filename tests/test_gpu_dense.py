@@ -373,3 +373,31 @@ def test_lu_solve_divides_by_pivots_beyond_the_reciprocal(n):
     lu.lu64.copy_(torch.from_numpy(np.diag(d).ravel()))
     y = lu.solve(torch.from_numpy(x).cuda()).cpu().numpy()
     np.testing.assert_array_equal(y, ref)
+
+
+@pytest.mark.parametrize("mmax,nb,said", [(32, 40, 32), (64, 40, 64), (64, 2051, 64), (128, 2051, 128),
+                                          (256, 2051, 256), (200, 40, 64), (200, 2051, 64),
+                                          (200, 2051, 100)])
+def test_block_gemv_of_many_blocks(mmax, nb, said):
+    """Few and many blocks of each size class, with rows and columns at the edges of
+    the waves' shares, and blocks taller than the call's mmax says; 260 eps of
+    the absolute sums."""
+    print(f"case block gemv many mmax={mmax} nb={nb} said={said}", flush=True)
+    rng = np.random.default_rng(nb + mmax + said)
+    ms = rng.choice([m for m in (1, 2, 31, 32, 33, 50, 63, 64, 65, 100, 127, 128, 129, 200, 256)
+                     if m <= mmax], nb)
+    ms[-1] = mmax
+    ks = rng.choice([0, 1, 7, 8, 9, 15, 16, 17, 31, 32, 33, 64, 65, 129], nb)
+    x_off, y_off = np.cumsum(ks) - ks, np.cumsum(ms) - ms
+    mats = [rng.normal(size=(m, k)) for m, k in zip(ms, ks)]
+    g = BlockGemv(ms, ks, x_off, y_off)
+    g.mmax = said
+    x, y0 = rng.normal(size=int(ks.sum()) + 1), rng.normal(size=int(ms.sum()))
+    y = torch.from_numpy(y0.copy()).cuda()
+    g(g.pack(mats), torch.from_numpy(x).cuda(), y, alpha=0.75, beta=-0.5)
+    got = y.cpu().numpy()
+    for M, xo, yo in zip(mats, x_off, y_off):
+        m, k = M.shape
+        xb, yb = x[xo:xo + k], y0[yo:yo + m]
+        scale = 0.75 * (np.abs(M) @ np.abs(xb)) + 0.5 * np.abs(yb)
+        assert (np.abs(got[yo:yo + m] - (0.75 * (M @ xb) - 0.5 * yb)) <= 260 * 2.3e-16 * scale).all()
