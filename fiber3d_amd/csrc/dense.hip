@@ -1076,7 +1076,7 @@ dense_gemv_kernel(int64_t waves_total, int32_t m, int32_t groups, int vec,
   }
 }
 
-int launch_lu_block(int precision, int64_t nb, const int32_t* n, const int64_t* a_off,
+int launch_lu_block(int precision, int64_t nb, int32_t nmax, const int32_t* n, const int64_t* a_off,
                     const int64_t* x_off, const int32_t* order, const double* A, double* lu64,
                     float* lu32, double* rs, double* cs, int32_t* piv, int32_t* perm,
                     int32_t* info, hipStream_t st);
@@ -1109,7 +1109,7 @@ extern "C" int f3d_lu_factor_batched(int precision, int64_t nb, int32_t nmax, co
     } else {
       F3D_REQUIRE(lu32 && rs && cs, F3D_EINVAL, "lu_factor: lu32/rs/cs is NULL");
     }
-    return launch_lu_block(precision, nb, n, a_off, x_off, order, A, lu64, lu32, rs, cs, piv,
+    return launch_lu_block(precision, nb, nmax, n, a_off, x_off, order, A, lu64, lu32, rs, cs, piv,
                            perm, info, st);
   }
   const unsigned grid = (unsigned)(nb < num_cus() ? nb : num_cus());

@@ -47,9 +47,6 @@ namespace f3d {
 
 constexpr int kWp = 16;     // panel width = MFMA tile edge
 constexpr int kWmax = 256;  // largest order
-// LDS column stride of a strip: 16 columns x 4 rows (an MFMA operand) and 64
-// rows of a column both spread over all banks
-constexpr int kWs = kWmax + 4;
 
 template <typename T>
 struct Mf16;
@@ -176,18 +173,22 @@ struct alignas(16) LuCand {
   T inv, u1;
 };
 
-template <typename T, int W>
+// For blocks of order up to NM.
+template <typename T, int W, int NM>
 struct LuShared {
+  // LDS column stride of a strip: 16 columns x 4 rows (an MFMA operand) and 64
+  // rows of a column both spread over all banks
+  static constexpr int kWs = NM + 4;
   T s[W * kWs];                       // the strip, column c at c * kWs + row
   LuCand<T> cand[2][4];
   T crow[2][4][kWp];                  // the candidates' rows
-  double srow[sizeof(T) == 4 ? kWmax : 1];  // FP32: row scales
+  double srow[sizeof(T) == 4 ? NM : 1];     // FP32: row scales
   double scol[sizeof(T) == 4 ? kWp : 1];    // FP32: column scales of 16 columns
-  unsigned char perm[kWmax];          // row of A now at a position
-  unsigned char pos[kWmax];           // position of a row of the strip
-  unsigned char piv[kWmax];           // interchange of every column
+  unsigned char perm[NM];             // row of A now at a position
+  unsigned char pos[NM];              // position of a row of the strip
+  unsigned char piv[NM];              // interchange of every column
   unsigned char prow[kWp];            // the panel's pivot rows
-  unsigned char pend[kWmax / W][kWmax];  // position of a row of A at a strip's end
+  unsigned char pend[NM / W][NM];     // position of a row of A at a strip's end
 };
 
 // x <- L_kk^-1 x for R columns per lane: lane e16 of a 16-lane row holds row
@@ -219,8 +220,8 @@ __device__ __forceinline__ double rl(double v, int w) {
   return __longlong_as_double(((unsigned long long)hi << 32) | lo);
 }
 
-template <typename T, int W>
-__device__ __forceinline__ void lu_block_body(LuShared<T, W>& sh, const int* __restrict__ n_arr,
+template <typename T, int W, int NM>
+__device__ __forceinline__ void lu_block_body(LuShared<T, W, NM>& sh, const int* __restrict__ n_arr,
                                               const long* __restrict__ a_off,
                                               const long* __restrict__ x_off,
                                               const int* __restrict__ order,
@@ -231,12 +232,14 @@ __device__ __forceinline__ void lu_block_body(LuShared<T, W>& sh, const int* __r
   typedef typename Mf16<T>::v4 v4;
   constexpr bool kEq = sizeof(T) == 4;  // FP32: equilibrate
   constexpr int kCt = W / kWp;          // column tiles
+  constexpr int kWs = LuShared<T, W, NM>::kWs;
   const int tid = threadIdx.x, lane = tid & 63;
+  const bool row = NM == kWmax || tid < NM;  // whether this thread has a row
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, e16 = lane & 15;
   const int b = order ? order[blockIdx.x] : (int)blockIdx.x;
   const int n = n_arr[b];
-  if (n < 1 || n > kWmax) {  // uniform per workgroup
+  if (n < 1 || n > NM) {  // uniform per workgroup
     if (tid == 0) info[b] = -1;
     return;
   }
@@ -247,7 +250,7 @@ __device__ __forceinline__ void lu_block_body(LuShared<T, W>& sh, const int* __r
   const long xo = x_off[b];
   int first_zero = 0;
 
-  sh.perm[tid] = (unsigned char)tid;
+  if (row) sh.perm[tid] = (unsigned char)tid;
   double sr = 1.0;
   if constexpr (kEq) {
     // row maxima, one thread per row
@@ -260,13 +263,13 @@ __device__ __forceinline__ void lu_block_body(LuShared<T, W>& sh, const int* __r
       for (int u = 0; u < 16; ++u) mx = fmax(mx, fabs(v[u]));
     }
     sr = tid < n ? pow2_scale_w(mx) : 1.0;
-    sh.srow[tid] = sr;
+    if (row) sh.srow[tid] = sr;
   }
   __syncthreads();
 
   for (int C0 = 0; C0 < npad; C0 += W) {
     const int ctn = min(kCt, (npad - C0) / kWp);  // column tiles of this strip
-    const int phys = sh.perm[tid];                // row of A of this thread's row
+    const int phys = row ? sh.perm[tid] : tid;    // row of A of this thread's row
     // ---- the strip, rows in the order of the positions so far -------------------
     for (int h0 = 0; h0 < 16 * ctn; h0 += 16) {
       double v[16];
@@ -286,7 +289,7 @@ __device__ __forceinline__ void lu_block_body(LuShared<T, W>& sh, const int* __r
           v[c] *= sp;
           const unsigned h =
               (unsigned)((unsigned long long)__double_as_longlong(v[c]) >> 32) & 0x7fffffffu;
-          hi[c * kWs + tid] = v[c] == v[c] ? h : 0u;
+          if (row) hi[c * kWs + tid] = v[c] == v[c] ? h : 0u;
         }
         lds_barrier();
         const int c = tid >> 4, t0 = tid & 15;  // 16 threads per column
@@ -312,17 +315,19 @@ __device__ __forceinline__ void lu_block_body(LuShared<T, W>& sh, const int* __r
         }
         lds_barrier();
 #pragma unroll
-        for (int c = 0; c < 16; ++c) dst[c * kWs] = (T)(v[c] * sh.scol[kEq ? c : 0]);
+        for (int c = 0; c < 16; ++c)
+          if (row) dst[c * kWs] = (T)(v[c] * sh.scol[kEq ? c : 0]);
       } else {
 #pragma unroll
-        for (int c = 0; c < 16; ++c) dst[c * kWs] = (T)v[c];
+        for (int c = 0; c < 16; ++c)
+          if (row) dst[c * kWs] = (T)v[c];
       }
       if (npad != n) {
         // the identity outside the real rows and columns
 #pragma unroll
         for (int c = 0; c < 16; ++c) {
           const int C = C0 + h0 + c;
-          if (phys >= n || C >= n) dst[c * kWs] = phys == C ? (T)1 : (T)0;
+          if (row && (phys >= n || C >= n)) dst[c * kWs] = phys == C ? (T)1 : (T)0;
         }
       }
     }
@@ -414,7 +419,7 @@ __device__ __forceinline__ void lu_block_body(LuShared<T, W>& sh, const int* __r
       T* __restrict__ panel = sh.s + 16 * ss * kWs;
       T a[kWp];
 #pragma unroll
-      for (int c = 0; c < kWp; ++c) a[c] = panel[c * kWs + tid];
+      for (int c = 0; c < kWp; ++c) a[c] = row ? panel[c * kWs + tid] : (T)0;
       bool live = mine && pos >= c0;
       int vat = 0;  // lane j: column j's pivot row | position << 16
       sfor<0, kWp>([&](auto J) __attribute__((always_inline)) {
@@ -561,7 +566,7 @@ __device__ __forceinline__ void lu_block_body(LuShared<T, W>& sh, const int* __r
   }
 
   // ---- rows of L that later strips moved ----------------------------------------
-  const int phys = sh.perm[tid];
+  const int phys = row ? sh.perm[tid] : tid;
   for (int C0 = 0; C0 + W < npad; C0 += W) {
     const bool low = tid >= C0 + W && tid < n;
     const int old = low ? min((int)sh.pend[C0 / W][phys], n - 1) : tid;
@@ -595,15 +600,21 @@ __device__ __forceinline__ void lu_block_body(LuShared<T, W>& sh, const int* __r
 // blocks per CU: 2.19).  One wavefront per block and a right-looking update in
 // memory took 1.85 and 7.3 ms; A read twice (FP32: row maxima first) and the
 // factor written once would take 0.15 and 1.1 ms at a large copy's rate.
+// FP64 blocks of order up to 64, where two per CU are not all of them, have strips
+// of 64 rows (19 KB) and four blocks per CU, with 128 registers: 3000 blocks of order 36
+// 259 -> 183 us, 64 325 -> 227 (one wavefront per block 226 and 325); but 512 of order
+// 48 45 -> 52, so fewer stay.  (FP32 has four per CU as it is: 3000 of order 36, 152
+// against 158.)
 constexpr int kLuW64 = 32, kLuW32 = 32;
 
-__global__ void __launch_bounds__(256, 2)
+template <int NM>
+__global__ void __launch_bounds__(256, NM == 64 ? 4 : 2)
 lu_block_f64_kernel(const int* __restrict__ n_arr, const long* __restrict__ a_off,
                     const long* __restrict__ x_off, const int* __restrict__ order,
                     const double* __restrict__ A, double* __restrict__ LU, int* __restrict__ piv,
                     int* __restrict__ perm, int* __restrict__ info) {
-  __shared__ LuShared<double, kLuW64> sh;
-  lu_block_body<double, kLuW64>(sh, n_arr, a_off, x_off, order, A, LU, nullptr, nullptr, piv, perm, info);
+  __shared__ LuShared<double, kLuW64, NM> sh;
+  lu_block_body<double, kLuW64, NM>(sh, n_arr, a_off, x_off, order, A, LU, nullptr, nullptr, piv, perm, info);
 }
 __global__ void __launch_bounds__(256, 4)
 lu_block_f32_kernel(const int* __restrict__ n_arr, const long* __restrict__ a_off,
@@ -611,21 +622,25 @@ lu_block_f32_kernel(const int* __restrict__ n_arr, const long* __restrict__ a_of
                     const double* __restrict__ A, float* __restrict__ LU, double* __restrict__ rs,
                     double* __restrict__ cs, int* __restrict__ piv, int* __restrict__ perm,
                     int* __restrict__ info) {
-  __shared__ LuShared<float, kLuW32> sh;
-  lu_block_body<float, kLuW32>(sh, n_arr, a_off, x_off, order, A, LU, rs, cs, piv, perm, info);
+  __shared__ LuShared<float, kLuW32, kWmax> sh;
+  lu_block_body<float, kLuW32, kWmax>(sh, n_arr, a_off, x_off, order, A, LU, rs, cs, piv, perm, info);
 }
 
-int launch_lu_block(int precision, int64_t nb, const int32_t* n, const int64_t* a_off,
+int launch_lu_block(int precision, int64_t nb, int32_t nmax, const int32_t* n, const int64_t* a_off,
                     const int64_t* x_off, const int32_t* order, const double* A, double* lu64,
                     float* lu32, double* rs, double* cs, int32_t* piv, int32_t* perm,
                     int32_t* info, hipStream_t st) {
-  if (precision == F3D_F64) {
-    F3D_LAUNCH(lu_block_f64_kernel, dim3((unsigned)nb), dim3(256), 0, st, n, (const long*)a_off,
-               (const long*)x_off, order, A, lu64, piv, perm, info);
+#define F3D_LB(K, ...)                                                                         \
+  F3D_LAUNCH(K, dim3((unsigned)nb), dim3(256), 0, st, n, (const long*)a_off, (const long*)x_off, \
+             order, A, __VA_ARGS__, piv, perm, info)
+  if (precision == F3D_F32C) {
+    F3D_LB(lu_block_f32_kernel, lu32, rs, cs);
+  } else if (nmax <= 64 && nb > 2 * (int64_t)num_cus()) {
+    F3D_LB(lu_block_f64_kernel<64>, lu64);
   } else {
-    F3D_LAUNCH(lu_block_f32_kernel, dim3((unsigned)nb), dim3(256), 0, st, n, (const long*)a_off,
-               (const long*)x_off, order, A, lu32, rs, cs, piv, perm, info);
+    F3D_LB(lu_block_f64_kernel<kWmax>, lu64);
   }
+#undef F3D_LB
   return F3D_OK;
 }
 

@@ -254,14 +254,15 @@ int f3d_stresslet_matrix(int64_t n, const double* pos, const double* nrm, int64_
 /*
  * A batch of `nb` square blocks; block b has order n[b] <= 256 and is stored
  * column-major at A + a_off[b] (leading dimension n[b]).  n, a_off, x_off and
- * order are DEVICE arrays (int32, int64, int64, int32).  `order` (nullable)
- * lists the blocks in the sequence the persistent workgroups pick them up
- * (largest first balances uneven sizes); NULL means 0..nb-1.
+ * order are DEVICE arrays (int32, int64, int64, int32); nmax is the largest
+ * n[b].  `order` (nullable)
+ * lists the blocks in the sequence the workgroups take them (largest first
+ * balances uneven sizes); NULL means 0..nb-1.
  *
  * f3d_lu_factor_batched replaces tstep_utils.build_block_diagonal_lu_
  * preconditioner_fiber (python/tstep/tstep_utils.py:1405-1419), i.e.
  * scipy.linalg.lu_factor (LAPACK dgetrf, partial pivoting, first maximal
- * |pivot| wins ties) per fiber, in ONE persistent launch.
+ * |pivot| wins ties) per fiber, in ONE launch.
  *   precision F3D_F64: A is factored in FP64 into lu64 (offsets a_off).
  *   precision F3D_F32C: A is first equilibrated by powers of two,
  *     As = diag(rs) A diag(cs), then factored in FP32 into lu32 (offsets

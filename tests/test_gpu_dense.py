@@ -401,3 +401,37 @@ def test_block_gemv_of_many_blocks(mmax, nb, said):
         xb, yb = x[xo:xo + k], y0[yo:yo + m]
         scale = 0.75 * (np.abs(M) @ np.abs(xb)) + 0.5 * np.abs(yb)
         assert (np.abs(got[yo:yo + m] - (0.75 * (M @ xb) - 0.5 * yb)) <= 260 * 2.3e-16 * scale).all()
+
+
+def test_lu_factor_of_many_small_blocks():
+    """Many blocks of order up to 64 take strips of 64 rows: the same factors,
+    interchanges and zero pivots as in small batches, to the bit, with ties, zero
+    columns, NaN and every order mixed."""
+    print("case lu many small blocks", flush=True)
+    rng = np.random.default_rng(77)
+    sizes = [int(n) for n in rng.integers(1, 65, 1100)]
+    sizes[:8] = [1, 15, 16, 17, 32, 33, 63, 64]
+    mats = []
+    for k, n in enumerate(sizes):
+        M = rng.normal(size=(n, n))
+        if k % 5 == 1:
+            M = rng.integers(-1, 2, size=(n, n)).astype(float)  # ties, some singular
+        elif k % 5 == 2:
+            M[:, n // 2] = 0.0
+        elif k % 50 == 3:
+            M[n // 3, n // 2] = np.nan
+        mats.append(M)
+    bs = BlockSet(sizes)
+    lu = BatchedLU(bs, bs.pack(mats), precision="f64", refine=0)
+    LU, piv = bs.unpack(lu.lu64), lu.piv.cpu().numpy()
+    perm, info = lu.perm.cpu().numpy(), lu.info.cpu().numpy()
+    for k0 in range(0, len(sizes), 400):
+        part = slice(k0, k0 + 400)
+        b2 = BlockSet(sizes[part])
+        l2 = BatchedLU(b2, b2.pack(mats[part]), precision="f64", refine=0)
+        rows = slice(int(bs.x_off_h[k0]), int(bs.x_off_h[k0]) + b2.nrows)
+        for a, b in zip(LU[part], b2.unpack(l2.lu64)):
+            np.testing.assert_array_equal(a, b)
+        np.testing.assert_array_equal(piv[rows], l2.piv.cpu().numpy())
+        np.testing.assert_array_equal(perm[rows], l2.perm.cpu().numpy())
+        np.testing.assert_array_equal(info[part], l2.info.cpu().numpy())
