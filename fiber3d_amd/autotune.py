@@ -212,6 +212,19 @@ def tune_pairsum(kernels=("oseen", "stresslet", "rotlet"), precisions=("f32c", "
 
     rng = np.random.default_rng(seed)
     nmax = max(GRID_NT + GRID_NS)
+    direct = os.environ.get("F3D_PAIRSUM_DIRECT")
+    # (the shapes are the general path's, also at sizes that the direct kernel takes)
+    os.environ["F3D_PAIRSUM_DIRECT"] = "0"
+    try:
+        return _tune_pairsum(torch, pairsum, rng, nmax, kernels, precisions, ks, log)
+    finally:
+        if direct is None:
+            del os.environ["F3D_PAIRSUM_DIRECT"]
+        else:
+            os.environ["F3D_PAIRSUM_DIRECT"] = direct
+
+
+def _tune_pairsum(torch, pairsum, rng, nmax, kernels, precisions, ks, log):
     X = torch.from_numpy(rng.uniform(0, 1, (nmax, 3))).cuda()
     F = torch.from_numpy(rng.normal(size=(nmax, 3))).cuda()
     NR = torch.nn.functional.normalize(torch.from_numpy(rng.normal(size=(nmax, 3))), dim=1).cuda()

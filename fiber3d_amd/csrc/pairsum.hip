@@ -1242,7 +1242,7 @@ struct Plan {
   int G;      // chunks per block (waves of a block, combined in LDS)
   int Pg;     // partial sums per target: ceil(P / G)
   int sort;   // sources and targets in spatial order
-  int forced; // shape set by the environment: no direct kernel
+  int forced; // by the environment: a shape of its own, or no direct kernel
 };
 
 static void set_groups(Plan& pl) {
@@ -1300,7 +1300,7 @@ static Plan make_plan(int kernel, int precision, int64_t ns, int64_t nt) {
   pl.K = env_int(precision == F3D_F64 ? "F3D_PAIRSUM_K64" : "F3D_PAIRSUM_K32", k0);
   if (pl.K != 1 && pl.K != 2 && pl.K != 4) pl.K = 2;
   pl.forced = env_int(precision == F3D_F64 ? "F3D_PAIRSUM_K64" : "F3D_PAIRSUM_K32", 0) != 0 ||
-              env_int("F3D_PAIRSUM_WAVES", 0) != 0;
+              env_int("F3D_PAIRSUM_WAVES", 0) != 0 || env_int("F3D_PAIRSUM_DIRECT", 1) == 0;
   pl.ns_pad = (int)align_up((size_t)(ns > 0 ? ns : 1), kTile);
   const int64_t waves_per_split = ceil_div(nt > 0 ? nt : 1, 64 * pl.K);
   int target_waves = env_int("F3D_PAIRSUM_WAVES", w0);
