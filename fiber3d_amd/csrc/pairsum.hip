@@ -1391,14 +1391,19 @@ static Plan make_plan_within(int kernel, int precision, int64_t ns, int64_t nt, 
 // Shape of pairsum_direct_kernel for a call (targets per lane, log2 of the
 // target lanes), or k = 0: the call takes the general path.
 //
-// The line: a workgroup reads all sources, so its share of them (ns / slices)
-// and the call's reads of LDS grow with ns, while the general path's scalar
-// records cost the same for every target.  Measured, general against direct,
-// us (FP64 Oseen; stresslet): 1024 x 1024 19.6 / 5.9 (19.4 / 6.5), 4096 sources
-// x 256 20.2 / 10.8 (20.1 / 13.9), 4096 x 4096 30.4 / 26.3 (32.0 / 30.7), 2048
-// x 16384 45.2 / 36.4 (46.6 / 42.6), 512 x 65536 39.1 / 32.8 (41.7 / 39.0);
-// past the line 8192 x 4096 46.3 / 47.3 (49.2 / 56.4), 1024 x 262144 222 / 227
-// (253 / 253), 8192 x 256 21.4 / 18.9 (21.2 / 25.0).
+// The line: both paths' times are estimated, and the call takes the direct
+// kernel where its estimate is no larger.  A workgroup of per = k << lg targets
+// reads all sources, and the last turn of the CUs costs as much as a full one:
+//   direct   3.2 us + turns per ns (a + b / per) ps, a = 222 (stresslet 250),
+//            b = 910 (1260): the share of the LDS reads shrinks with per;
+//   general  15 us + 0.565 (0.67) ps a pair + 20 ps a target: three launches.
+// Measured, general against direct, us (FP64 Oseen; stresslet): 1024 x 1024
+// 16.4 / 5.5 (16.1 / 6.4), 4096 sources x 256 17.0 / 11.5 (16.8 / 14.3), 4096 x
+// 2000 17.5 / 17.8 (17.5 / 22.7), 4096 x 5000 27.0 / 39.9 (28.1 / 46.1), 3000 x
+// 9000 34.4 / 50.6 (36.1 / 57.3), 512 x 40000 24.4 / 32.9 (25.6 / 36.5), 128 x
+// 200000 33.1 / 28.6 (34.7 / 31.4).  Of 600 calls with 16 to 4096 sources the
+// chosen path takes at most 1.1 times the other's time.  Past 4096 sources or
+// 2^25 pairs the general path is the faster (8192 x 4096 36.6 / 47.3).
 //
 // Within it: 256 to 512 workgroups (two per CU), with at least four target
 // lanes once every CU has a workgroup (fewer distinct LDS reads per wave); two
@@ -1409,12 +1414,19 @@ constexpr int64_t kDirectPairs = 1ll << 25;
 struct DirectShape {
   int k, lg;
 };
-static DirectShape direct_shape(const Plan& pl, int64_t ns, int64_t nt) {
+static DirectShape direct_shape(const Plan& pl, int kind, int64_t ns, int64_t nt) {
   if (pl.forced || pl.sort || ns > kDirectSources || ns * nt > kDirectPairs) return {0, 0};
   DirectShape d{nt > 2048 ? 2 : 1, 0};
   while (d.lg < 6 && (nt > ((int64_t)512 * d.k << d.lg) || (d.lg < 2 && nt > (int64_t)256 << d.lg)))
     ++d.lg;
-  return d;
+  const bool stresslet = kind == F3D_STRESSLET;
+  const int per = d.k << d.lg;
+  const double turns = (double)ceil_div(ceil_div(nt, (int64_t)per), (int64_t)num_cus());
+  const double direct = 3.2e6 + turns * per * (double)ns *
+                                    (stresslet ? 250.0 + 1260.0 / per : 222.0 + 910.0 / per);
+  const double general =
+      15e6 + (stresslet ? 0.67 : 0.565) * (double)(ns * nt) + 20.0 * (double)nt;
+  return direct <= general ? d : DirectShape{0, 0};
 }
 
 // Whether the output overlaps an input: the direct kernel's workgroups read
@@ -1442,7 +1454,7 @@ static int launch_pairsum(const Plan& pl, uint32_t flags, int64_t ns, const Sour
   factor *= TwoOverR<T, KIND>::scale;
   const bool timed = g_timer.on && g_timer.n < kTimerSlots;
   if constexpr (!kQuant) {
-    const DirectShape d = direct_shape(pl, ns, nt);
+    const DirectShape d = direct_shape(pl, KIND, ns, nt);
     if (d.k > 0 && !direct_aliases(ns, src, nt, tpos, t_sp, t_sc, lo, hi, out, o_sp, o_sc)) {
       if (timed) F3D_HIP_CHECK(hipEventRecord(g_timer.ev[2 * g_timer.n], st));
       const dim3 grid((unsigned)ceil_div(nt, (int64_t)d.k << d.lg));

@@ -243,6 +243,26 @@ def test_one_launch_sums_match_the_general_path(kernel, ns, nt, monkeypatch):
             assert rel2(got, ref) < tol, form
 
 
+@pytest.mark.parametrize("kernel", ["oseen", "rotlet", "stresslet"])
+@pytest.mark.parametrize("ns,nt,one", [(4096, 2048, True), (4096, 5000, False),
+                                       (3000, 9000, False), (512, 40000, False),
+                                       (128, 200000, True), (4097, 2048, False)])
+def test_one_launch_sums_stop_where_their_last_turn_is_short(kernel, ns, nt, one, monkeypatch):
+    """A second turn of the CUs for a few workgroups makes the one launch the
+    slower path (4096 x 5000: 40 against 27 us): such a call takes the general
+    path, bit for bit; the others agree with it (64 x 1e-14, as above).  The
+    stresslet's line lies lower: 22.7 against 17.5 us at 4096 x 2000."""
+    s, t, d, n = (_dev(a) for a in _problem(ns + nt, ns, nt))
+    call = lambda: FK.pairsum(kernel, s, d, t, src_nrm=n, eta=0.7).cpu().numpy()
+    got = call()
+    monkeypatch.setenv("F3D_PAIRSUM_DIRECT", "0")
+    ref = call()
+    if (kernel, ns) == ("stresslet", 4096):
+        one = False
+    assert np.array_equal(got, ref) != one
+    assert rel2(got, ref) < 64 * 1e-14
+
+
 @pytest.mark.parametrize("n", [258, 1400])
 def test_one_launch_shell_matches_the_general_path(n, monkeypatch):
     """The shell operator's epilogue (singularity subtraction, completion sum,
