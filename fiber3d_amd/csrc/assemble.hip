@@ -115,8 +115,15 @@ fiber_deriv_kernel(int nfib, int N, int rows, const long* __restrict__ node0,
 // 12 points); later ones, of a denser D, are read from memory.
 constexpr int kBandSteps = 10;
 
+// Workgroups that fit a CU (registers: 141 of 16 nodes, 203 of 32, 242 of 64).  A
+// fiber of up to 16 nodes is one tile with four steps; in the form of 32 nodes
+// half of its products and registers were padding: 9 nodes, 3000 fibers 73.6 ->
+// 51.3 us, 256 fibers 16.8 -> 13.5, one 12.8 -> 10.1 (whole assembly).  A fourth
+// workgroup spills: 48.0, 14.5, 10.1.
+constexpr int asm_per_cu(int nmax) { return nmax <= 16 ? 3 : 2; }
+
 template <int NMAX>
-__global__ void __launch_bounds__(kAsmThreads, 2)
+__global__ void __launch_bounds__(kAsmThreads, asm_per_cu(NMAX))
 fiber_assemble_kernel(int nfib, int N, const long* __restrict__ node0,
                       const double* __restrict__ length, const long* __restrict__ a_off,
                       const long* __restrict__ f_off, const long* __restrict__ q_off,
@@ -277,7 +284,7 @@ fiber_assemble_kernel(int nfib, int N, const long* __restrict__ node0,
       }
       // element e of lane (g, c16): row 16 rt + c16 of column 16 jt + 4 e + g.
       // The row tiles trade 16-lane rows, so that a store covers all rows of
-      // one column (NMAX 64) or of two (32) instead of 16 rows of four.
+      // one column (NMAX 64) or of two (32) instead of 16 rows of four (16).
       double* __restrict__ dst;
       int col_stride;
       if (a < 4) {
@@ -298,14 +305,15 @@ fiber_assemble_kernel(int nfib, int N, const long* __restrict__ node0,
           swap_rows<32>(col[1], col[3]);
           swap_rows<16>(col[0], col[1]);
           swap_rows<16>(col[2], col[3]);
-        } else {
+        } else if constexpr (RT == 2) {
           swap_rows<16>(col[0], col[1]);
         }
 #pragma unroll
         for (int q = 0; q < RT; ++q) {
-          // RT 4: column q, row lane; RT 2: columns q and q + 2, row lane % 32
-          const int r = RT == 4 ? lane : (lane & 31);
-          const int jc = 16 * jt + 4 * e + (RT == 4 ? q : q + 2 * (lane >> 5));
+          // RT 4: column q, row lane; RT 2: columns q and q + 2, row lane % 32;
+          // RT 1: columns 0 .. 3, row lane % 16
+          const int r = lane & (NMAX - 1);
+          const int jc = 16 * jt + 4 * e + q + RT * (lane / NMAX);
           if (r < rows && jc < N) dst[jc * col_stride + r] = col[q];
         }
       }
@@ -557,8 +565,8 @@ extern "C" int f3d_fiber_assemble(int64_t nfib, int32_t N, const int64_t* node0,
                   F_out && Q0 && Q1 && Q2 && xs_out && xss_out && w_out,
               F3D_EINVAL, "fiber_assemble: NULL argument");
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  // persistent: two workgroups fit a CU
-  const int64_t most = 2 * (int64_t)num_cus();
+  // persistent: as many workgroups as fit a CU
+  const int64_t most = asm_per_cu(N <= 16 ? 16 : kAsmNmax) * (int64_t)num_cus();
   const unsigned grid = (unsigned)(nfib < most ? nfib : most);
   const unsigned fgrid = (unsigned)(nfib < 4 * most ? nfib : 4 * most);
   const int64_t dwaves = ceil_div(3 * nfib, (int64_t)64);
@@ -577,7 +585,9 @@ extern "C" int f3d_fiber_assemble(int64_t nfib, int32_t N, const int64_t* node0,
   F3D_LAUNCH(fiber_force_kernel<NM>, dim3(fgrid), dim3(256), 0, st, (int)nfib, (int)N,          \
              (const long*)node0, length, (const long*)f_off, D0, (const double*)xs_out,         \
              (const double*)xss_out, E, F_out)
-  if (N <= 32) {
+  if (N <= 16) {
+    F3D_ASM(16);
+  } else if (N <= 32) {
     F3D_ASM(32);
   } else {
     F3D_ASM(64);

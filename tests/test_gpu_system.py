@@ -235,6 +235,15 @@ def test_hip_assembly_at_tile_edges(N, nfib, dense):
     assert rel2(t(hip.rhs), t(ref.rhs)) < 1e-12
 
 
+@pytest.mark.parametrize("N,nfib,dense", [(8, 3, False), (8, 900, False), (9, 1, True),
+                                          (9, 300, False), (13, 200, True), (15, 2, False),
+                                          (16, 1601, False)])
+def test_hip_assembly_of_short_fibers(N, nfib, dense):
+    """Up to 16 nodes: the kernels of one row tile, with one, two and four
+    workgroups per fiber and with more fibers than workgroups."""
+    test_hip_assembly_at_tile_edges(N, nfib, dense)
+
+
 def test_ellipsoidal_periphery_matches_oracle():
     """An ellipsoidal shell (semi-axes 3, 2.5, 2; 900 nodes) around 12
     fibers: right-hand side, operator in FP64 and FP32-compensated,
