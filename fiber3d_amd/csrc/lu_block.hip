@@ -38,7 +38,8 @@
 // column; the solves refine in FP64 against the unscaled FP64 matrix.
 // Orders that are not a multiple of 16 are padded with an identity block that
 // is never stored: padded rows and columns stay decoupled from the real ones,
-// so the real factors are exactly those of the unpadded matrix.
+// so the real factors are exactly those of the unpadded matrix (the steps of
+// padded columns are skipped).
 #include "common.h"
 
 #include <type_traits>
@@ -426,6 +427,9 @@ __device__ __forceinline__ void lu_block_body(LuShared<T, W, NM>& sh, const int*
         constexpr int j = decltype(J)::value;
         constexpr int buf = j & 1;
         const int c = c0 + j;
+        // (a padded column changes nothing that is stored: 3000 FP64 blocks of order
+        // 4 56.7 -> 33.0 us, of order 68 465 -> 421)
+        if (c >= n) return;
         // (a padded row pivots padded columns only)
         const unsigned kh = live && (phys < n) == (c < n) ? abs_key(a[j]) : 0u;
         // (off the chain: every row's own reciprocal while the wave searches)
