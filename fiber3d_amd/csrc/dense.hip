@@ -852,29 +852,34 @@ lu_solve_kernel(const int* __restrict__ n_arr, const long* __restrict__ a_off,
 
 // ---------------------------------------------------------------------------
 // y_b = sum over terms of alpha M_b x_b, plus beta y_b; M_b column-major m x k, m
-// <= 64 kSlots: a workgroup of W waves per block, all terms in one launch
+// <= 64 kSlots: a workgroup of four waves per block, all terms in one launch
 // (a fiber's rows of the operator have four: A and the three Q_c; in launches
 // of their own these took 22 + 3 x 7.5 us for 1000 fibers of 32 nodes, here
 // 40.9, and 6 + 3 x 4.6 us for 32 fibers, here 9.2).  A lane has row lane of each 64-row
 // segment (R 64), or, for m <= 32, row lane % 32 of every other column (R 32).
-// The waves take groups of columns in turn, UL loads of a lane in flight; their
-// sums meet in LDS in a fixed order.
+// The waves take groups of 16 loads in turn; their sums meet in LDS in a fixed
+// order, the same for every launch form (the force rows cancel by 1e6 and more, so
+// another order moves a step's densities by up to 1e-8).
 // Bound by the loads of M: by HBM where the blocks fill the chip, by the chain
-// of one wave's column groups where they do not, which four waves shorten.
+// of one wave's column groups where they do not, which the four waves shorten.
 // Measured, against one wave per block and four columns in flight: 1000 blocks
 // of 128 x 128 21.9 us (6.0 TB/s) for 32, 3000 of 32 x 128 17.7 for 23, 32
 // blocks of 128 x 128 6.1 us for 18, of 114 x 32 3.9 for 10.
-// Many small blocks are bound by the waves' start instead, and four waves have
-// nothing to do in a few columns: 4096 blocks of 50 x 16 took 11.1 us with four
-// waves and 16 loads, 8.3 with 8 loads (84 registers for 122), 5.7 with one wave.
+// Many small blocks are bound by the waves' start instead: 4096 blocks of 50 x 16
+// took 10.8 us with 16 loads in flight and the sums of four terms' groups in LDS, 8.2
+// with 8 loads (57 registers for 116) and 2 KB; one wave a block 6.6, but then 64 x 64
+// 23.1 for 21.7.
+constexpr int kGemvThreads = 256;
 
-// acc += alpha M x for the lane's rows from r0 on
-template <int R, int SL, int UL, int W>
+// acc += alpha M x for the lane's rows from r0 on, over every fourth group of 16 /
+// SL steps, from the group `part`
+template <int R, int SL, int UL>
 __device__ __forceinline__ void block_gemv_cols(const double* __restrict__ M,
                                                 const double* __restrict__ x, int m, int kk,
-                                                double alpha, int r0, int wv, int lane,
+                                                double alpha, int r0, int part, int lane,
                                                 double (&acc)[SL]) {
   constexpr int C = 64 / R;    // columns side by side in a wave
+  constexpr int G = 16 / SL;   // steps of a column group
   constexpr int U = UL / SL;   // steps whose loads are in flight together
   const int sub = R == 64 ? 0 : lane / R;
   int row[SL];
@@ -884,20 +889,25 @@ __device__ __forceinline__ void block_gemv_cols(const double* __restrict__ M,
     sum[s] = 0.0;
     row[s] = min(r0 + lane % R + 64 * s, m - 1);
   }
-  for (int j0 = wv * (U * C); j0 < kk; j0 += W * U * C) {
-    double v[U][SL], xv[U];
+  for (int jg = part * (G * C); jg < kk; jg += 4 * G * C) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int j = j0 + u * C + sub, jc = min(j, kk - 1);
-      xv[u] = x[jc];
+    for (int q = 0; q < G / U; ++q) {
+      const int j0 = jg + q * (U * C);
+      if (q > 0 && j0 >= kk) break;
+      double v[U][SL], xv[U];
 #pragma unroll
-      for (int s = 0; s < SL; ++s) v[u][s] = M[(long)jc * m + row[s]];
-    }
+      for (int u = 0; u < U; ++u) {
+        const int j = j0 + u * C + sub, jc = min(j, kk - 1);
+        xv[u] = x[jc];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const bool in = j0 + u * C + sub < kk;  // past the end: adds nothing
+        for (int s = 0; s < SL; ++s) v[u][s] = M[(long)jc * m + row[s]];
+      }
 #pragma unroll
-      for (int s = 0; s < SL; ++s) sum[s] = in ? fma(v[u][s], xv[u], sum[s]) : sum[s];
+      for (int u = 0; u < U; ++u) {
+        const bool in = j0 + u * C + sub < kk;  // past the end: adds nothing
+#pragma unroll
+        for (int s = 0; s < SL; ++s) sum[s] = in ? fma(v[u][s], xv[u], sum[s]) : sum[s];
+      }
     }
   }
 #pragma unroll
@@ -910,15 +920,16 @@ struct GemvTerms {
 };
 
 // SLM: 64-row segments of the tallest block that was announced (a taller one
-// goes by pieces); GM: groups of W waves, which take the terms in turn.
-template <int SLM, int UL, int W, int GM>
-__global__ void __launch_bounds__(W == 1 ? 64 : 64 * W * F3D_GEMV_TERMS)
+// goes by pieces); UL: loads of a lane in flight; GM: groups of four waves, which
+// take the terms in turn.
+template <int SLM, int UL, int GM>
+__global__ void __launch_bounds__(kGemvThreads * F3D_GEMV_TERMS)
 block_gemv_kernel(int terms, const GemvTerms tt, const long* __restrict__ y_off,
                   double* __restrict__ y, double beta) {
-  __shared__ double red[W == 1 ? 1 : W * GM][W == 1 ? 1 : 64 * SLM];
+  __shared__ double red[4 * GM][64 * SLM];
   const int b = blockIdx.x;
-  const int t = threadIdx.x, lane = t & 63, groups = GM == 1 ? 1 : blockDim.x / (64 * W);
-  const int wv = W == 1 ? 0 : __builtin_amdgcn_readfirstlane(t >> 6);
+  const int t = threadIdx.x, lane = t & 63, groups = GM == 1 ? 1 : blockDim.x / kGemvThreads;
+  const int wv = __builtin_amdgcn_readfirstlane(t >> 6);
   int m = 0;  // rows of the block: of its tallest term
   for (int q = 0; q < terms; ++q) {
     const int mq = tt.t[q].m[b];
@@ -934,39 +945,29 @@ block_gemv_kernel(int terms, const GemvTerms tt, const long* __restrict__ y_off,
 #pragma unroll
       for (int s = 0; s < SL.value; ++s) acc[s] = 0.0;
 #pragma unroll 1
-      for (int q = wv / W; q < terms; q += groups) {
+      for (int q = wv / 4; q < terms; q += groups) {
         const f3d_gemv_term& g = tt.t[q];
         const int mq = g.m[b];
         if (mq > r0)
-          block_gemv_cols<R.value, SL.value, UL, W>(g.M + g.m_off[b], g.x + g.x_off[b], mq,
-                                                    g.k[b], g.alpha, r0, wv % W, lane, acc);
+          block_gemv_cols<R.value, SL.value, UL>(g.M + g.m_off[b], g.x + g.x_off[b], mq, g.k[b],
+                                                 g.alpha, r0, wv % 4, lane, acc);
       }
       if (R.value == 32) acc[0] += __shfl_xor(acc[0], 32, 64);
 #pragma unroll
-      for (int s = 0; s < SL.value; ++s) {
-        if constexpr (W == 1) {
-          // (one wave: its own rows, with no exchange)
-          const int r = r0 + 64 * s + lane;
-          if (lane < R.value && r < m) yb[r] = beta == 0.0 ? acc[s] : fma(beta, yb[r], acc[s]);
-        } else {
-          red[wv][64 * s + lane] = acc[s];
-        }
-      }
+      for (int s = 0; s < SL.value; ++s) red[wv][64 * s + lane] = acc[s];
     };
     if (m <= 32) sums(integral_constant<int, 32>{}, integral_constant<int, 1>{});
     else if (SLM == 1 || mr <= 64) sums(integral_constant<int, 64>{}, integral_constant<int, 1>{});
     else if (mr <= 128) sums(integral_constant<int, 64>{}, integral_constant<int, SLM == 1 ? 1 : 2>{});
     else sums(integral_constant<int, 64>{}, integral_constant<int, SLM>{});
-    if constexpr (W > 1) {
-      __syncthreads();
-      if (t < min(mr, 64 * SLM)) {
-        double v = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
-        for (int g = 1; g < groups; ++g)
-          v += (red[W * g][t] + red[W * g + 1][t]) + (red[W * g + 2][t] + red[W * g + 3][t]);
-        yb[r0 + t] = beta == 0.0 ? v : fma(beta, yb[r0 + t], v);
-      }
-      if (SLM < kSlots) __syncthreads();  // (after the last piece too: faster code)
+    __syncthreads();
+    if (t < min(mr, 64 * SLM)) {
+      double v = (red[0][t] + red[1][t]) + (red[2][t] + red[3][t]);
+      for (int g = 1; g < groups; ++g)
+        v += (red[4 * g][t] + red[4 * g + 1][t]) + (red[4 * g + 2][t] + red[4 * g + 3][t]);
+      yb[r0 + t] = beta == 0.0 ? v : fma(beta, yb[r0 + t], v);
     }
+    if (SLM < kSlots) __syncthreads();  // (after the last piece too: faster code)
   };
   if constexpr (SLM == kSlots) {
     if (m > 0) piece(integral_constant<int, 0>{});
@@ -1245,25 +1246,20 @@ extern "C" int f3d_block_gemv_sum(int64_t nb, int32_t mmax, int32_t terms,
     tt.t[q] = g;
   }
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-#define F3D_GV(SLM, UL, W, GM, G)                                                         \
-  F3D_LAUNCH((block_gemv_kernel<SLM, UL, W, GM>), dim3((unsigned)nb), dim3(64 * W * (G)), 0, st, \
-             terms, tt, (const long*)y_off, y, beta)
-  // One product of blocks of at most 128 rows takes 8 loads a wave, and one wave a
-  // block where there are many (8 per CU: a CU then has its waves from several).  us,
-  // with one wave, four, and the four waves of 16 loads that longer products take: 50 x
-  // 16, 2048 blocks 3.9, 4.8, 5.7, 4096 5.7, 8.3, 11.2; 64 x 64, 1000 blocks 8.0, 5.7, 5.9,
-  // 2048 12.9, 12.8, 13.9; 82 x 24, 1500 6.1, 5.7, 6.9, 4096 13.2, 15.0, 16.3; 128 x 128, 2048
-  // 41.6, 42.5, 42.0; but 192 x 192, 256 blocks 29, 15, 16.  (Sums of several terms
-  // have long ones among them: up to 1.3 times slower by one wave.)
-  const bool many = nb >= 8 * (int64_t)num_cus();
-  if (terms == 1 && mmax <= 64 && many) F3D_GV(1, 8, 1, 1, 1);
-  else if (terms == 1 && mmax <= 64) F3D_GV(1, 8, 4, 1, 1);
-  else if (terms == 1 && mmax <= 128 && many) F3D_GV(kSlots, 16, 1, 1, 1);
-  else if (terms == 1 && mmax <= 128) F3D_GV(kSlots, 8, 4, 1, 1);
+#define F3D_GV(SLM, UL, GM, G)                                                            \
+  F3D_LAUNCH((block_gemv_kernel<SLM, UL, GM>), dim3((unsigned)nb), dim3(kGemvThreads * (G)), 0, \
+             st, terms, tt, (const long*)y_off, y, beta)
+  // One product of blocks of at most 64 rows has 8 loads of a lane in flight, and so
+  // have many blocks (8 per CU) of at most 128; us, for 16 loads: 6 x 16, 32 blocks 2.6
+  // for 3.1, 4096 5.5, 10.6; 50 x 16, 32 3.0, 2.9, 4096 8.1, 10.7; 64 x 64, 1000 5.8, 5.8, 4096
+  // 21.7, 23.3; 82 x 24, 4096 13.4, 17.0; 114 x 32, 4096 20.0, 22.0; but 114 x 128, 256 7.1,
+  // 6.7.  (Sums of several terms have long ones among them.)
+  if (terms == 1 && mmax <= 64) F3D_GV(1, 8, 1, 1);
+  else if (terms == 1 && mmax <= 128 && nb >= 8 * (int64_t)num_cus()) F3D_GV(kSlots, 8, 1, 1);
   // Four waves a term where the blocks leave CUs idle (32 blocks: 9.2 us for 12.8 with
   // the terms one after the other); elsewhere four waves a block, since the
   // waves of short terms would only hold their places (1000 blocks: 40.9 us for 48.2).
-  else F3D_GV(kSlots, 16, 4, F3D_GEMV_TERMS, nb <= num_cus() ? terms : 1);
+  else F3D_GV(kSlots, 16, F3D_GEMV_TERMS, nb <= num_cus() ? terms : 1);
 #undef F3D_GV
   return F3D_OK;
 }

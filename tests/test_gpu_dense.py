@@ -435,3 +435,26 @@ def test_lu_factor_of_many_small_blocks():
         np.testing.assert_array_equal(piv[rows], l2.piv.cpu().numpy())
         np.testing.assert_array_equal(perm[rows], l2.perm.cpu().numpy())
         np.testing.assert_array_equal(info[part], l2.info.cpu().numpy())
+
+
+@pytest.mark.parametrize("nb", [3, 300, 2100])
+def test_block_gemv_forms_agree_to_the_bit(nb):
+    """A block's product is the same whatever the call's other blocks are: the
+    forms for at most 64 and 128 rows keep the order of the one for all."""
+    print(f"case block gemv forms nb={nb}", flush=True)
+    rng = np.random.default_rng(nb)
+    ms = rng.choice([1, 14, 31, 32, 33, 50, 63, 64], nb)
+    ks = rng.choice([1, 7, 8, 9, 15, 16, 17, 33, 64, 65, 130], nb)
+    mats = [rng.normal(size=(m, k)) for m, k in zip(ms, ks)]
+    got = []
+    for tall in (64, 100, 256):
+        m, k = np.append(ms, tall), np.append(ks, 40)
+        rest = np.random.default_rng(1)
+        g = BlockGemv(m, k, np.cumsum(k) - k, np.cumsum(m) - m)
+        x = np.append(np.random.default_rng(2).normal(size=int(ks.sum())), rest.normal(size=40))
+        y = torch.ones(int(m.sum()), dtype=torch.float64, device="cuda")
+        M = g.pack(mats + [rest.normal(size=(tall, 40))])
+        g(M, torch.from_numpy(x).cuda(), y, alpha=0.7, beta=0.3)
+        got.append(y.cpu().numpy()[:int(ms.sum())])
+    np.testing.assert_array_equal(got[0], got[2])
+    np.testing.assert_array_equal(got[1], got[2])
