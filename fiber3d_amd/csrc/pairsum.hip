@@ -1080,7 +1080,8 @@ reduce_kernel(const T* __restrict__ part_hi, const T* __restrict__ part_lo, int 
 //
 // What bounds a small call is the chain of dependent launches and, inside
 // one, of sources: 64 per wave in pairsum_kernel, ns 2^lg / 256 here.  1024 x
-// 1024 Oseen: 19.6 us in four launches, 5.9 us here; 32 x 1024: 19.6 and 3.1.
+// 1024 Oseen: 16.4 us in the general path's launches, 5.5 us here; 16 x 1000: 17.8
+// and 3.0.
 constexpr int kDirectStage = 512;
 
 template <int KIND, int K, bool MASK>
