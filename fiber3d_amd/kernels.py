@@ -155,12 +155,12 @@ def _addr(t):
 def _as_common(ts):
     """Make a list of (N,3) tensors (None allowed) share one (sp, sc) and device."""
     ref = next(t for t in ts if t is not None)
-    st = _strides3(ref)
+    st, dev = _strides3(ref), ref.get_device()
     out = []
     for t in ts:
         if t is None:
             out.append(None)
-        elif _strides3(t) != st or t.device != ref.device:
+        elif _strides3(t) != st or t.get_device() != dev:
             out.append(torch.empty_strided(ref.shape, ref.stride(), dtype=ref.dtype,
                                            device=ref.device).copy_(t))
         else:
@@ -231,12 +231,14 @@ def periphery_apply(pos, nrm, w, ex, ey, ez, q, add=None, eta=1.0, reg=5e-3, eps
     elif _strides3(out) != (sp, sc):
         raise ValueError("out must share the layout of the inputs")
     prec = _PREC[precision]
+    need = lib.f3d_periphery_workspace_size(prec, n)
+    at = _here()
     with _ws_lock:
-        ws = workspace(lib.f3d_periphery_workspace_size(prec, n))
+        ws = workspace(need, at=at)
         rc = lib.f3d_periphery_apply(
-            prec, n, L.ptr(pos), L.ptr(nrm), L.ptr(w), L.ptr(ex), L.ptr(ey), L.ptr(ez), L.ptr(q),
-            L.ptr(add), sp, sc, float(eta), float(reg), float(eps), L.ptr(out), L.ptr(ws),
-            ws.numel(), _stream())
+            prec, n, pos.data_ptr(), _addr(nrm), _addr(w), _addr(ex), _addr(ey), _addr(ez),
+            _addr(q), _addr(add), sp, sc, float(eta), float(reg), float(eps), out.data_ptr(),
+            ws.data_ptr(), ws.numel(), at[1])
     L.check(rc, "f3d_periphery_apply")
     return out
 
