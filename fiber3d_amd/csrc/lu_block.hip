@@ -423,13 +423,10 @@ __device__ __forceinline__ void lu_block_body(LuShared<T, W, NM>& sh, const int*
       for (int c = 0; c < kWp; ++c) a[c] = row ? panel[c * kWs + tid] : (T)0;
       bool live = mine && pos >= c0;
       int vat = 0;  // lane j: column j's pivot row | position << 16
-      sfor<0, kWp>([&](auto J) __attribute__((always_inline)) {
+      auto column = [&](auto J) __attribute__((always_inline)) {
         constexpr int j = decltype(J)::value;
         constexpr int buf = j & 1;
         const int c = c0 + j;
-        // (a padded column changes nothing that is stored: 3000 FP64 blocks of order
-        // 4 56.7 -> 33.0 us, of order 68 465 -> 421)
-        if (c >= n) return;
         // (a padded row pivots padded columns only)
         const unsigned kh = live && (phys < n) == (c < n) ? abs_key(a[j]) : 0u;
         // (off the chain: every row's own reciprocal while the wave searches)
@@ -500,6 +497,13 @@ __device__ __forceinline__ void lu_block_body(LuShared<T, W, NM>& sh, const int*
         const int p = bat >> 16;
         pos = pos == c ? p : (pos == p ? c : pos);
         vat = lane == j ? bat : vat;
+      };
+      // (padded columns change nothing that is stored: 3000 FP64 blocks of order 4
+      // 56.7 -> 33.0 us, of order 68 465 -> 421.  Four columns at a time: a test per
+      // column costs FP32 1%)
+      sfor<0, kWp / 4>([&](auto Q) __attribute__((always_inline)) {
+        constexpr int q = 4 * decltype(Q)::value;
+        if (q == 0 || c0 + q < n) sfor<q, q + 4>(column);
       });
       if (wv == 0 && lane < kWp) {
         sh.piv[c0 + lane] = (unsigned char)(vat >> 16);
