@@ -22,7 +22,7 @@ import numpy as np
 import torch
 
 from . import _lib as L
-from .kernels import _addr, _stream
+from .kernels import _addr, _here, _stream
 
 EPI_STORE, EPI_BIAS_RELU, EPI_RELU_GRAD, EPI_ATOMIC, EPI_BIAS = 0, 1, 2, 3, 4
 
@@ -88,10 +88,10 @@ class MLP:
         H1 = X.new_empty((M, self.width))
         H2 = torch.empty_like(H1)
         Y = X.new_empty((M, self.n_out))
-        p = _addr
         rc = L.load().f3d_mlp_forward(
-            M, self.n_in, self.width, self.n_out, p(X), X.stride(0), X.stride(1), p(W1),
-            p(b1), p(W2), p(b2), p(W3), p(b3), p(H1), p(H2), p(Y), _stream())
+            M, self.n_in, self.width, self.n_out, X.data_ptr(), *X.stride()[:2], W1.data_ptr(),
+            _addr(b1), W2.data_ptr(), _addr(b2), W3.data_ptr(), _addr(b3), H1.data_ptr(),
+            H2.data_ptr(), Y.data_ptr(), _here()[1])
         L.check(rc, "f3d_mlp_forward")
         if keep:
             self._cache = (X, H1, H2)
@@ -109,11 +109,10 @@ class MLP:
                  + [X.new_empty(s[1:]) for s in self.shapes])
         need = lib.f3d_mlp_workspace_size(M, self.n_in, self.width, self.n_out)
         ws = X.new_empty(-(-need // 4))
-        p = _addr
         rc = lib.f3d_mlp_backward(
-            M, self.n_in, self.width, self.n_out, p(X), X.stride(0), X.stride(1), p(H1), p(H2),
-            p(dY), dY.stride(0), dY.stride(1), p(W2), p(W3),
-            *(p(g) for g in grads), p(ws), need, _stream())
+            M, self.n_in, self.width, self.n_out, X.data_ptr(), *X.stride()[:2], H1.data_ptr(),
+            H2.data_ptr(), dY.data_ptr(), *dY.stride(), W2.data_ptr(), W3.data_ptr(),
+            *[g.data_ptr() for g in grads], ws.data_ptr(), need, _here()[1])
         L.check(rc, "f3d_mlp_backward")
         return grads
 
@@ -124,7 +123,7 @@ class MLP:
         self.t += 1
         fused = []
         f32 = torch.float32
-        here = torch.cuda.current_device() if torch.cuda.is_initialized() else -2
+        here, stream = _here() if torch.cuda.is_initialized() else (-2, None)
         for p, grad, m, v in zip(self.params, grads, self.m, self.v):
             g = grad.contiguous()
             if (p.dtype is f32 and g.dtype is f32 and m.dtype is f32 and v.dtype is f32
@@ -145,7 +144,7 @@ class MLP:
         ptrs = lambda ts: (ctypes.c_void_p * k)(*ts)
         sizes = (ctypes.c_int64 * k)(*(q[0].numel() for q in fused))
         rc = L.load().f3d_adam(k, sizes, ptrs(p), ptrs(g), ptrs(m), ptrs(v), lr, b1, b2, eps,
-                               self.t, _stream())
+                               self.t, stream)
         L.check(rc, "f3d_adam")
 
     def _adam_torch(self, p, g, m, v, lr, b1, b2, eps):
@@ -163,8 +162,8 @@ class MLP:
             loss = Y.new_empty(())
             need = lib.f3d_mse_workspace_size()
             ws = Y.new_empty(-(-need // 4))
-            rc = lib.f3d_mse(Y.numel(), _addr(Y), _addr(target), _addr(dY), _addr(loss),
-                             _addr(ws), need, _stream())
+            rc = lib.f3d_mse(Y.numel(), Y.data_ptr(), target.data_ptr(), dY.data_ptr(),
+                             loss.data_ptr(), ws.data_ptr(), need, _here()[1])
             L.check(rc, "f3d_mse")
         else:
             # torch broadcasts and converts the target, or refuses it
